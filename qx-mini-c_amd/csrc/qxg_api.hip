@@ -55,18 +55,19 @@ void qxl_head(hipStream_t, const float *, const float *, const QTensor *, uint32
               uint32_t *, bool, Timer = Timer());
 __global__ void qxp_embed(const uint8_t *, uint64_t, const uint32_t *, float *);
 __global__ void qxp_norm(const float *, const float *, uint32_t, float *);
+__global__ void qxp_ffn_norm(const float *, const float *, uint32_t, float *, uint8_t *, float *);
 __global__ void qxp_norm_pack(const float *, const float *, uint32_t, uint32_t, uint4 *, float *);
 __global__ void qxp_qk(const float *, const float *, const float *, Tables, int8_t *, int8_t *, float *, float *,
                        uint32_t, uint32_t, uint32_t, float *);
 __global__ void qxp_attn(const float *, const int8_t *, const int8_t *, const float *, const float *, uint32_t, uint32_t,
                          uint32_t, uint32_t, float *);
-__global__ void qxp_router(const float *, const float *, uint32_t, uint32_t, double *);
-__global__ void qxp_route(const double *, uint32_t, uint32_t, uint32_t *, double *);
-__global__ void qxp_group(const uint32_t *, uint32_t, uint32_t, uint32_t, int32_t *, uint32_t *, uint32_t *, uint32_t *);
-__global__ void qxp_combine(const float *, const float *, const uint32_t *, const double *, float *, float *);
+__global__ void qxp_router(const float *, const float *, uint32_t, uint32_t, double *, uint32_t *);
+__global__ void qxp_route(const double *, uint32_t, uint32_t, double *, uint32_t *, uint32_t *);
+__global__ void qxp_combine(const float *, const float *, const double *, float *, float *);
+__global__ void qxp_pack_ctx(const float *, uint32_t, uint32_t, uint4 *, float *);
 void qxp_launch_gemm(hipStream_t, int, const PfGemm &, const PfTables &, uint32_t, uint32_t, Timer);
-void qxp_launch_pack(hipStream_t, int, const float *, const int32_t *, const uint32_t *, uint32_t, uint32_t, uint4 *,
-                     float *);
+void qxp_launch_gate_up(hipStream_t, uint32_t, const PfExperts &, const PfTables &, uint32_t, Timer);
+void qxp_launch_down(hipStream_t, uint32_t, const PfExperts &, const PfTables &, uint32_t, Timer);
 }
 
 namespace {
@@ -170,11 +171,11 @@ struct qxg_ctx {
         bool ready = false;
         PfTables P{};
         float *X = nullptr, *X1 = nullptr, *XN = nullptr, *QKV = nullptr, *QR = nullptr, *CTX = nullptr;
-        float *H = nullptr, *Y = nullptr, *rscale = nullptr, *dump = nullptr;
+        float *HS = nullptr, *Y = nullptr, *rscale = nullptr, *xscale = nullptr, *dump = nullptr;
         uint4 *apk = nullptr;
+        uint8_t *XP = nullptr, *HP = nullptr;
         double *lg = nullptr, *w = nullptr;
-        uint32_t *ids = nullptr, *tok_slot = nullptr, *mgroups = nullptr, *meta = nullptr, *tokens = nullptr;
-        int32_t *slot_token = nullptr;
+        uint32_t *cnt = nullptr, *list = nullptr, *tokens = nullptr;
         std::vector<void *> all;
     } pf;
     // stage-probe outputs (allocated on first use)
@@ -690,10 +691,6 @@ bool build_arenas(qxg_ctx *c, char *err, uint64_t n) {
 }
 
 // ---- batched prefill
-constexpr uint32_t PF_EXPERT_MT = QXG_PF_EXPERT_MT;               // row tiles per expert GEMM wave
-constexpr uint32_t PF_SLOTS = QXP_MAX * QXG_TOPK + 32 * 128;       // expert slots, padded per expert
-constexpr uint32_t PF_MGROUPS = QXP_MAX * QXG_TOPK / 32 + 128;     // bound on expert m-groups
-
 // fp16 bits of a small integer (|v| < 2048: exact)
 uint16_t f16_int(int v) {
     if (v == 0) return 0;
@@ -717,48 +714,38 @@ bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
         B.all.push_back(*p);
         return true;
     };
-    const uint64_t T = QXP_MAX;
+    const uint64_t T = QXP_MAX, PAIRS = T * QXG_TOPK;
     bool ok = alloc((void **)&B.X, T * 2048 * 4) && alloc((void **)&B.X1, T * 2048 * 4) &&
               alloc((void **)&B.XN, T * 2048 * 4) && alloc((void **)&B.QKV, T * 5120 * 4) &&
               alloc((void **)&B.QR, T * 4096 * 4) && alloc((void **)&B.CTX, T * 4096 * 4) &&
-              alloc((void **)&B.H, (uint64_t)PF_SLOTS * QXG_FFN * 4) && alloc((void **)&B.Y, (uint64_t)PF_SLOTS * 2048 * 4) &&
-              alloc((void **)&B.rscale, (uint64_t)PF_SLOTS * 4) && alloc((void **)&B.dump, T * 2048 * 4) &&
-              alloc((void **)&B.apk, (uint64_t)PF_SLOTS * 2048 * 4) && alloc((void **)&B.lg, T * 128 * 8) &&
-              alloc((void **)&B.w, T * 8 * 8) && alloc((void **)&B.ids, T * 8 * 4) && alloc((void **)&B.tok_slot, T * 8 * 4) &&
-              alloc((void **)&B.mgroups, PF_MGROUPS * 4) && alloc((void **)&B.meta, 16) && alloc((void **)&B.tokens, T * 4) &&
-              alloc((void **)&B.slot_token, (uint64_t)PF_SLOTS * 4);
-    // codebooks: IQ2_XS / IQ3_XXS grids and the IQ4_XS byte table as fp16, sign masks
-    std::vector<uint16_t> g2(512 * 8), g3(256 * 4), sg(128 * 8);
+              alloc((void **)&B.XP, T * 8192) && alloc((void **)&B.xscale, T * 4) && alloc((void **)&B.HP, PAIRS * 3072) &&
+              alloc((void **)&B.HS, PAIRS * 8 * 4) && alloc((void **)&B.Y, PAIRS * 2048 * 4) &&
+              alloc((void **)&B.rscale, T * 4) && alloc((void **)&B.dump, T * 2048 * 4) &&
+              alloc((void **)&B.apk, T * 4096 * 4) && alloc((void **)&B.lg, T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
+              alloc((void **)&B.cnt, 128 * 4) && alloc((void **)&B.list, 128ull * QXP_LIST * 4) &&
+              alloc((void **)&B.tokens, T * 4);
+    // codebooks: grids as magnitude bytes, sign bytes (0x80 where negative), the IQ4_XS byte table as fp16
+    std::vector<uint8_t> g2(512 * 8), g2s(1024 * 8), g3(256 * 4), g3s(512 * 4), sg7(128 * 8), sg8(256 * 8);
     std::vector<uint32_t> kv2(256);
-    for (int i = 0; i < 512; ++i)
-        for (int j = 0; j < 8; ++j) g2[i * 8 + j] = f16_int(qx_iq2xs_levels[(qx_iq2xs_packed[i] >> (2 * j)) & 3]);
-    for (int i = 0; i < 256; ++i)
-        for (int j = 0; j < 4; ++j) g3[i * 4 + j] = f16_int(qx_iq3xxs_levels[(qx_iq3xxs_packed[i] >> (3 * j)) & 7]);
+    for (int i = 0; i < 512 * 8; ++i) g2[i] = qx_iq2xs_levels[(qx_iq2xs_packed[i >> 3] >> (2 * (i & 7))) & 3];
+    for (int i = 0; i < 1024 * 8; ++i) g2s[i] = qx_iq2xs_levels[(qx_iq2s_packed[i >> 3] >> (2 * (i & 7))) & 3];
+    for (int i = 0; i < 256 * 4; ++i) g3[i] = qx_iq3xxs_levels[(qx_iq3xxs_packed[i >> 2] >> (3 * (i & 3))) & 7];
+    for (int i = 0; i < 512 * 4; ++i) g3s[i] = qx_iq3s_levels[(qx_iq3s_packed[i >> 2] >> (3 * (i & 3))) & 7];
+    for (uint32_t i = 0; i < 256; ++i)
+        for (int j = 0; j < 8; ++j) sg8[i * 8 + j] = ((i >> j) & 1) ? 0x80 : 0;
     for (uint32_t i = 0; i < 128; ++i) {
         const uint32_t sbits = i | ((uint32_t)(__builtin_popcount(i) & 1) << 7);   // ksigns (ggml)
-        for (int j = 0; j < 8; ++j) sg[i * 8 + j] = ((sbits >> j) & 1) ? 0x8000 : 0;
+        for (int j = 0; j < 8; ++j) sg7[i * 8 + j] = sg8[sbits * 8 + j];
     }
     for (uint32_t b = 0; b < 256; ++b)
         kv2[b] = (uint32_t)f16_int(qx_iq4nl_values[b & 15]) | ((uint32_t)f16_int(qx_iq4nl_values[b >> 4]) << 16);
-    // the real checkpoint's IQ2_S / IQ3_S grids as fp16, and sign masks of an explicit sign byte
-    std::vector<uint16_t> g2s(1024 * 8), g3s(512 * 4), sg8(256 * 8);
-    for (int i = 0; i < 1024; ++i)
-        for (int j = 0; j < 8; ++j) g2s[i * 8 + j] = f16_int(qx_iq2xs_levels[(qx_iq2s_packed[i] >> (2 * j)) & 3]);
-    for (int i = 0; i < 512; ++i)
-        for (int j = 0; j < 4; ++j) g3s[i * 4 + j] = f16_int(qx_iq3s_levels[(qx_iq3s_packed[i] >> (3 * j)) & 7]);
-    for (uint32_t i = 0; i < 256; ++i)
-        for (int j = 0; j < 8; ++j) sg8[i * 8 + j] = ((i >> j) & 1) ? 0x8000 : 0;
-    ok = ok && alloc((void **)&B.P.g2h, g2.size() * 2) && alloc((void **)&B.P.g3h, g3.size() * 2) &&
-         alloc((void **)&B.P.sgn, sg.size() * 2) && alloc((void **)&B.P.kv2, kv2.size() * 4) &&
-         alloc((void **)&B.P.g2sh, g2s.size() * 2) && alloc((void **)&B.P.g3sh, g3s.size() * 2) &&
-         alloc((void **)&B.P.sgn8, sg8.size() * 2);
-    ok = ok && hip_ok(hipMemcpy(B.P.g2h, g2.data(), g2.size() * 2, hipMemcpyHostToDevice), err, n, "prefill tables") &&
-         hip_ok(hipMemcpy(B.P.g3h, g3.data(), g3.size() * 2, hipMemcpyHostToDevice), err, n, "prefill tables") &&
-         hip_ok(hipMemcpy(B.P.sgn, sg.data(), sg.size() * 2, hipMemcpyHostToDevice), err, n, "prefill tables") &&
-         hip_ok(hipMemcpy(B.P.kv2, kv2.data(), kv2.size() * 4, hipMemcpyHostToDevice), err, n, "prefill tables") &&
-         hip_ok(hipMemcpy(B.P.g2sh, g2s.data(), g2s.size() * 2, hipMemcpyHostToDevice), err, n, "prefill tables") &&
-         hip_ok(hipMemcpy(B.P.g3sh, g3s.data(), g3s.size() * 2, hipMemcpyHostToDevice), err, n, "prefill tables") &&
-         hip_ok(hipMemcpy(B.P.sgn8, sg8.data(), sg8.size() * 2, hipMemcpyHostToDevice), err, n, "prefill tables");
+    auto table = [&](void **p, const void *v, uint64_t bytes) {
+        return alloc(p, bytes) && hip_ok(hipMemcpy(*p, v, bytes, hipMemcpyHostToDevice), err, n, "prefill tables");
+    };
+    ok = ok && table((void **)&B.P.g2, g2.data(), g2.size()) && table((void **)&B.P.g2s, g2s.data(), g2s.size()) &&
+         table((void **)&B.P.g3, g3.data(), g3.size()) && table((void **)&B.P.g3s, g3s.data(), g3s.size()) &&
+         table((void **)&B.P.sg7, sg7.data(), sg7.size()) && table((void **)&B.P.sg8, sg8.data(), sg8.size()) &&
+         table((void **)&B.P.kv2, kv2.data(), kv2.size() * 4);
     if (!ok) {
         for (void *p : B.all) (void)hipFree(p);
         B.all.clear();
@@ -783,8 +770,7 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, float *moe_d
                        B.rscale);
     // per-layer formats of the real checkpoint: V and O in Q5_K or IQ4_XS, gate/up in IQ2_S or
     // IQ2_XS, down in IQ3_XXS, IQ3_S or IQ4_XS (type ids of the QXF1 manifest)
-    const bool vo_q5 = w.wv->type == 13, gu_s = w.gate->type == 22;
-    const int dn_kind = w.down->type == 21 ? QXP_DOWN_IQ3S : w.down->type == 23 ? QXP_DOWN_IQ4 : QXP_DOWN;
+    const bool vo_q5 = w.wv->type == 13;
     PfGemm g{};
     g.w[0] = pf_mat(w.wq); g.w[1] = pf_mat(w.wk); g.w[2] = pf_mat(w.wv);
     g.w_start[0] = 0; g.w_start[1] = 4096; g.w_start[2] = vo_q5 ? none : 4608;
@@ -800,35 +786,26 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, float *moe_d
     qx_launch(qxp_attn, dim3(4, (T + 3) / 4), dim3(256), 0, s, timer_for(c, 13), (const float *)B.QR,
               (const int8_t *)c->kc, (const int8_t *)c->vc, (const float *)c->ks, (const float *)c->vs, l, c->kv_ctx, p0, T,
               B.CTX);
-    qxp_launch_pack(s, 4096, B.CTX, nullptr, nullptr, mt * 32, T, B.apk, B.rscale);
+    hipLaunchKernelGGL(qxp_pack_ctx, dim3(mt * 8), dim3(256), 0, s, (const float *)B.CTX, mt * 32, T, B.apk, B.rscale);
     g = PfGemm{};
     g.w[0] = pf_mat(w.wo); g.w_start[1] = none; g.w_start[2] = none;
     g.kb = 16; g.apk = B.apk; g.rscale = B.rscale; g.mtiles = mt; g.nvalid = T; g.out = B.X1; g.ld = 2048;
     g.resid = B.X;
     qxp_launch_gemm(s, vo_q5 ? QXP_O_Q5 : QXP_O, g, B.P, 2048 / 128, mt, timer_for(c, 9));
-    // MoE half: RMSNorm, router logits, top-8, grouping by expert, gate/up + SwiGLU, down, combine
-    hipLaunchKernelGGL(qxp_norm, dim3((T + 3) / 4), dim3(256), 0, s, (const float *)B.X1, w.ffn_norm, T, B.XN);
+    // MoE half: RMSNorm, router logits, top-8 and the experts' pair lists, gate/up + SwiGLU, down, combine
+    hipLaunchKernelGGL(qxp_ffn_norm, dim3((T + 3) / 4), dim3(256), 0, s, (const float *)B.X1, w.ffn_norm, T, B.XN, B.XP,
+                       B.xscale);
     qx_launch(qxp_router, dim3((T + 15) / 16, (E + 15) / 16), dim3(512), 0, s, timer_for(c, 12), (const float *)B.XN,
-              w.router, T, E, B.lg);
-    hipLaunchKernelGGL(qxp_route, dim3((T + 3) / 4), dim3(256), 0, s, (const double *)B.lg, T, E, B.ids, B.w);
-    hipLaunchKernelGGL(qxp_group, dim3(1), dim3(1024), 0, s, (const uint32_t *)B.ids, T, E, PF_EXPERT_MT, B.slot_token,
-                       B.tok_slot, B.mgroups, B.meta);
-    const uint32_t slots_ub = T * QXG_TOPK + 32 * E;        // padded slots never exceed this
-    const uint32_t mg_ub = (T * QXG_TOPK + 31) / 32 + E;      // nor the m-groups this
-    qxp_launch_pack(s, 2048, B.XN, B.slot_token, B.meta, slots_ub, none, B.apk, B.rscale);
-    g = PfGemm{};
-    g.w[0] = pf_mat(w.gate); g.w[1] = pf_mat(w.up); g.w_start[1] = none; g.w_start[2] = none;
-    g.rows = QXG_FFN; g.kb = 8; g.apk = B.apk; g.rscale = B.rscale; g.mgroups = B.mgroups; g.meta = B.meta;
-    g.out = B.H; g.ld = QXG_FFN;
-    qxp_launch_gemm(s, gu_s ? QXP_GU_IQ2S : QXP_GU, g, B.P, QXG_FFN / 128, mg_ub, timer_for(c, 10));
-    qxp_launch_pack(s, 768, B.H, nullptr, B.meta, slots_ub, none, B.apk, B.rscale);
-    g = PfGemm{};
-    g.w[0] = pf_mat(w.down); g.w_start[1] = none; g.w_start[2] = none;
-    g.rows = 2048; g.kb = 3; g.apk = B.apk; g.rscale = B.rscale; g.mgroups = B.mgroups; g.meta = B.meta;
-    g.out = B.Y; g.ld = 2048;
-    qxp_launch_gemm(s, dn_kind, g, B.P, 2048 / 128, mg_ub, timer_for(c, 11));
-    hipLaunchKernelGGL(qxp_combine, dim3(T), dim3(256), 0, s, (const float *)B.X1, (const float *)B.Y,
-                       (const uint32_t *)B.tok_slot, (const double *)B.w, B.X, moe_dump);
+              w.router, T, E, B.lg, B.cnt);
+    hipLaunchKernelGGL(qxp_route, dim3((T + 31) / 32), dim3(1024), 0, s, (const double *)B.lg, T, E, B.w, B.cnt, B.list);
+    PfExperts x{};
+    x.w[0] = pf_mat(w.gate); x.w[1] = pf_mat(w.up); x.w[2] = pf_mat(w.down);
+    x.experts = E; x.cnt = B.cnt; x.list = B.list; x.xp = B.XP; x.xs = B.xscale; x.hp = B.HP; x.hs = B.HS;
+    x.h_pairs = w.down->type == 23; x.y = B.Y;
+    qxp_launch_gate_up(s, w.gate->type, x, B.P, T, timer_for(c, 10));
+    qxp_launch_down(s, w.down->type, x, B.P, T, timer_for(c, 11));
+    hipLaunchKernelGGL(qxp_combine, dim3(T), dim3(256), 0, s, (const float *)B.X1, (const float *)B.Y, (const double *)B.w,
+                       B.X, moe_dump);
 }
 // Token-step prefill: one decode step per prompt token (embedding, every layer), the head
 // on the last when run_head; residual_out row i is token i's final residual.

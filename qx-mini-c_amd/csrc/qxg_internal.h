@@ -203,20 +203,19 @@ struct QxDArgs {
 
 // ---- batched prefill (qxg_prefill.hip)
 #define QXP_MAX 512   // tokens per prefill chunk
-// 32-row tiles per wave of the expert GEMMs.  One tile keeps a workgroup at 64 KiB of
-// LDS and few enough registers for two workgroups per CU: gate/up 118 -> 102 us and
-// down 87 -> 65 us per layer at T = 512 against two tiles (one workgroup per CU).
-#define QXG_PF_EXPERT_MT 1
+// entries of one expert's pair list: every (token, rank) pair of a chunk (an expert takes a
+// token once, except where non-finite logits make the top-8 repeat it)
+#define QXP_LIST (QXP_MAX * QXG_TOPK)
 
-// fp16 codebooks of the prefill GEMMs (built on the host at first use)
+// codebooks of the prefill GEMMs (built on the host at first use)
 struct PfTables {
-    uint4 *g2h;      // IQ2_XS grid: 512 x 8 fp16 values
-    uint2 *g3h;      // IQ3_XXS grid: 256 x 4 fp16 values
-    uint4 *sgn;      // 7-bit sign index -> 8 fp16 sign masks (0x8000 where negative)
+    uint2 *g2;       // IQ2_XS grid: 512 x 8 magnitude bytes
+    uint2 *g2s;      // IQ2_S grid: 1024 x 8
+    uint32_t *g3;    // IQ3_XXS grid: 256 x 4
+    uint32_t *g3s;   // IQ3_S grid: 512 x 4
+    uint2 *sg7;      // 7-bit sign index -> 8 sign bytes (0x80 where negative)
+    uint2 *sg8;      // sign byte -> 8 sign bytes
     uint32_t *kv2;   // IQ4_XS byte -> {fp16 kvalue[low nibble], fp16 kvalue[high nibble]}
-    uint4 *g2sh;     // IQ2_S grid: 1024 x 8 fp16 values
-    uint2 *g3sh;     // IQ3_S grid: 512 x 4 fp16 values
-    uint4 *sgn8;     // sign byte -> 8 fp16 sign masks (IQ2_S, IQ3_S)
 };
 
 // One quantized matrix [rows x K] in the repacked layout (expert e's rows follow e*rows).
@@ -226,29 +225,36 @@ struct PfMat {
     const uint16_t *d;        // fp16 d per block (IQ2_XS, IQ3_XXS, IQ2_S, IQ3_S)
 };
 
-// Arguments of one prefill GEMM launch: Y[row][col] = sum_k A[row][k] * W[col][k], A the
-// packed activations (rows = tokens or expert slots), W up to three matrices stacked
-// along the output columns (Q, K, V) or, for the expert GEMMs, expert e's slice.
+// Arguments of one dense prefill GEMM launch: Y[row][col] = sum_k A[row][k] * W[col][k], A the
+// packed activations (rows = tokens), W up to three matrices stacked along the output
+// columns (Q, K, V).
 struct PfGemm {
     PfMat w[3];
     uint32_t w_start[3];       // first output column of each stacked matrix
-    uint32_t rows;             // rows of one expert's matrix (expert GEMMs)
     uint32_t kb;               // 256-value blocks per matrix row (K / 256)
     const uint4 *apk;          // packed activations
     const float *rscale;       // per packed row: 1/s, 0 for a non-finite row
-    const uint32_t *mgroups;   // expert GEMMs: {expert, first m-tile, m-tiles}; null: dense
-    const uint32_t *meta;      // expert GEMMs: meta[0] = number of m-groups
-    uint32_t mtiles, nvalid;   // dense: m-tiles of 32 rows, valid rows
+    uint32_t mtiles, nvalid;   // m-tiles of 32 rows, valid rows
     float *out;                // output rows of ld floats
     uint32_t ld;
     const float *resid;        // residual added by the O projection epilogue
-    float *dump;               // O projection output without the residual (optional)
     uint32_t xcd_rows;         // row-tile classes across the 8 XCDs (1, 2, 4 or 8; the launcher sets it)
 };
 // GEMM kinds of qxp_launch_gemm (format and epilogue of the weight matrix)
-enum QxpGemmKind : int {
-    QXP_QKV = 0, QXP_O = 1, QXP_GU = 2, QXP_DOWN = 3,              // the benchmark mix
-    QXP_V_Q5 = 4, QXP_O_Q5 = 5, QXP_GU_IQ2S = 6, QXP_DOWN_IQ3S = 7, QXP_DOWN_IQ4 = 8   // real-checkpoint layers
+enum QxpGemmKind : int { QXP_QKV = 0, QXP_O = 1, QXP_V_Q5 = 4, QXP_O_Q5 = 5 };
+
+// Arguments of the routed-expert GEMMs (qxg_pf_experts.hip); pair p = 8 * token + rank.
+struct PfExperts {
+    PfMat w[3];                // gate, up, down: expert e's rows follow e * rows
+    uint32_t experts;
+    const uint32_t *cnt;       // pairs of each expert
+    const uint32_t *list;      // [expert][QXP_LIST] its pairs
+    const uint8_t *xp;         // packed normed activations, 8192 bytes a token
+    const float *xs;           // per token: 1 / the row's power-of-two scale, 0 for a non-finite row
+    uint8_t *hp;               // packed SwiGLU rows, 3072 bytes a pair
+    float *hs;                 // [pair][8]: 1 / scale of each 128 values (6 used), NaN for non-finite ones
+    uint32_t h_pairs;          // hp in the order of an IQ4_XS down matrix
+    float *y;                  // [pair][2048] down rows
 };
 
 // Optional start/stop events recorded around one launch on its stream.  Created with

@@ -1,0 +1,550 @@
+// Routed-expert GEMMs of the batched prefill (CDNA4, gfx950).
+//
+// Precision is that of qxg_prefill.hip: a weight is an f32 block scale times an integer
+// code that fp16 holds exactly, an activation row is scaled by a power of two and split
+// into fp16 hi + lo, the matrix cores accumulate in f32.  Here:
+//
+// Rows.  qxp_route lists each expert's (token, rank) pairs, p = 8 * token + rank; a
+// workgroup takes up to 64 of one expert's pairs and a range of its weight rows, so every
+// code is formed once for up to two 32-row tiles.  Activations are packed per token
+// (gate/up, gathered through the list while they are staged) and per pair (down, written
+// by gate/up's epilogue); no copy of them is sorted or padded by expert.
+//
+// Tiles.  v_mfma_f32_32x32x16_f16: lane l holds, for A, row l%32 and, for B, column l%32,
+// each 8 values of K at lane half h = l/32; result register r of lane l is row
+// 8*(r/4) + 4*h + r%4, column l%32.  (With one wave on a SIMD the 16x16x32 form reaches 1.2
+// PFLOP/s here, this one 1.6.)  Which 8 values a lane half holds is free as long as A and B
+// agree: a lane takes its part of a weight block whole, and the rows are packed in lines of
+// 128 bytes, line k / 2 and in it [k % 2][hi, lo][h][8 fp16] for k-step k:
+//     gate/up: K = 256 b + 128 h + 8 s + j, k-step 16 b + s    (sub-blocks 4h .. 4h + 3)
+//     down:    K = 128 q + 64 h + 8 s + j, k-step 8 q + s      (two sub-blocks of a half block)
+//     down in IQ4_XS: K = 32 i + 8 h + 4 t + j / 2 + 16 (j % 2), k-step 2 i + t   (a scale per 32)
+//
+// Staging.  A stage is 128 values of K of the pass's rows, 4 lines a row, copied to LDS by
+// load-to-LDS instructions of 8 rows x one whole line; the 16-byte chunk c of row r lies at
+// place c ^ (r % 8) of its line, so the column-wise reads spread over all banks.
+//
+// Codes.  The codebooks are bytes in LDS, 8 or 4 magnitudes an entry, with a second table
+// of sign bytes (0x80 where negative).  A magnitude byte and its sign byte side by side are
+// a subnormal fp16 number, sign * mag * 2^-24, so one v_perm forms two of them and one
+// v_pk_mul by (2 s + 1) * 2^11 makes the codes, exactly, at 2^-13 (11 significant bits; the
+// block scale takes the 2^13).  Random 16-byte reads of ready fp16 entries and fp16 sign masks
+// kept the LDS busy for most of the kernel; these take about 6 cycles each.
+//
+// What bounds them: the matrix cores at their sustained rate (about 1.4 PFLOP/s for tens of us,
+// power-limited), with twice the algorithmic work for hi and lo, where experts hold many pairs; the
+// weights' bytes and the about 20 vector instructions per 8 codes where they hold few.
+#include "qxg_dev.h"
+
+namespace {
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef float f4x __attribute__((ext_vector_type(4)));
+typedef float f16x __attribute__((ext_vector_type(16)));
+
+enum { FMT_IQ2 = 0, FMT_IQ2S = 1, FMT_IQ3 = 2, FMT_IQ3S = 3, FMT_IQ4 = 4 };
+
+DEV f16x mfma(uint4 a, uint4 b, f16x c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, a), __builtin_bit_cast(h8v, b), c, 0, 0, 0);
+}
+DEV f16x zero16() {
+    f16x z;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+    return z;
+}
+// lane i's 16 bytes at base + off land at lds + 16 i (lds the same in every lane)
+DEV void dma16(const void *base, uint32_t off, const void *lds) {
+    const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)lds);
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
+}
+// waits until at most N of the wave's loads (the youngest) are outstanding
+template <int N>
+DEV void wait_loads() {
+    static_assert(N < 16, "the wait's low counter bits");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | N);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// two signed codes (sign byte over magnitude byte, a subnormal fp16) times m
+DEV uint32_t code2(uint32_t mag, uint32_t sgn, uint32_t sel, h2v m) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, perm(sgn, mag, sel)) * m);
+}
+struct Codes { uint32_t m0, m1; uint2 sg; };   // 8 magnitude bytes and their sign bytes
+DEV uint4 conv(const Codes &c, h2v m) {
+    return make_uint4(code2(c.m0, c.sg.x, 0x05010400u, m), code2(c.m0, c.sg.x, 0x07030602u, m),
+                      code2(c.m1, c.sg.y, 0x05010400u, m), code2(c.m1, c.sg.y, 0x07030602u, m));
+}
+DEV h2v odd_mul(uint32_t n) {   // (2 n + 1) * 2^11, n < 16: exact
+    const _Float16 f = (_Float16)(uint16_t)((n << 12) | 2048u);
+    return h2v{f, f};
+}
+constexpr float CODE_SCALE = 8192.0f;   // 2^13: the codes above are at 2^-13
+
+DEV uint32_t word_at(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+DEV uint32_t byte_at(const uint4 &v, int i) { return (word_at(v, i >> 2) >> (8 * (i & 3))) & 255u; }
+DEV uint32_t ldu16(const void *p) { return *reinterpret_cast<const uint16_t *>(p); }
+DEV uint32_t ldu32(const void *p) { return *reinterpret_cast<const uint32_t *>(p); }
+DEV uint2 ldu64(const void *p) { return *reinterpret_cast<const uint2 *>(p); }
+DEV uint4 ldu128(const void *p) { return *reinterpret_cast<const uint4 *>(p); }
+
+constexpr int RT = 2;                    // 32-row tiles of a workgroup pass, at most
+constexpr int ROWS = 32 * RT;            // pairs per pass
+constexpr int STAGE = 4 * ROWS * 8;      // uint4 per stage: 4 lines of 8 chunks a row
+
+// The four lines from line0 on of the pass's rows: wave w copies line w, 8 rows an
+// instruction; off[i] is the lane's row 8 i + lane / 8 and its chunk of the line.
+template <int MT>
+DEV void stage_rows(const void *rows, const uint32_t (&off)[4 * MT], uint32_t line0, uint4 *buf, int wave) {
+#pragma unroll
+    for (int i = 0; i < 4 * MT; ++i) dma16(rows, off[i] + (line0 + wave) * 128, buf + (wave * ROWS + 8 * i) * 8);
+}
+template <int MT>
+DEV void stage_offsets(uint32_t (&off)[4 * MT], const uint32_t *s_row, uint32_t row_bytes, int lane) {
+#pragma unroll
+    for (int i = 0; i < 4 * MT; ++i) off[i] = s_row[8 * i + (lane >> 3)] * row_bytes + (((lane & 7) ^ (lane >> 3)) << 4);
+}
+// A fragments of k-step s of the stage: lane's row l%32 of each tile, lane half l/32
+struct ALane { uint32_t at[4]; };   // byte offset of chunk 2 i + h in the lane's row of line 0
+DEV ALane a_lane(int lane) {
+    ALane a;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a.at[i] = (lane & 31) * 128 + ((((2 * i + (lane >> 5)) ^ lane) & 7) << 4);
+    return a;
+}
+template <int MT>
+DEV void a_read(uint4 (&ah)[MT], uint4 (&al)[MT], const uint4 *buf, const ALane &a, int s) {
+    const uint8_t *p = reinterpret_cast<const uint8_t *>(buf) + (s >> 1) * (ROWS * 128);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        ah[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1)]);
+        al[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1) + 1]);
+    }
+}
+
+// ---------------------------------------------------------------- gate/up weights
+template <int F> struct GuBlk;                                               // the lane's half of a block
+template <> struct GuBlk<FMT_IQ2> { uint4 q[2]; uint32_t sc, d; };           // 16 grid/sign words, 4 scale bytes
+template <> struct GuBlk<FMT_IQ2S> { uint4 q, sg; uint32_t qh, sc, d; };     // 16 grid bytes, sign bytes, 4 x 8 high bits
+template <int F> constexpr int GU_LOADS = F == FMT_IQ2 ? 4 : 5;              // load instructions of gu_load
+DEV void gu_load(GuBlk<FMT_IQ2> &w, const PfMat &m, uint32_t bi, int h) {
+    w.q[0] = ldu128(m.qs + bi * 64u + 32 * h);
+    w.q[1] = ldu128(m.qs + bi * 64u + 32 * h + 16);
+    w.sc = ldu32(m.p1 + bi * 8u + 4 * h);
+    w.d = ldu16(m.d + bi);
+}
+DEV void gu_load(GuBlk<FMT_IQ2S> &w, const PfMat &m, uint32_t bi, int h) {
+    w.q = ldu128(m.qs + bi * 64u + 16 * h);
+    w.sg = ldu128(m.qs + bi * 64u + 32 + 16 * h);
+    w.qh = ldu32(m.p2 + bi * 8u + 4 * h);
+    w.sc = ldu32(m.p1 + bi * 8u + 4 * h);
+    w.d = ldu16(m.d + bi);
+}
+// IQ2_XS (src/qx_format.c:1914-1933): entry 16h + s is grid word q & 511, sign index q >> 9,
+// scaled by the nibble s / 2 of the lane's four scale bytes
+DEV Codes gu_look(const GuBlk<FMT_IQ2> &w, int s, const uint2 *grid, const uint2 *sgn) {
+    const uint32_t q = word_at(w.q[s >> 3], (s >> 1) & 3) >> (16 * (s & 1));
+    const uint2 m = grid[q & 511u];
+    return Codes{m.x, m.y, sgn[(q >> 9) & 127u]};
+}
+// IQ2_S (src/qx_format.c:1961-1984): grid byte with two high bits, explicit sign byte
+DEV Codes gu_look(const GuBlk<FMT_IQ2S> &w, int s, const uint2 *grid, const uint2 *sgn) {
+    const uint2 m = grid[byte_at(w.q, s) | (((w.qh >> (2 * s)) & 3u) << 8)];
+    return Codes{m.x, m.y, sgn[byte_at(w.sg, s)]};
+}
+
+// k-steps 8 half .. 8 half + 7 of a block: gate (tile 0) and up (1) of the wave's 32 columns.
+// Tile i's codes are looked up two tiles ahead and formed one ahead.
+template <int F, int MT>
+DEV void gu_half(const GuBlk<F> (&w)[2], int half, const uint4 *buf, const ALane &at, f16x (&G)[2][MT], const uint2 *grid,
+                 const uint2 *sgn) {
+    Codes c0 = gu_look(w[0], 8 * half, grid, sgn), c1 = gu_look(w[1], 8 * half, grid, sgn);
+    uint4 ah[MT], al[MT];
+    a_read<MT>(ah, al, buf, at, 0);
+    h2v m[2] = {odd_mul((w[0].sc >> (16 * half)) & 15u), odd_mul((w[1].sc >> (16 * half)) & 15u)};
+    uint4 b = conv(c0, m[0]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int s = i >> 1, f = i & 1, sn = (i + 1) >> 1, fn = (i + 1) & 1;
+        uint4 bn = b, nh[MT], nl[MT];
+        if (i < 15) {
+            if (sn && !(sn & 1)) m[fn] = odd_mul((w[fn].sc >> (16 * half + 4 * (sn >> 1))) & 15u);
+            bn = conv(c1, m[fn]);
+        }
+        if (i < 14) c1 = gu_look(w[f], 8 * half + s + 1, grid, sgn);
+        if (f == 1 && s < 7) a_read<MT>(nh, nl, buf, at, s + 1);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(ah[mt], b, G[f][mt]);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(al[mt], b, G[f][mt]);
+        b = bn;
+        if (f == 1 && s < 7) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) { ah[mt] = nh[mt]; al[mt] = nl[mt]; }
+        }
+    }
+}
+
+// x / y for finite y >= 1 by the hardware reciprocal, one Newton step and a residual
+// correction: within an f32 rounding of the quotient, at a third of the exact division's cost
+DEV float div_ge1(float x, float y) {
+    float r = __builtin_amdgcn_rcpf(y);
+    r = fmaf(fmaf(-y, r, 1.0f), r, r);
+    const float q = x * r;
+    return fmaf(fmaf(-q, y, x), r, q);
+}
+DEV float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }   // 2^e, -126 <= e <= 127
+
+template <int F, int MT>
+DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *list, uint32_t n, const uint2 *grid,
+                 const uint2 *sgn, uint4 *buf, uint32_t *s_row, float *s_xs) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
+    const uint32_t bi = (e * QXG_FFN + 128 * cg + 32 * wave + col) * 8;   // tiles 0 and 1: this row of gate and of up
+    GuBlk<F> cur[2], nxt[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) gu_load(cur[f], a.w[f], bi, h);
+    if (tid < 32 * MT) {
+        const uint32_t t = list[min((uint32_t)tid, n - 1)] >> 3;
+        s_row[tid] = t;
+        s_xs[tid] = a.xs[t];
+    }
+    __syncthreads();   // the rows' tokens, and the tables
+    uint32_t off[4 * MT];
+    stage_offsets<MT>(off, s_row, 8192u, lane);   // 2048 values, 4 bytes each
+    stage_rows<MT>(a.xp, off, 0, buf, wave);
+    const ALane at = a_lane(lane);
+    f16x acc[2][MT];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[f][mt] = zero16();
+#pragma unroll 1
+    for (uint32_t b = 0; b < 8; ++b) {
+        f16x G[2][MT];
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) G[f][mt] = zero16();
+        wait_loads<0>();
+        __syncthreads();   // the block's first half is staged; every wave is past the last block's second half
+        stage_rows<MT>(a.xp, off, 8 * b + 4, buf + STAGE, wave);
+        __builtin_amdgcn_sched_barrier(0);   // the weights' loads stay the youngest: the wait below leaves them in flight
+        const uint32_t bn = b < 7 ? b + 1 : 7;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) gu_load(nxt[f], a.w[f], bi + bn, h);
+        __builtin_amdgcn_sched_barrier(0);
+        gu_half<F, MT>(cur, 0, buf, at, G, grid, sgn);
+        wait_loads<2 * GU_LOADS<F>>();
+        __syncthreads();
+        if (b < 7) stage_rows<MT>(a.xp, off, 8 * b + 8, buf, wave);
+        gu_half<F, MT>(cur, 1, buf + STAGE, at, G, grid, sgn);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            const float d = fp16_exact(cur[f].d) * (0.125f * CODE_SCALE);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[f][mt][r] = fmaf(d, G[f][mt][r], acc[f][mt][r]);
+            cur[f] = nxt[f];
+        }
+    }
+    // SwiGLU (qx_silu, src/qx_format.c:2511-2513, in f32: relative error ~1e-7 against the
+    // reference's double) into LDS, rows of 128 values
+    __syncthreads();
+    float *hs = reinterpret_cast<float *>(buf);
+    constexpr int LD = 132;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
+            const float rs = s_xs[row];
+            float gv = acc[0][mt][r] * rs, uv = acc[1][mt][r] * rs;
+            gv = isfinite(gv) ? gv : 0.0f;   // (src/qx_format.c:4284)
+            uv = isfinite(uv) ? uv : 0.0f;
+            const float ex = expf(-gv);      // (infinite below -88: the quotient is 0)
+            hs[row * LD + 32 * wave + col] = (ex < INFINITY ? div_ge1(gv, 1.0f + ex) : 0.0f) * uv;
+        }
+    __syncthreads();
+    // each row's 128 values become the down projection's packed operand, 16 lanes a row with 8
+    // values each, under a power-of-two scale of their own; a non-finite value makes the
+    // scale a NaN, which zeroes the pair's down row (its own non-finite rule)
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+        const uint32_t row = 16 * i + (tid >> 4), c = tid & 15;
+        // chunk c of the 128 values: k-step and lane half of the down operand's order
+        const uint32_t ks = 8 * cg + (a.h_pairs ? 2 * (c >> 2) + ((c >> 1) & 1) : c & 7), hh = a.h_pairs ? c & 1 : c >> 3;
+        const float *src = hs + row * LD + (a.h_pairs ? 32 * (c >> 2) + 8 * (c & 1) + 4 * ((c >> 1) & 1) : 8 * c);
+        const float4 p = *reinterpret_cast<const float4 *>(src);
+        const float4 q = *reinterpret_cast<const float4 *>(src + (a.h_pairs ? 16 : 4));
+        float v[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+        if (a.h_pairs) { v[1] = q.x; v[2] = p.y; v[3] = q.y; v[4] = p.z; v[5] = q.z; v[6] = p.w; }
+        float mx = 0.0f;
+        bool fin = true;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            fin = fin && isfinite(v[j]);
+            mx = fmaxf(mx, fabsf(v[j]));
+        }
+        mx = fin ? mx : INFINITY;   // the 16 lanes' largest, infinite where a value is not finite
+        mx = fmaxf(mx, dppf<DPP_XOR1>(mx)); mx = fmaxf(mx, dppf<DPP_XOR2>(mx));
+        mx = fmaxf(mx, dppf<DPP_ROR4>(mx)); mx = fmaxf(mx, dppf<DPP_ROR8>(mx));
+        const bool ok = mx < INFINITY;
+        int sh = 140 - (int)(__float_as_uint(mx) >> 23);   // mx 2^sh in [2^13, 2^14) (zero and subnormal: 2^100)
+        sh = sh > 100 ? 100 : sh < -100 ? -100 : sh;
+        if (row < n) {
+            const uint32_t pr = list[row];
+            const float sc = exp2i(sh);
+            h8v hi, lo;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float y = ok ? v[j] * sc : 0.0f;
+                const _Float16 t = (_Float16)y;
+                hi[j] = t;
+                lo[j] = (_Float16)(y - (float)t);
+            }
+            uint8_t *o = a.hp + (uint64_t)pr * 3072 + (ks >> 1) * 128 + (ks & 1) * 64 + hh * 16;
+            *reinterpret_cast<uint4 *>(o) = __builtin_bit_cast(uint4, hi);
+            *reinterpret_cast<uint4 *>(o + 32) = __builtin_bit_cast(uint4, lo);
+            if (c == 0) a.hs[(uint64_t)pr * 8 + cg] = ok ? exp2i(-sh) : __builtin_nanf("");
+        }
+    }
+}
+
+// ---------------------------------------------------------------- down weights
+template <int F> struct DnHalf;                                             // the lane's part of a half block (128 values)
+template <> struct DnHalf<FMT_IQ3> { uint4 q; uint2 aux; uint32_t d; };     // 16 grid bytes, signs and scales
+template <> struct DnHalf<FMT_IQ3S> { uint4 q; uint2 sg; uint32_t qh, sc, d; };   // 16 grid bytes, 8 sign bytes, high bits, scales
+template <> struct DnHalf<FMT_IQ4> { uint2 q[4]; uint2 m; };                // 8 bytes of each of the half's sub-blocks, meta
+DEV void dn_load(DnHalf<FMT_IQ3> &w, const PfMat &m, uint32_t bi, int half, int h) {
+    w.q = ldu128(m.qs + bi * 64u + 32 * half + 16 * h);
+    w.aux = ldu64(m.p1 + bi * 32u + 16 * half + 8 * h);
+    w.d = ldu16(m.d + bi);
+}
+DEV void dn_load(DnHalf<FMT_IQ3S> &w, const PfMat &m, uint32_t bi, int half, int h) {
+    w.q = ldu128(m.qs + bi * 64u + 32 * half + 16 * h);
+    w.sg = ldu64(m.p1 + bi * 32u + 16 * half + 8 * h);
+    w.qh = ldu16(m.p2 + bi * 16u + 4 * half + 2 * h);
+    w.sc = m.p2[bi * 16u + 8 + 2 * half + h];
+    w.d = ldu16(m.d + bi);
+}
+DEV void dn_load(DnHalf<FMT_IQ4> &w, const PfMat &m, uint32_t bi, int half, int h) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w.q[i] = ldu64(m.qs + bi * 128u + 64 * half + 16 * i + 8 * h);
+    w.m = ldu64(m.p1 + bi * 8u);
+}
+// k-step s of the half: entry s of the lane's 8 (sub-block s / 4 of its two)
+// IQ3_XXS (src/qx_format.c:1935-1959)
+DEV Codes dn_look(const DnHalf<FMT_IQ3> &w, int s, const uint32_t *grid, const uint2 *sgn) {
+    return Codes{grid[byte_at(w.q, 2 * s)], grid[byte_at(w.q, 2 * s + 1)], sgn[((s < 4 ? w.aux.x : w.aux.y) >> (7 * (s & 3))) & 127u]};
+}
+DEV h2v dn_mul(const DnHalf<FMT_IQ3> &w, int sub) { return odd_mul((sub ? w.aux.y : w.aux.x) >> 28); }
+// IQ3_S (src/qx_format.c:1986-2030): high index bits in qh, explicit sign bytes, nibble scales
+DEV Codes dn_look(const DnHalf<FMT_IQ3S> &w, int s, const uint32_t *grid, const uint2 *sgn) {
+    const uint32_t i0 = byte_at(w.q, 2 * s) | (((w.qh >> (2 * s)) & 1u) << 8);
+    const uint32_t i1 = byte_at(w.q, 2 * s + 1) | (((w.qh >> (2 * s + 1)) & 1u) << 8);
+    return Codes{grid[i0], grid[i1], sgn[((s < 4 ? w.sg.x : w.sg.y) >> (8 * (s & 3))) & 255u]};
+}
+DEV h2v dn_mul(const DnHalf<FMT_IQ3S> &w, int sub) { return odd_mul((w.sc >> (4 * sub)) & 15u); }
+// IQ4_XS (src/qx_format.c:2032-2053): a byte is the codes of values j and 16 + j of a sub-block
+DEV Codes dn_look(const DnHalf<FMT_IQ4> &w, int s, const uint32_t *kv2, const uint2 *) {
+    const uint32_t q = s & 1 ? w.q[s >> 1].y : w.q[s >> 1].x;
+    return Codes{kv2[q & 255u], kv2[(q >> 8) & 255u], make_uint2(kv2[(q >> 16) & 255u], kv2[q >> 24])};
+}
+DEV h2v dn_mul(const DnHalf<FMT_IQ4> &, int) { return h2v{0, 0}; }
+DEV float dn_scale(const DnHalf<FMT_IQ3> &w, int, int) { return fp16_exact(w.d) * (0.25f * CODE_SCALE); }
+DEV float dn_scale(const DnHalf<FMT_IQ3S> &w, int, int) { return fp16_exact(w.d) * CODE_SCALE; }
+DEV float dn_scale(const DnHalf<FMT_IQ4> &w, int half, int i) {   // sub-block i of the half
+    const int ib = 4 * half + i;
+    const uint32_t sh = w.m.x >> 16, sl = (w.m.y >> (8 * (ib >> 1))) & 255u;
+    const int ls = (int)(((sl >> (4 * (ib & 1))) & 15u) | (((sh >> (2 * ib)) & 3u) << 4));
+    return fp16_exact(w.m.x & 0xffffu) * (float)(ls - 32);
+}
+
+template <int F, int MT>
+DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *list, uint32_t n, const uint32_t *grid,
+                 const uint2 *sgn, uint4 *buf, uint32_t *s_row, float *s_hs) {
+    constexpr bool PER32 = F == FMT_IQ4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
+    uint32_t bi[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) bi[f] = (e * 2048u + 256 * cg + 64 * wave + 32 * f + col) * 3;
+    DnHalf<F> cur[2], nxt[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) dn_load(cur[f], a.w[2], bi[f], 0, h);
+    if (tid < 32 * MT) s_row[tid] = list[min((uint32_t)tid, n - 1)];
+    __syncthreads();   // the rows' pairs, and the tables
+    uint32_t off[4 * MT];
+    stage_offsets<MT>(off, s_row, 3072u, lane);   // 768 values, 4 bytes each
+    stage_rows<MT>(a.hp, off, 0, buf, wave);
+    const ALane at = a_lane(lane);
+    for (int i = tid; i < 6 * 32 * MT; i += 256)   // the rows' scales of each 128 values
+        s_hs[(i / (32 * MT)) * ROWS + i % (32 * MT)] = a.hs[(uint64_t)s_row[i % (32 * MT)] * 8 + i / (32 * MT)];
+    f16x acc[2][MT];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[f][mt] = zero16();
+#pragma unroll 1
+    for (int st = 0; st < 6; ++st) {
+        wait_loads<0>();
+        __syncthreads();   // stage st is in; every wave is past stage st - 1
+        const int sn = st < 5 ? st + 1 : 5;
+        if (st < 5) stage_rows<MT>(a.hp, off, 4 * sn, buf + (sn & 1) * STAGE, wave);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) dn_load(nxt[f], a.w[2], bi[f] + (sn >> 1), sn & 1, h);
+        const uint4 *sb = buf + (st & 1) * STAGE;
+        f16x G[2][MT];
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) G[f][mt] = zero16();
+        // the column's scale (of the block or of sub-block i) times the rows' scales, onto acc
+        auto flush = [&](int f, int i) {
+            const float d = dn_scale(cur[f], st & 1, i);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const f4x hsr = *reinterpret_cast<const f4x *>(s_hs + st * ROWS + 32 * mt + 8 * q + 4 * h);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[f][mt][4 * q + r] = fmaf(d * hsr[r], G[f][mt][4 * q + r], acc[f][mt][4 * q + r]);
+                        if (PER32) G[f][mt][4 * q + r] = 0.0f;
+                    }
+                }
+        };
+        auto form = [&](const Codes &c, int f, int s) {
+            return PER32 ? make_uint4(c.m0, c.m1, c.sg.x, c.sg.y) : conv(c, dn_mul(cur[f], s >> 2));
+        };
+        Codes c1 = dn_look(cur[1], 0, grid, sgn);
+        uint4 ah[MT], al[MT];
+        a_read<MT>(ah, al, sb, at, 0);
+        uint4 b = form(dn_look(cur[0], 0, grid, sgn), 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int s = i >> 1, f = i & 1;
+            uint4 bn = b, nh[MT], nl[MT];
+            if (i < 15) bn = form(c1, (i + 1) & 1, (i + 1) >> 1);
+            if (i < 14) c1 = dn_look(cur[f], s + 1, grid, sgn);
+            if (f == 1 && s < 7) a_read<MT>(nh, nl, sb, at, s + 1);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(ah[mt], b, G[f][mt]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(al[mt], b, G[f][mt]);
+            if (PER32 && (s & 1)) flush(f, s >> 1);
+            b = bn;
+            if (f == 1 && s < 7) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) { ah[mt] = nh[mt]; al[mt] = nl[mt]; }
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            if (!PER32) flush(f, 0);
+            cur[f] = nxt[f];
+        }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (row >= n) continue;
+            float *o = a.y + (uint64_t)s_row[row] * 2048 + 256 * cg + 64 * wave + col;
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const float y = acc[f][mt][r];
+                o[32 * f] = isfinite(y) ? y : 0.0f;   // (src/qx_format.c:4284)
+            }
+        }
+}
+}  // namespace
+
+namespace {
+// The work items are (expert, pass) pairs in expert order: an expert with c pairs has
+// ceil(c / ROWS) passes of evenly many row tiles (real prompts crowd onto a few experts: every
+// pass is its own workgroup, so one expert's passes run side by side).  Every wave finds its
+// workgroup's item from the 128 counts (two a lane, a scan over the wave).
+DEV bool expert_item(const uint32_t *cnt, uint32_t item, uint32_t &e, uint32_t &m0, uint32_t &n) {
+    const int lane = threadIdx.x & 63;
+    const uint2 c = reinterpret_cast<const uint2 *>(cnt)[lane];   // (zero past the last expert)
+    const uint32_t p0 = (c.x + ROWS - 1) / ROWS, p1 = (c.y + ROWS - 1) / ROWS;
+    uint32_t incl = p0 + p1;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
+    }
+    const uint64_t past = __ballot(incl > item);
+    if (!past) return false;
+    const int l = __builtin_ctzll(past);
+    const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(incl - p0 - p1), l);
+    const uint32_t q0 = (uint32_t)__builtin_amdgcn_readlane((int)p0, l), q1 = (uint32_t)__builtin_amdgcn_readlane((int)p1, l);
+    const bool second = item - before >= q0;
+    const uint32_t cc = (uint32_t)__builtin_amdgcn_readlane((int)(second ? c.y : c.x), l);
+    const uint32_t pass = item - before - (second ? q0 : 0u), passes = second ? q1 : q0;
+    const uint32_t tiles = (cc + 31) / 32, rows = (tiles + passes - 1) / passes * 32;
+    e = 2u * l + second;
+    m0 = pass * rows;
+    n = m0 < cc ? min(rows, cc - m0) : 0u;
+    return n != 0;
+}
+}  // namespace
+
+// Workgroup L of the grid (XCD L % 8, round-robin): the column groups of an item run on one
+// XCD, so the item's gathered rows are fetched into one L2.
+#define EXPERT_TILE(GROUPS)                                                                        \
+    const uint32_t j_ = blockIdx.x >> 3, cg = j_ % (GROUPS);                                       \
+    uint32_t e, m0, n;                                                                             \
+    if (!expert_item(a.cnt, (j_ / (GROUPS)) * 8 + (blockIdx.x & 7u), e, m0, n)) return;            \
+    const uint32_t *list = a.list + (uint64_t)e * QXP_LIST + m0;
+
+template <int F>
+__global__ __launch_bounds__(256, 2) void qxp_gate_up(PfExperts a, PfTables P) {
+    EXPERT_TILE(6u)
+    constexpr int NG = F == FMT_IQ2 ? 512 : 1024, NS = F == FMT_IQ2 ? 128 : 256;
+    __shared__ uint2 s_grid[NG], s_sgn[NS];
+    __shared__ uint4 s_buf[2 * STAGE];   // two stages; the epilogue's rows of 132 floats
+    __shared__ uint32_t s_row[ROWS];
+    __shared__ float s_xs[ROWS];
+    for (int i = threadIdx.x; i < NG; i += 256) s_grid[i] = (F == FMT_IQ2 ? P.g2 : P.g2s)[i];
+    for (int i = threadIdx.x; i < NS; i += 256) s_sgn[i] = (F == FMT_IQ2 ? P.sg7 : P.sg8)[i];
+    if (n <= 32) gu_pass<F, 1>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
+    else gu_pass<F, 2>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
+}
+
+template <int F>
+__global__ __launch_bounds__(256, 2) void qxp_down(PfExperts a, PfTables P) {
+    EXPERT_TILE(8u)
+    constexpr int NG = F == FMT_IQ3S ? 512 : 256, NS = F == FMT_IQ3 ? 128 : F == FMT_IQ3S ? 256 : 1;
+    __shared__ uint32_t s_grid[NG];
+    __shared__ uint2 s_sgn[NS];
+    __shared__ uint4 s_buf[2 * STAGE];
+    __shared__ uint32_t s_row[ROWS];
+    __shared__ float s_hs[6 * ROWS];
+    for (int i = threadIdx.x; i < NG; i += 256) s_grid[i] = (F == FMT_IQ3 ? P.g3 : F == FMT_IQ3S ? P.g3s : P.kv2)[i];
+    if (NS > 1) for (int i = threadIdx.x; i < NS; i += 256) s_sgn[i] = (F == FMT_IQ3 ? P.sg7 : P.sg8)[i];
+    if (n <= 32) dn_pass<F, 1>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
+    else dn_pass<F, 2>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
+}
+
+extern "C" {
+// gate/up (IQ2_XS or IQ2_S) and down (IQ3_XXS, IQ3_S or IQ4_XS) of T tokens; the grid holds
+// the most items T tokens can make
+static uint32_t item_bound(const PfExperts &a, uint32_t T) {
+    const uint32_t pairs = T * QXG_TOPK, most = pairs / ROWS + (a.experts < pairs ? a.experts : pairs);
+    return (most + 7) / 8 * 8;
+}
+void qxp_launch_gate_up(hipStream_t s, uint32_t type, const PfExperts &a, const PfTables &P, uint32_t T, Timer tm) {
+    const dim3 grid(6 * item_bound(a, T));
+    if (type == 22) qx_launch(qxp_gate_up<FMT_IQ2S>, grid, dim3(256), 0, s, tm, a, P);
+    else qx_launch(qxp_gate_up<FMT_IQ2>, grid, dim3(256), 0, s, tm, a, P);
+}
+void qxp_launch_down(hipStream_t s, uint32_t type, const PfExperts &a, const PfTables &P, uint32_t T, Timer tm) {
+    const dim3 grid(8 * item_bound(a, T));
+    if (type == 21) qx_launch(qxp_down<FMT_IQ3S>, grid, dim3(256), 0, s, tm, a, P);
+    else if (type == 23) qx_launch(qxp_down<FMT_IQ4>, grid, dim3(256), 0, s, tm, a, P);
+    else qx_launch(qxp_down<FMT_IQ3>, grid, dim3(256), 0, s, tm, a, P);
+}
+}

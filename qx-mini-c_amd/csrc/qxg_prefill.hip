@@ -4,8 +4,8 @@
 // and every expert matrix is one GEMM over the tokens (or over the tokens routed to
 // that expert) on the matrix cores.
 //
-// Precision scheme of the GEMMs (fp16 MFMA 32x32x16, f32 accumulation).  Every
-// weight of the formats used is, exactly,
+// Precision scheme of the GEMMs (fp16 MFMA, f32 accumulation).  Every weight of the
+// formats used is, exactly,
 //     IQ2_XS   w = (d/8) * [(2s+1) * grid * sign]        |code| <= 31*43 = 1333
 //     IQ3_XXS  w = (d/4) * [(2a+1) * grid * sign]        |code| <= 31*62 = 1922
 //     IQ4_XS   w = (d*(ls-32)) * kvalue                  |code| <= 127
@@ -15,13 +15,13 @@
 // lo fp16, |e| <= 2^-22 |x*s|.  A code times an fp16 value is exact in f32; the matrix
 // cores sum the products in f32 over one block (IQ2_XS, IQ3_XXS: 256 values) or one
 // group (IQ4_XS: 32 values), that partial sum is multiplied by its f32 scale once, and
-// the row result is divided by s.  The integer codes come from fp16 codebooks in LDS.
+// the row result is divided by s.  The routed experts' GEMMs are in qxg_pf_experts.hip.
 //
-// MFMA operand layout (v_mfma_f32_32x32x16_f16): lane l holds, for A, row l%32 and
-// k = 8*(l/32) + j (j < 8); for B, column l%32 and the same k; result register r of
-// lane l is (row 8*(r/4) + 4*(l/32) + r%4, column l%32).  Rows are tokens (or expert
-// slots), columns are weight rows, so each lane's results share one weight row and
-// its scale.  Activations are packed once per GEMM in exactly this fragment order:
+// Dense GEMMs (Q/K/V, O): MFMA operand layout of v_mfma_f32_32x32x16_f16: lane l holds,
+// for A, row l%32 and k = 8*(l/32) + j (j < 8); for B, column l%32 and the same k; result
+// register r of lane l is (row 8*(r/4) + 4*(l/32) + r%4, column l%32).  Rows are tokens,
+// columns are weight rows, so each lane's results share one weight row and its scale.
+// Activations are packed once per GEMM in exactly this fragment order:
 //     apk[((mtile * KS + kstep) * 2 + piece) * 64 + lane] = 8 fp16 values (uint4).
 #include "qxg_dev.h"
 
@@ -30,45 +30,22 @@ typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f16x __attribute__((ext_vector_type(16)));
 
-enum { FMT_IQ4 = 0, FMT_IQ2 = 1, FMT_IQ3 = 2, FMT_Q5 = 3, FMT_IQ2S = 4, FMT_IQ3S = 5 };
-enum { EPI_STORE = 0, EPI_RESID = 1, EPI_SWIGLU = 2 };
+enum { FMT_IQ4 = 0, FMT_Q5 = 3 };
+enum { EPI_STORE = 0, EPI_RESID = 1 };
 
 DEV f16x mfma(uint4 a, uint4 b, f16x c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, a), __builtin_bit_cast(h8v, b), c, 0, 0, 0);
 }
 
-DEV uint32_t hmul2(uint32_t v, h2v m) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, v) * m); }
-DEV uint4 hmul8(uint4 v, uint32_t mul) {
-    const _Float16 f = (_Float16)(float)mul;   // 1..31: exact
-    const h2v m = {f, f};
-    return make_uint4(hmul2(v.x, m), hmul2(v.y, m), hmul2(v.z, m), hmul2(v.w, m));
-}
 DEV uint32_t comp(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
 // ---------------------------------------------------------------- weight blocks per lane
 // The lane's share of one 256-value block of its weight row: lane half h = l/32 takes
 // k = 16*s + 8*h + j of every k-step s (16 per block).
 template <int F> struct Blk;
-template <> struct Blk<FMT_IQ2> { uint4 q[4]; uint2 sc; uint32_t d; };    // qs (32 x u16), scales, d
-template <> struct Blk<FMT_IQ3> { uint4 q[4]; uint4 a[2]; uint32_t d; };  // qs (64 x u8), aux (8 x u32), d
 template <> struct Blk<FMT_IQ4> { uint2 q[8]; uint2 m; };                 // qs bytes 16ib+8h..+8, meta
 template <> struct Blk<FMT_Q5> { uint2 q[8]; uint2 qh[2]; uint4 m; };     // qs 32p+16t+8h..+8, qh 16t+8h..+8, meta
-template <> struct Blk<FMT_IQ2S> { uint4 g[2], sg[2]; uint2 qh, sc; uint32_t d; };   // grid, sign, qh, scale bytes
-template <> struct Blk<FMT_IQ3S> { uint4 q[4], sg[2], hs; uint32_t d; };  // grid, sign bytes, {qh[8], scales[4]}
 
-DEV void blk_load(Blk<FMT_IQ2> &b, const PfMat &w, uint64_t bi, int) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(w.qs + bi * 64);
-    b.q[0] = p[0]; b.q[1] = p[1]; b.q[2] = p[2]; b.q[3] = p[3];
-    b.sc = *reinterpret_cast<const uint2 *>(w.p1 + bi * 8);
-    b.d = w.d[bi];
-}
-DEV void blk_load(Blk<FMT_IQ3> &b, const PfMat &w, uint64_t bi, int) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(w.qs + bi * 64);
-    b.q[0] = p[0]; b.q[1] = p[1]; b.q[2] = p[2]; b.q[3] = p[3];
-    const uint4 *a = reinterpret_cast<const uint4 *>(w.p1 + bi * 32);
-    b.a[0] = a[0]; b.a[1] = a[1];
-    b.d = w.d[bi];
-}
 DEV void blk_load(Blk<FMT_IQ4> &b, const PfMat &w, uint64_t bi, int h) {
     const uint8_t *q = w.qs + bi * 128 + 8 * h;
 #pragma unroll
@@ -84,53 +61,11 @@ DEV void blk_load(Blk<FMT_Q5> &b, const PfMat &w, uint64_t bi, int h) {
     b.qh[1] = *reinterpret_cast<const uint2 *>(w.p2 + bi * 32 + 16 + 8 * h);
     b.m = *reinterpret_cast<const uint4 *>(w.p1 + bi * 16);
 }
-DEV void blk_load(Blk<FMT_IQ2S> &b, const PfMat &w, uint64_t bi, int) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(w.qs + bi * 64);
-    b.g[0] = p[0]; b.g[1] = p[1]; b.sg[0] = p[2]; b.sg[1] = p[3];
-    b.qh = *reinterpret_cast<const uint2 *>(w.p2 + bi * 8);
-    b.sc = *reinterpret_cast<const uint2 *>(w.p1 + bi * 8);
-    b.d = w.d[bi];
-}
-DEV void blk_load(Blk<FMT_IQ3S> &b, const PfMat &w, uint64_t bi, int) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(w.qs + bi * 64);
-    b.q[0] = p[0]; b.q[1] = p[1]; b.q[2] = p[2]; b.q[3] = p[3];
-    const uint4 *g = reinterpret_cast<const uint4 *>(w.p1 + bi * 32);
-    b.sg[0] = g[0]; b.sg[1] = g[1];
-    b.hs = *reinterpret_cast<const uint4 *>(w.p2 + bi * 16);
-    b.d = w.d[bi];
-}
-DEV uint32_t byte_of(const uint4 (&v)[2], uint32_t i) { return (comp(v[i >> 4], (i >> 2) & 3) >> (8 * (i & 3))) & 255u; }
-DEV uint32_t byte_of4(const uint4 (&v)[4], uint32_t i) { return (comp(v[i >> 4], (i >> 2) & 3) >> (8 * (i & 3))) & 255u; }
-
-// B fragment of k-step s (8 fp16 codes).  IQ2_XS (src/qx_format.c:1914-1933): element
-// 32ib+8l+j = db(l<2 ? lo : hi nibble of scales[ib]) * grid[q&511][j] * sign, q = qs[4ib+l];
-// k-step s = 2ib + l/2, so q = qs[2s + h] and the nibble is s&1.
-DEV uint4 frag(const Blk<FMT_IQ2> &b, int s, int h, const uint4 *G2, const uint4 *SG, const uint32_t *) {
-    const uint32_t q = (comp(b.q[s >> 2], s & 3) >> (16 * h)) & 0xffffu;
-    const uint32_t scb = ((s >> 1) < 4 ? b.sc.x : b.sc.y) >> (8 * ((s >> 1) & 3));
-    const uint32_t nib = (scb >> (4 * (s & 1))) & 15u;
-    uint4 g = G2[q & 511u];
-    const uint4 m = SG[q >> 9];
-    g.x ^= m.x; g.y ^= m.y; g.z ^= m.z; g.w ^= m.w;
-    return hmul8(g, 2u * nib + 1u);
-}
-// IQ3_XXS (src/qx_format.c:1935-1959): element 32ib+8l+j (j<4) from grid3[qs[8ib+2l]],
-// j>=4 from grid3[qs[8ib+2l+1]], signs ksigns[(aux[ib] >> 7l) & 127], scale
-// d*(2(aux>>28)+1)/4; k-step s = 2ib + l/2.
-DEV uint4 frag(const Blk<FMT_IQ3> &b, int s, int h, const uint4 *, const uint4 *SG, const uint32_t *G3) {
-    const int ib = s >> 1, l = 2 * (s & 1) + h;
-    const uint32_t dw = comp(b.q[ib >> 1], (2 * ib + (s & 1)) & 3) >> (16 * h);
-    const uint32_t aux = comp(b.a[ib >> 2], ib & 3);
-    const uint2 g1 = reinterpret_cast<const uint2 *>(G3)[dw & 255u];
-    const uint2 g2 = reinterpret_cast<const uint2 *>(G3)[(dw >> 8) & 255u];
-    const uint4 m = SG[(aux >> (7 * l)) & 127u];
-    const uint4 g = make_uint4(g1.x ^ m.x, g1.y ^ m.y, g2.x ^ m.z, g2.y ^ m.w);
-    return hmul8(g, 2u * (aux >> 28) + 1u);
-}
+// B fragment of k-step s (8 fp16 codes).
 // IQ4_XS (src/qx_format.c:2032-2053): element 32ib+j = kvalue[qs[16ib+j] & 15],
 // 32ib+16+j = kvalue[qs[16ib+j] >> 4]; k-step 2ib takes the low nibbles of the lane's
 // 8 bytes, 2ib+1 the high nibbles.
-DEV uint4 frag(const Blk<FMT_IQ4> &b, int s, int, const uint4 *, const uint4 *, const uint32_t *KV2) {
+DEV uint4 frag(const Blk<FMT_IQ4> &b, int s, const uint32_t *KV2) {
     const uint2 q = b.q[s >> 1];
     uint32_t p[8];
 #pragma unroll
@@ -149,7 +84,7 @@ DEV uint32_t u8pair_h2(uint32_t w4, bool hi) {
     const h2v k = {(_Float16)1024.0f, (_Float16)1024.0f};
     return __builtin_bit_cast(uint32_t, v - k);
 }
-DEV uint4 frag(const Blk<FMT_Q5> &b, int s, int, const uint4 *, const uint4 *, const uint32_t *) {
+DEV uint4 frag(const Blk<FMT_Q5> &b, int s, const uint32_t *) {
     const int ib = s >> 1, t = s & 1;
     const uint2 q = b.q[2 * (ib >> 1) + t], qh = b.qh[t];
     const uint32_t nsh = 4 * (ib & 1);
@@ -157,47 +92,12 @@ DEV uint4 frag(const Blk<FMT_Q5> &b, int s, int, const uint4 *, const uint4 *, c
     const uint32_t c1 = ((q.y >> nsh) & 0x0f0f0f0fu) | (((qh.y >> ib) & 0x01010101u) << 4);
     return make_uint4(u8pair_h2(c0, false), u8pair_h2(c0, true), u8pair_h2(c1, false), u8pair_h2(c1, true));
 }
-// IQ2_S (src/qx_format.c:1961-1984): entry e = 4ib + l (l = 2t + h) of the block: grid
-// index qs[e] | ((qh[ib] >> 2l) & 3) << 8, explicit sign byte qs[32 + e], halves scaled by
-// the nibble t of scales[ib] as IQ2_XS.
-DEV uint4 frag(const Blk<FMT_IQ2S> &b, int s, int h, const uint4 *G2S, const uint4 *SG8, const uint32_t *) {
-    const int ib = s >> 1, t = s & 1, l = 2 * t + h;
-    const uint32_t e = 4 * ib + l;
-    const uint32_t qh = ((ib < 4 ? b.qh.x : b.qh.y) >> (8 * (ib & 3))) & 255u;
-    const uint32_t idx = byte_of(b.g, e) | (((qh >> (2 * l)) & 3u) << 8);
-    uint4 g = G2S[idx];
-    const uint4 m = SG8[byte_of(b.sg, e)];
-    g.x ^= m.x; g.y ^= m.y; g.z ^= m.z; g.w ^= m.w;
-    const uint32_t scb = ((ib < 4 ? b.sc.x : b.sc.y) >> (8 * (ib & 3))) & 255u;
-    return hmul8(g, 2u * ((scb >> (4 * t)) & 15u) + 1u);
-}
-// IQ3_S (src/qx_format.c:1986-2030): k-step s = 2ib + t, lane half h: grid entries
-// e = 8ib + 4t + 2h + {0, 1} (4 values each), index qs[e] | (bit e%8 of qh[ib]) << 8, sign
-// byte signs[4ib + 2t + h], scale d*(2 sc + 1), sc the nibble ib&1 of scales[ib/2].
-DEV uint4 frag(const Blk<FMT_IQ3S> &b, int s, int h, const uint4 *, const uint4 *SG8, const uint32_t *G3S) {
-    const int ib = s >> 1, t = s & 1;
-    const uint32_t e = 8 * ib + 4 * t + 2 * h;
-    const uint32_t qh = (comp(b.hs, ib >> 2) >> (8 * (ib & 3))) & 255u;
-    const uint32_t i1 = byte_of4(b.q, e) | (((qh >> (e & 7)) & 1u) << 8);
-    const uint32_t i2 = byte_of4(b.q, e + 1) | (((qh >> ((e + 1) & 7)) & 1u) << 8);
-    const uint2 g1 = reinterpret_cast<const uint2 *>(G3S)[i1];
-    const uint2 g2 = reinterpret_cast<const uint2 *>(G3S)[i2];
-    const uint4 m = SG8[byte_of(b.sg, 4 * ib + 2 * t + h)];
-    const uint4 g = make_uint4(g1.x ^ m.x, g1.y ^ m.y, g2.x ^ m.z, g2.y ^ m.w);
-    const uint32_t scw = (b.hs.z >> (8 * (ib >> 1))) & 255u;
-    return hmul8(g, 2u * ((scw >> (4 * (ib & 1))) & 15u) + 1u);
-}
-
-// f32 scale of the partial sums: the block's d/8 or d/4; IQ4_XS: group ib's d*(ls-32)
-DEV float blk_scale(const Blk<FMT_IQ2> &b, int) { return fp16_exact(b.d) * 0.125f; }
-DEV float blk_scale(const Blk<FMT_IQ3> &b, int) { return fp16_exact(b.d) * 0.25f; }
+// f32 scale of the partial sums: group ib's d*(ls-32)
 DEV float blk_scale(const Blk<FMT_IQ4> &b, int ib) {
     const uint32_t sh = b.m.x >> 16, sl = (b.m.y >> (8 * (ib >> 1))) & 255u;
     const int ls = (int)(((sl >> (4 * (ib & 1))) & 15u) | (((sh >> (2 * ib)) & 3u) << 4));
     return fp16_exact(b.m.x & 0xffffu) * (float)(ls - 32);
 }
-DEV float blk_scale(const Blk<FMT_IQ2S> &b, int) { return fp16_exact(b.d) * 0.125f; }
-DEV float blk_scale(const Blk<FMT_IQ3S> &b, int) { return fp16_exact(b.d); }
 // Q5_K sub-block ib: scale d*sc and offset dmin*m (6-bit sc, m: get_scale_min_k4,
 // src/qx_format.c:2079-2087); meta = {d, dmin, scales[12]}
 DEV uint32_t q5_scale_byte(const uint4 &m, int i) { return (comp(m, 1 + (i >> 2)) >> (8 * (i & 3))) & 255u; }
@@ -231,216 +131,60 @@ DEV f16x zero16() {
 }  // namespace
 
 // ================================================================= GEMM
-// One wave: NSUB column tiles of 32 weight rows x NM row tiles of 32 tokens/slots, over
-// all of K.  GU: the two column tiles are gate and up at the same rows (SwiGLU epilogue).
-// Workgroup = 4 waves on 4 consecutive column tiles of the same row tiles.  The row
-// tiles' fragments of one 256-value block (32 KiB per row tile) are copied by the whole
-// workgroup into one of two LDS stages while the previous block is multiplied, and the
-// next block's weights are loaded into registers at the same time, so each block's
-// loads have one block of matrix work to arrive.  The loop has no data-dependent
-// branches: the last iteration re-loads the last block (never used).
-struct GemmLds {
-    uint4 *g2, *sg, *a;   // a: two stages of `stage` uint4 each
-    uint32_t *t;
-    uint32_t stage;
-};
-
-// A fragments of block kb of NM row tiles: thread tid holds uint4 tid + 256*i (i < 8),
-// kept in native 4-dword vectors (register-promoted; the uint4 struct array is not)
+// One wave: a column tile of 32 weight rows x a row tile of 32 tokens, over all of K.
+// Workgroup = 4 waves on 4 consecutive column tiles of the same row tile.  The row tile's
+// fragments of one 256-value block (32 KiB) are copied by the whole workgroup into one of
+// two LDS stages while the previous block is multiplied, and the next block's weights are
+// loaded into registers at the same time, so each block's loads have one block of matrix
+// work to arrive.  The loop has no data-dependent branches: the last iteration re-loads the
+// last block (never used).
+// A fragments of block kb: thread tid holds uint4 tid + 256*i (i < 8), kept in native
+// 4-dword vectors (register-promoted; the uint4 struct array is not)
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-template <int NM>
-DEV void a_load(v4u (&ra)[NM * 8], const uint4 *A, uint32_t KS, uint32_t kb) {
+DEV void a_load(v4u (&ra)[8], const uint4 *A, uint32_t kb) {
     const v4u *a = reinterpret_cast<const v4u *>(A);
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ra[m * 8 + i] = a[((uint64_t)m * KS + kb * 16) * 128 + 256 * i];
+    for (int i = 0; i < 8; ++i) ra[i] = a[(uint64_t)kb * 16 * 128 + 256 * i];
 }
-template <int NM>
-DEV void a_store(const v4u (&ra)[NM * 8], uint4 *stage, int tid) {
+DEV void a_store(const v4u (&ra)[8], uint4 *stage, int tid) {
     v4u *st = reinterpret_cast<v4u *>(stage);
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) st[m * 2048 + tid + 256 * i] = ra[m * 8 + i];
+    for (int i = 0; i < 8; ++i) st[tid + 256 * i] = ra[i];
 }
 
-// the 16 k-steps of one block: partial sums per block (IQ2_XS, IQ3_XXS) or per group of
-// two k-steps (IQ4_XS), each scaled once into acc
-template <int F, int NSUB, int NM>
-DEV void block_mma(const Blk<F> (&bk)[NSUB], const uint4 *sa, f16x (&acc)[NSUB][NM], const GemmLds &L, int h,
-                   int lane) {
-    constexpr bool PER32 = F == FMT_IQ4 || F == FMT_Q5;   // a scale per 32-value group
-    constexpr int NG = PER32 ? 8 : 1;
-    float scl[NSUB][NG], ofs[NSUB][NG];
+// the 16 k-steps of one block: partial sums per group of two k-steps, each scaled once into acc
+template <int F>
+DEV void block_mma(const Blk<F> &bk, const uint4 *sa, f16x &acc, const uint32_t *t, int lane) {
+    float scl[8], ofs[8];
 #pragma unroll
-    for (int n = 0; n < NSUB; ++n)
-#pragma unroll
-        for (int q = 0; q < NG; ++q) {
-            scl[n][q] = blk_scale(bk[n], q);
-            ofs[n][q] = F == FMT_Q5 ? blk_offset(bk[n], q) : 0.0f;
-        }
-    f16x G[NSUB][NM];
-    f16x S[NM];   // Q5_K: sums of the activations over the group (B = all ones), for the dmin term
-#pragma unroll
-    for (int n = 0; n < NSUB; ++n)
-#pragma unroll
-        for (int m = 0; m < NM; ++m) G[n][m] = zero16();
-#pragma unroll
-    for (int m = 0; m < NM; ++m) S[m] = zero16();
+    for (int q = 0; q < 8; ++q) {
+        scl[q] = blk_scale(bk, q);
+        ofs[q] = F == FMT_Q5 ? blk_offset(bk, q) : 0.0f;
+    }
+    f16x G = zero16(), S = zero16();   // S, Q5_K: sums of the activations over the group (B = all ones), for the dmin term
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
-        uint4 ah[NM], al[NM];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            ah[m] = sa[m * 2048 + s * 128 + lane];
-            al[m] = sa[m * 2048 + s * 128 + 64 + lane];
-        }
+        const uint4 ah = sa[s * 128 + lane], al = sa[s * 128 + 64 + lane];
         if (F == FMT_Q5) {
             const uint4 ones = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);   // fp16 1.0
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                S[m] = mfma(ah[m], ones, S[m]);
-                S[m] = mfma(al[m], ones, S[m]);
-            }
+            S = mfma(ah, ones, S);
+            S = mfma(al, ones, S);
         }
+        const uint4 b = frag(bk, s, t);
+        G = mfma(ah, b, G);
+        G = mfma(al, b, G);
+        if (s & 1) {
 #pragma unroll
-        for (int n = 0; n < NSUB; ++n) {
-            const uint4 b = frag(bk[n], s, h, L.g2, L.sg, L.t);
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                G[n][m] = mfma(ah[m], b, G[n][m]);
-                G[n][m] = mfma(al[m], b, G[n][m]);
+            for (int r = 0; r < 16; ++r) {
+                acc[r] = fmaf(scl[s >> 1], G[r], acc[r]);
+                if (F == FMT_Q5) acc[r] = fmaf(-ofs[s >> 1], S[r], acc[r]);
             }
-        }
-        if (PER32 && (s & 1)) {
-#pragma unroll
-            for (int n = 0; n < NSUB; ++n)
-#pragma unroll
-                for (int m = 0; m < NM; ++m) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        acc[n][m][r] = fmaf(scl[n][s >> 1], G[n][m][r], acc[n][m][r]);
-                        if (F == FMT_Q5) acc[n][m][r] = fmaf(-ofs[n][s >> 1], S[m][r], acc[n][m][r]);
-                    }
-                    G[n][m] = zero16();
-                }
-            if (F == FMT_Q5)
-#pragma unroll
-                for (int m = 0; m < NM; ++m) S[m] = zero16();
+            G = zero16();
+            if (F == FMT_Q5) S = zero16();
         }
         // LDS reads of later k-steps stay behind this point: the unrolled loop would
         // otherwise hoist all of them into registers
         if (s & 1) asm volatile("" ::: "memory");
-    }
-    if (!PER32) {
-#pragma unroll
-        for (int n = 0; n < NSUB; ++n)
-#pragma unroll
-            for (int m = 0; m < NM; ++m)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[n][m][r] = fmaf(scl[n][0], G[n][m][r], acc[n][m][r]);
-    }
-}
-
-template <int F, int NSUB, int NM, int EPI>
-DEV void gemm_body(const PfGemm &g, const GemmLds &L, uint32_t e, uint32_t mt0, uint32_t bx) {
-    constexpr bool GU = EPI == EPI_SWIGLU;
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
-    const uint32_t KB = g.kb, KS = 16 * KB;
-    const uint32_t nt = bx * 4 + wave;                    // column tile group of this wave
-    const uint32_t c0 = GU ? 32 * nt : 32 * NSUB * nt;     // first output column
-    PfMat W[NSUB];
-    uint64_t rowblk[NSUB];
-#pragma unroll
-    for (int n = 0; n < NSUB; ++n) {
-        const uint32_t c = GU ? c0 : c0 + 32 * n;
-        const int mi = GU ? n : (c >= g.w_start[2] ? 2 : c >= g.w_start[1] ? 1 : 0);
-        W[n] = g.w[mi];
-        const uint32_t r = (GU ? c0 : c - g.w_start[mi]) + col;
-        rowblk[n] = ((uint64_t)e * g.rows + r) * KB;
-    }
-    const uint4 *A = g.apk + (uint64_t)mt0 * KS * 128 + tid;
-    uint4 *stage0 = L.a, *stage1 = L.a + L.stage;
-
-    f16x acc[NSUB][NM];
-#pragma unroll
-    for (int n = 0; n < NSUB; ++n)
-#pragma unroll
-        for (int m = 0; m < NM; ++m) acc[n][m] = zero16();
-    // weights of even blocks in b0, odd blocks in b1; A of block kb in stage kb&1
-    Blk<F> b0[NSUB], b1[NSUB];
-    v4u ra[NM * 8];
-    const uint32_t k1 = KB > 1 ? 1 : 0;
-#pragma unroll
-    for (int n = 0; n < NSUB; ++n) blk_load(b0[n], W[n], rowblk[n], h);
-    a_load<NM>(ra, A, KS, 0);
-    a_store<NM>(ra, stage0, tid);
-    a_load<NM>(ra, A, KS, k1);
-#pragma unroll
-    for (int n = 0; n < NSUB; ++n) blk_load(b1[n], W[n], rowblk[n] + k1, h);
-    __syncthreads();   // tables and stage 0
-
-    // per block: multiply, stage the next block's A (its stage was last read two blocks
-    // back, before the barrier that ended the previous block), then start the loads of
-    // the block after it (clamped to the last block: always in bounds, never used)
-#pragma unroll 1
-    for (uint32_t kb = 0; kb < KB; kb += 2) {
-        block_mma<F, NSUB, NM>(b0, stage0, acc, L, h, lane);
-        a_store<NM>(ra, stage1, tid);
-        {
-            const uint32_t kn = kb + 2 < KB ? kb + 2 : KB - 1;
-            a_load<NM>(ra, A, KS, kn);
-#pragma unroll
-            for (int n = 0; n < NSUB; ++n) blk_load(b0[n], W[n], rowblk[n] + kn, h);
-        }
-        __syncthreads();
-        if (kb + 1 >= KB) break;
-        block_mma<F, NSUB, NM>(b1, stage1, acc, L, h, lane);
-        a_store<NM>(ra, stage0, tid);
-        {
-            const uint32_t kn = kb + 3 < KB ? kb + 3 : KB - 1;
-            a_load<NM>(ra, A, KS, kn);
-#pragma unroll
-            for (int n = 0; n < NSUB; ++n) blk_load(b1[n], W[n], rowblk[n] + kn, h);
-        }
-        __syncthreads();
-    }
-
-    // epilogue: lane's column c, rows 8*(r/4) + 4h + r%4 of each row tile
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        const uint32_t rbase = (mt0 + m) * 32 + 4 * h;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t row = rbase + 8 * (r >> 2) + (r & 3);
-            if (!g.mgroups && row >= g.nvalid) continue;
-            const float rs = g.rscale[row];
-            if (EPI == EPI_SWIGLU) {
-                float gv = acc[0][m][r] * rs, uv = acc[1][m][r] * rs;
-                gv = isfinite(gv) ? gv : 0.0f;
-                uv = isfinite(uv) ? uv : 0.0f;
-                // qx_silu (src/qx_format.c:2511-2513) in f32: relative error ~1e-7 against the
-                // reference's double, far inside the 1e-5 bar; a double exp per output was a
-                // large share of the epilogue
-                const float sg = gv / (1.0f + expf(-gv));
-                g.out[(uint64_t)row * g.ld + c0 + col] = sg * uv;
-            } else {
-#pragma unroll
-                for (int n = 0; n < NSUB; ++n) {
-                    const uint32_t c = c0 + 32 * n + col;
-                    float y = acc[n][m][r] * rs;
-                    y = isfinite(y) ? y : 0.0f;   // non-finite projection outputs -> 0 (src/qx_format.c:4284)
-                    const uint64_t o = (uint64_t)row * g.ld + c;
-                    if (EPI == EPI_RESID) {
-                        if (g.dump) g.dump[o] = y;
-                        g.out[o] = g.resid[o] + y;
-                    } else {
-                        g.out[o] = y;
-                    }
-                }
-            }
-        }
     }
 }
 
@@ -458,39 +202,69 @@ DEV void xcd_tile(uint32_t a, uint32_t &bx, uint32_t &by) {
     by = (j / nxb) * a + r / b;
 }
 
-template <int F, int NSUB, int MT, int EPI>
-__global__ __launch_bounds__(256, MT == 1 && F != FMT_IQ2S ? 2 : 1) void qxp_gemm(PfGemm g, PfTables P) {   // (IQ2_S: 86 KB of LDS, one per CU)
-    uint32_t e = 0, mt0, nmt, bx, by;
-    xcd_tile(g.xcd_rows, bx, by);
-    if (g.mgroups) {
-        if (by >= g.meta[0]) return;   // whole workgroup
-        const uint32_t mg = g.mgroups[by];
-        e = mg & 255u; mt0 = (mg >> 8) & 0xfffu; nmt = mg >> 20;
-    } else {
-        mt0 = by * MT;
-        if (mt0 >= g.mtiles) return;   // whole workgroup: a padding row
-        nmt = min((uint32_t)MT, g.mtiles - mt0);
+template <int F, int EPI>
+__global__ __launch_bounds__(256, 2) void qxp_gemm(PfGemm g, PfTables P) {
+    uint32_t bx, mt0;
+    xcd_tile(g.xcd_rows, bx, mt0);
+    if (mt0 >= g.mtiles) return;   // whole workgroup: a padding row
+    __shared__ uint32_t s_t[F == FMT_IQ4 ? 256 : 1];
+    __shared__ uint4 s_a[2 * 2048];   // [stage][(kstep*2 + piece)*64 + lane]
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
+    if (F == FMT_IQ4) s_t[tid] = P.kv2[tid];
+    const uint32_t KB = g.kb, KS = 16 * KB;
+    const uint32_t c = 32 * (bx * 4 + wave);   // first output column
+    const int mi = c >= g.w_start[2] ? 2 : c >= g.w_start[1] ? 1 : 0;
+    const PfMat W = g.w[mi];
+    const uint64_t rowblk = (uint64_t)(c - g.w_start[mi] + col) * KB;
+    const uint4 *A = g.apk + (uint64_t)mt0 * KS * 128 + tid;
+    uint4 *stage0 = s_a, *stage1 = s_a + 2048;
+
+    f16x acc = zero16();
+    // weights of even blocks in b0, odd blocks in b1; A of block kb in stage kb&1
+    Blk<F> b0, b1;
+    v4u ra[8];
+    const uint32_t k1 = KB > 1 ? 1 : 0;
+    blk_load(b0, W, rowblk, h);
+    a_load(ra, A, 0);
+    a_store(ra, stage0, tid);
+    a_load(ra, A, k1);
+    blk_load(b1, W, rowblk + k1, h);
+    __syncthreads();   // tables and stage 0
+
+    // per block: multiply, stage the next block's A (its stage was last read two blocks
+    // back, before the barrier that ended the previous block), then start the loads of
+    // the block after it (clamped to the last block: always in bounds, never used)
+#pragma unroll 1
+    for (uint32_t kb = 0; kb < KB; kb += 2) {
+        block_mma<F>(b0, stage0, acc, s_t, lane);
+        a_store(ra, stage1, tid);
+        {
+            const uint32_t kn = kb + 2 < KB ? kb + 2 : KB - 1;
+            a_load(ra, A, kn);
+            blk_load(b0, W, rowblk + kn, h);
+        }
+        __syncthreads();
+        if (kb + 1 >= KB) break;
+        block_mma<F>(b1, stage1, acc, s_t, lane);
+        a_store(ra, stage0, tid);
+        {
+            const uint32_t kn = kb + 3 < KB ? kb + 3 : KB - 1;
+            a_load(ra, A, kn);
+            blk_load(b1, W, rowblk + kn, h);
+        }
+        __syncthreads();
     }
-    constexpr int NG2 = F == FMT_IQ2 ? 512 : F == FMT_IQ2S ? 1024 : 1;        // fp16 grid entries of 8
-    constexpr int NSG = F == FMT_IQ2 || F == FMT_IQ3 ? 128 : F == FMT_IQ2S || F == FMT_IQ3S ? 256 : 1;   // sign masks
-    constexpr int NT4 = F == FMT_IQ3 ? 512 : F == FMT_IQ3S ? 1024 : F == FMT_IQ4 ? 256 : 1;   // words
-    __shared__ uint4 s_g2[NG2];
-    __shared__ uint4 s_sg[NSG];
-    __shared__ uint32_t s_t[NT4];
-    __shared__ uint4 s_a[2 * MT * 2048];   // [stage][row tile][(kstep*2 + piece)*64 + lane]
-    const int tid = threadIdx.x;
-    {
-        const uint4 *g2 = F == FMT_IQ2S ? P.g2sh : P.g2h;
-        const uint4 *sg = F == FMT_IQ2S || F == FMT_IQ3S ? P.sgn8 : P.sgn;
-        const uint32_t *t4 = F == FMT_IQ3 ? reinterpret_cast<const uint32_t *>(P.g3h)
-                           : F == FMT_IQ3S ? reinterpret_cast<const uint32_t *>(P.g3sh) : P.kv2;
-        if (NG2 > 1) for (int i = tid; i < NG2; i += 256) s_g2[i] = g2[i];
-        if (NSG > 1) for (int i = tid; i < NSG; i += 256) s_sg[i] = sg[i];
-        if (NT4 > 1) for (int i = tid; i < NT4; i += 256) s_t[i] = t4[i];
+
+    // epilogue: lane's column c + col, rows 8*(r/4) + 4h + r%4 of the row tile
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const uint32_t row = mt0 * 32 + 4 * h + 8 * (r >> 2) + (r & 3);
+        if (row >= g.nvalid) continue;
+        float y = acc[r] * g.rscale[row];
+        y = isfinite(y) ? y : 0.0f;   // non-finite projection outputs -> 0 (src/qx_format.c:4284)
+        const uint64_t o = (uint64_t)row * g.ld + c + col;
+        g.out[o] = EPI == EPI_RESID ? g.resid[o] + y : y;
     }
-    const GemmLds L{s_g2, s_sg, s_a, s_t, MT * 2048};
-    if (MT == 2 && nmt == 2) gemm_body<F, NSUB, (MT == 2 ? 2 : 1), EPI>(g, L, e, mt0, bx);
-    else gemm_body<F, NSUB, 1, EPI>(g, L, e, mt0, bx);
 }
 
 // ================================================================= element-wise stages
@@ -501,7 +275,7 @@ extern "C" __global__ __launch_bounds__(256) void qxp_embed(const uint8_t *emb, 
 }
 
 // RMSNorm of each token's 2048-vector (qx_apply_f32_rmsnorm, src/qx_format.c:3358-3371);
-// wave per token.
+// wave per token (the stage probes).
 extern "C" __global__ __launch_bounds__(256) void qxp_norm(const float *x, const float *w, uint32_t T, float *y) {
     const int lane = threadIdx.x & 63;
     const uint32_t t = blockIdx.x * 4 + wave_id();
@@ -513,6 +287,18 @@ extern "C" __global__ __launch_bounds__(256) void qxp_norm(const float *x, const
     float4 *o = reinterpret_cast<float4 *>(y + (uint64_t)t * 2048 + 32 * lane);
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+}
+
+// shift of the power-of-two scale 2^sh that takes a row's largest magnitude (mx: the lane's)
+// into [2^13, 2^14); every lane gets it
+DEV int row_shift(float mx, bool ok) {
+    mx = fmaxf(mx, dppf<DPP_XOR1>(mx)); mx = fmaxf(mx, dppf<DPP_XOR2>(mx));
+    mx = fmaxf(mx, dppf<DPP_ROR4>(mx)); mx = fmaxf(mx, dppf<DPP_ROR8>(mx));
+    mx = fmaxf(fmaxf(rdlanef(mx, 0), rdlanef(mx, 16)), fmaxf(rdlanef(mx, 32), rdlanef(mx, 48)));
+    int ex = 0;
+    if (mx > 0.0f && ok) (void)frexpf(mx, &ex);   // mx = f * 2^ex, f in [0.5, 1)
+    const int sh = 14 - ex;
+    return sh > 100 ? 100 : sh < -100 ? -100 : sh;
 }
 
 // Packs one row of the A operand held by a wave, NC chunks of 8 values per lane (chunk
@@ -532,13 +318,7 @@ DEV void pack_row(const float (&v)[NC][8], const int (&c)[NC], uint32_t r, uint4
             mx = fmaxf(mx, fabsf(v[i][j]));
         }
     const bool ok = __ballot(!fin) == 0;
-    mx = fmaxf(mx, dppf<DPP_XOR1>(mx)); mx = fmaxf(mx, dppf<DPP_XOR2>(mx));
-    mx = fmaxf(mx, dppf<DPP_ROR4>(mx)); mx = fmaxf(mx, dppf<DPP_ROR8>(mx));
-    mx = fmaxf(fmaxf(rdlanef(mx, 0), rdlanef(mx, 16)), fmaxf(rdlanef(mx, 32), rdlanef(mx, 48)));
-    int ex = 0;
-    if (mx > 0.0f && ok) (void)frexpf(mx, &ex);   // mx = f * 2^ex, f in [0.5, 1)
-    int sh = 14 - ex;
-    sh = sh > 100 ? 100 : sh < -100 ? -100 : sh;
+    const int sh = row_shift(mx, ok);
     const float sc = ldexpf(1.0f, sh);
     if (lane == 0) rscale[r] = ok ? ldexpf(1.0f, -sh) : 0.0f;
     const uint32_t mt = r >> 5, i32 = r & 31;
@@ -559,25 +339,21 @@ DEV void pack_row(const float (&v)[NC][8], const int (&c)[NC], uint32_t r, uint4
     }
 }
 
-// Packs row r of the A operand (r < rows, and r < nrows[1] when nrows is non-null):
-// source row map ? map[r] : r of src (K floats; rows r >= nvalid and negative map
-// entries are padding and pack zeros), through pack_row.  Wave per row, chunks
-// lane + 64 i, no workgroup barriers.
-template <int K>
-__global__ __launch_bounds__(256) void qxp_pack(const float *src, const int32_t *map, const uint32_t *nrows,
-                                                uint32_t rows, uint32_t nvalid, uint4 *apk, float *rscale) {
-    constexpr int CH = K / 8, PL = (CH + 63) / 64;
+// Packs row r < rows of the O GEMM's A operand from the 4096-value rows of src; rows r >=
+// nvalid pack zeros.  Wave per row, chunks lane + 64 i, no workgroup barriers.
+extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src, uint32_t rows, uint32_t nvalid, uint4 *apk,
+                                                               float *rscale) {
+    constexpr int PL = 8;
     const int lane = threadIdx.x & 63;
     const uint32_t r = blockIdx.x * 4 + wave_id();
-    if (r >= rows || (nrows && r >= nrows[1])) return;   // whole wave
-    const int32_t sr = r >= nvalid ? -1 : map ? map[r] : (int32_t)r;
+    if (r >= rows) return;   // whole wave
     float v[PL][8];
     int c[PL];
 #pragma unroll
     for (int i = 0; i < PL; ++i) {
         c[i] = lane + 64 * i;
-        if (c[i] < CH && sr >= 0) {
-            const float4 *p = reinterpret_cast<const float4 *>(src + (uint64_t)sr * K + 8 * c[i]);
+        if (r < nvalid) {
+            const float4 *p = reinterpret_cast<const float4 *>(src + (uint64_t)r * 4096 + 8 * c[i]);
             const float4 a = p[0], b = p[1];
             v[i][0] = a.x; v[i][1] = a.y; v[i][2] = a.z; v[i][3] = a.w;
             v[i][4] = b.x; v[i][5] = b.y; v[i][6] = b.z; v[i][7] = b.w;
@@ -586,10 +362,54 @@ __global__ __launch_bounds__(256) void qxp_pack(const float *src, const int32_t 
             for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
         }
     }
-    pack_row<PL, K>(v, c, r, apk, rscale);
+    pack_row<PL, 4096>(v, c, r, apk, rscale);
 }
 
-// RMSNorm of token r (qxp_norm's arithmetic: 32 consecutive values per lane) fused with
+// RMSNorm of each token's 2048-vector (qx_apply_f32_rmsnorm, src/qx_format.c:3358-3371) as
+// f32 rows for the router and as the gate/up GEMM's packed rows (lines of two k-steps,
+// [hi, lo][h][8] each; k-step 16 b + s and lane half h hold K = 256 b + 128 h + 8 s + j);
+// rscale[t] = 1/s, or 0 (and zeros) when the row has a non-finite value.  Wave per token, 32
+// values a lane.
+extern "C" __global__ __launch_bounds__(256) void qxp_ffn_norm(const float *x, const float *w, uint32_t T, float *y,
+                                                               uint8_t *xp, float *rscale) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t t = blockIdx.x * 4 + wave_id();
+    if (t >= T) return;   // whole wave
+    float v[32], ww[32];
+    load32(x + (uint64_t)t * 2048 + 32 * lane, v);
+    load32(w + 32 * lane, ww);
+    rmsnorm32(v, ww);
+    float4 *o = reinterpret_cast<float4 *>(y + (uint64_t)t * 2048 + 32 * lane);
+    float mx = 0.0f;
+    bool fin = true;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        fin = fin && isfinite(v[i]);
+        mx = fmaxf(mx, fabsf(v[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    const bool ok = __ballot(!fin) == 0;
+    const int sh = row_shift(mx, ok);
+    const float sc = ldexpf(1.0f, sh);
+    if (lane == 0) rscale[t] = ok ? ldexpf(1.0f, -sh) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t c = 4 * lane + i, at = (16 * (c >> 5) + (c & 15)) * 64 + ((c >> 4) & 1) * 16;
+        h8v hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float q = ok ? v[8 * i + j] * sc : 0.0f;
+            const _Float16 a = (_Float16)q;
+            hi[j] = a;
+            lo[j] = (_Float16)(q - (float)a);
+        }
+        *reinterpret_cast<uint4 *>(xp + (uint64_t)t * 8192 + at) = __builtin_bit_cast(uint4, hi);
+        *reinterpret_cast<uint4 *>(xp + (uint64_t)t * 8192 + at + 32) = __builtin_bit_cast(uint4, lo);
+    }
+}
+
+// RMSNorm of token r (32 consecutive values per lane) fused with
 // its packing as the Q/K/V GEMM's A operand; rows r >= nvalid pack zeros.
 extern "C" __global__ __launch_bounds__(256) void qxp_norm_pack(const float *x, const float *w, uint32_t rows,
                                                                 uint32_t nvalid, uint4 *apk, float *rscale) {
@@ -888,10 +708,11 @@ extern "C" __global__ __launch_bounds__(256) void qxp_attn(const float *qr, cons
 // are added in LDS in a fixed order.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 extern "C" __global__ __launch_bounds__(512) void qxp_router(const float *xn, const float *router, uint32_t T,
-                                                             uint32_t experts, double *logits) {
+                                                             uint32_t experts, double *logits, uint32_t *cnt) {
     __shared__ double part[8][16][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int i = lane & 15, g = lane >> 4;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && tid < 128) cnt[tid] = 0u;   // for qxp_route, the next launch
     const uint32_t t = blockIdx.x * 16 + i;   // < 512: xn holds QXP_MAX rows
     const uint32_t e = blockIdx.y * 16 + i, er = e < experts ? e : 0u;
     const float4 *xa = reinterpret_cast<const float4 *>(xn + (uint64_t)t * 2048 + wave * 256 + g * 64);
@@ -919,104 +740,59 @@ extern "C" __global__ __launch_bounds__(512) void qxp_router(const float *xn, co
     }
 }
 
-// Top-8 experts and renormalised weights per token (wave per token; the decode path's
-// selection, src/qx_format.c:5265-5285).
-extern "C" __global__ __launch_bounds__(256) void qxp_route(const double *logits, uint32_t T, uint32_t experts,
-                                                            uint32_t *ids, double *wts) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t t = blockIdx.x * 4 + wave_id();
-    if (t >= T) return;
+// Top-8 experts and renormalised weights per token (the decode path's selection,
+// src/qx_format.c:5265-5285), and the experts' pair lists: pair p = 8 t + rank joins list e at
+// the next free place.  The order within a list varies from run to run; a pair's row of the
+// expert GEMMs does not depend on its place.  A workgroup takes 32 tokens, two a wave, counts
+// its pairs by expert in LDS and claims the list places with one atomic per expert (pairs that
+// each took their place themselves waited on the crowded experts' counters: 20 us).
+extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logits, uint32_t T, uint32_t experts,
+                                                             double *wts, uint32_t *cnt, uint32_t *list) {
+    __shared__ uint32_t s_n[128], s_at[128];
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (tid < 128) s_n[tid] = 0u;
+    __syncthreads();
     const int E = (int)experts;
-    const double l0 = lane < E ? logits[(uint64_t)t * 128 + lane] : 0.0;
-    const double l1 = lane + 64 < E ? logits[(uint64_t)t * 128 + lane + 64] : 0.0;
-    uint32_t id[QXG_TOPK];
-    double w[QXG_TOPK];
-    wave_top8(l0, l1, E, id, w);
+    uint32_t e[2] = {0, 0}, place[2] = {0, 0};
 #pragma unroll
-    for (int q = 0; q < QXG_TOPK; ++q)
-        if (lane == q) { ids[t * 8 + q] = id[q] < experts ? id[q] : 0u; wts[t * 8 + q] = w[q]; }
-}
-
-// Token -> expert grouping (one block): expert e's tokens, ascending, take slots
-// off[e] .. off[e]+n_e of an expert-major layout padded to 32 per expert; tok_slot[t][r]
-// is the slot of (token t, rank r), slot_token the inverse (-1 on padding).  m-groups of
-// up to MT row tiles per expert feed the expert GEMMs; meta = {m-groups, padded slots}.
-extern "C" __global__ __launch_bounds__(1024) void qxp_group(const uint32_t *ids, uint32_t T, uint32_t experts,
-        uint32_t mt_per_group, int32_t *slot_token, uint32_t *tok_slot, uint32_t *mgroups, uint32_t *meta) {
-    __shared__ uint32_t bm[128][QXP_MAX / 32];
-    __shared__ uint32_t cnt[128], off[129];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < 128 * (QXP_MAX / 32); i += 1024) (&bm[0][0])[i] = 0u;
-    __syncthreads();
-    for (uint32_t p = tid; p < T * 8; p += 1024) {
-        const uint32_t t = p >> 3, e = ids[p];
-        atomicOr(&bm[e][t >> 5], 1u << (t & 31));
-    }
-    __syncthreads();
-    if (tid < 128) {
-        uint32_t c = 0;
-        for (int w = 0; w < QXP_MAX / 32; ++w) c += __popc(bm[tid][w]);
-        cnt[tid] = c;
-    }
-    __syncthreads();
-    if (tid < 64) {   // wave 0: experts 2l, 2l+1 per lane; exclusive scans of row tiles and m-groups
-        uint32_t mt[2], ng[2];
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t t = blockIdx.x * 32 + 2 * wave_id() + i;
+        if (t >= T) break;   // whole wave
+        const double l0 = lane < E ? logits[(uint64_t)t * 128 + lane] : 0.0;
+        const double l1 = lane + 64 < E ? logits[(uint64_t)t * 128 + lane + 64] : 0.0;
+        uint32_t id[QXG_TOPK];
+        double w[QXG_TOPK];
+        wave_top8(l0, l1, E, id, w);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t e = 2 * tid + j;
-            mt[j] = e < experts ? (cnt[e] + 31) / 32 : 0u;
-            ng[j] = (mt[j] + mt_per_group - 1) / mt_per_group;
-        }
-        const uint32_t smt = mt[0] + mt[1], sng = ng[0] + ng[1];
-        uint32_t imt = smt, ing = sng;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t a = __shfl_up(imt, o), b = __shfl_up(ing, o);
-            if (tid >= o) { imt += a; ing += b; }
-        }
-        uint32_t tile = imt - smt, gi = ing - sng;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t e = 2 * tid + j;
-            if (e <= 128u) off[e] = 32 * tile;
-            for (uint32_t g = 0; g < mt[j]; g += mt_per_group) {
-                const uint32_t k = mt[j] - g < mt_per_group ? mt[j] - g : mt_per_group;
-                mgroups[gi++] = e | ((tile + g) << 8) | (k << 20);
+        for (int q = 0; q < QXG_TOPK; ++q)
+            if (lane == q) {
+                e[i] = id[q] < experts ? id[q] : 0u;
+                wts[t * 8 + q] = w[q];
+                place[i] = atomicAdd(&s_n[e[i]], 1u);
             }
-            tile += mt[j];
-        }
-        if (tid == 63) {   // totals (experts past `experts` hold no tiles)
-            off[experts] = 32 * imt;
-            meta[0] = ing;
-            meta[1] = 32 * imt;
-        }
     }
     __syncthreads();
-    for (uint32_t p = tid; p < T * 8; p += 1024) {
-        const uint32_t t = p >> 3, e = ids[p], w = t >> 5;
-        uint32_t rank = __popc(bm[e][w] & ((1u << (t & 31)) - 1u));
-        for (uint32_t i = 0; i < w; ++i) rank += __popc(bm[e][i]);
-        const uint32_t slot = off[e] + rank;
-        tok_slot[p] = slot;
-        slot_token[slot] = (int32_t)t;
+    if (tid < 128 && s_n[tid]) s_at[tid] = atomicAdd(&cnt[tid], s_n[tid]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t t = blockIdx.x * 32 + 2 * wave_id() + i;
+        if (t < T && lane < QXG_TOPK) list[(uint64_t)e[i] * QXP_LIST + s_at[e[i]] + place[i]] = t * 8 + lane;
     }
-    if (tid < (int)experts)
-        for (uint32_t s = off[tid] + cnt[tid]; s < off[tid + 1]; ++s) slot_token[s] = -1;
 }
 
-// x[t][i] = x1[t][i] + sum_r (float)(w_r * (double)y[slot(t,r)][i]), ranks in order
+// x[t][i] = x1[t][i] + sum_r (float)(w_r * (double)y[8 t + r][i]), ranks in order
 // (src/qx_format.c:5296-5309); block per token.
-extern "C" __global__ __launch_bounds__(256) void qxp_combine(const float *x1, const float *y, const uint32_t *tok_slot,
-                                                              const double *wts, float *x, float *moe_dump) {
+extern "C" __global__ __launch_bounds__(256) void qxp_combine(const float *x1, const float *y, const double *wts, float *x,
+                                                              float *moe_dump) {
     const uint32_t t = blockIdx.x;
-    uint32_t sl[QXG_TOPK];
     double w[QXG_TOPK];
 #pragma unroll
-    for (int r = 0; r < QXG_TOPK; ++r) { sl[r] = tok_slot[t * 8 + r]; w[r] = wts[t * 8 + r]; }
+    for (int r = 0; r < QXG_TOPK; ++r) w[r] = wts[t * 8 + r];
     for (int i = threadIdx.x; i < 2048; i += 256) {
         float m = 0.0f;
 #pragma unroll
-        for (int r = 0; r < QXG_TOPK; ++r) m += (float)(w[r] * (double)y[(uint64_t)sl[r] * 2048 + i]);
+        for (int r = 0; r < QXG_TOPK; ++r) m += (float)(w[r] * (double)y[((uint64_t)t * 8 + r) * 2048 + i]);
         if (moe_dump) moe_dump[(uint64_t)t * 2048 + i] = m;
         x[(uint64_t)t * 2048 + i] = x1[(uint64_t)t * 2048 + i] + m;
     }
@@ -1027,49 +803,26 @@ extern "C" {
 void qxp_launch_gemm(hipStream_t s, int kind, const PfGemm &g0, const PfTables &P, uint32_t grid_x, uint32_t grid_y,
                      Timer tm) {
     // row classes per kind (xcd_tile): Q/K/V 2 (4 MB of activations, 5.6 MB of weights),
-    // O 4 (8 MB, 4.5 MB), experts 8 (an expert tile's activations in one L2; its weights
-    // are read by that tile only)
+    // O 4 (8 MB, 4.5 MB)
     PfGemm g = g0;
-    g.xcd_rows = kind == QXP_QKV || kind == QXP_V_Q5 ? 2u : kind == QXP_O || kind == QXP_O_Q5 ? 4u : 8u;
+    g.xcd_rows = kind == QXP_QKV || kind == QXP_V_Q5 ? 2u : 4u;
     const uint32_t b = 8u / g.xcd_rows;
     if (grid_x % b) g.xcd_rows = 8u;   // (the column counts here are multiples of 8 workgroups)
     grid_y = (grid_y + g.xcd_rows - 1) / g.xcd_rows * g.xcd_rows;
     const dim3 grid(grid_x, grid_y);
     switch (kind) {
-    case QXP_QKV:       // Q/K/V (or Q/K): IQ4_XS, 32 columns per wave
-    case QXP_DOWN_IQ4:  // expert down, IQ4_XS (the kernel reads the expert groups from g)
-        qx_launch(qxp_gemm<FMT_IQ4, 1, 1, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
+    case QXP_QKV:       // Q/K/V (or Q/K): IQ4_XS
+        qx_launch(qxp_gemm<FMT_IQ4, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
         break;
     case QXP_O:         // O projection + residual: IQ4_XS
-        qx_launch(qxp_gemm<FMT_IQ4, 1, 1, EPI_RESID>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    case QXP_GU:        // expert gate/up + SwiGLU: IQ2_XS
-        qx_launch(qxp_gemm<FMT_IQ2, 2, QXG_PF_EXPERT_MT, EPI_SWIGLU>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    case QXP_DOWN:      // expert down: IQ3_XXS
-        qx_launch(qxp_gemm<FMT_IQ3, 1, QXG_PF_EXPERT_MT, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
+        qx_launch(qxp_gemm<FMT_IQ4, EPI_RESID>, grid, dim3(256), 0, s, tm, g, P);
         break;
     case QXP_V_Q5:      // V alone: Q5_K
-        qx_launch(qxp_gemm<FMT_Q5, 1, 1, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
+        qx_launch(qxp_gemm<FMT_Q5, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
         break;
-    case QXP_O_Q5:      // O projection + residual: Q5_K
-        qx_launch(qxp_gemm<FMT_Q5, 1, 1, EPI_RESID>, grid, dim3(256), 0, s, tm, g, P);
+    default:            // O projection + residual: Q5_K
+        qx_launch(qxp_gemm<FMT_Q5, EPI_RESID>, grid, dim3(256), 0, s, tm, g, P);
         break;
-    case QXP_GU_IQ2S:   // expert gate/up + SwiGLU: IQ2_S
-        qx_launch(qxp_gemm<FMT_IQ2S, 2, QXG_PF_EXPERT_MT, EPI_SWIGLU>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    default:            // expert down: IQ3_S
-        qx_launch(qxp_gemm<FMT_IQ3S, 1, QXG_PF_EXPERT_MT, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    }
-}
-void qxp_launch_pack(hipStream_t s, int K, const float *src, const int32_t *map, const uint32_t *nrows, uint32_t rows,
-                     uint32_t nvalid, uint4 *apk, float *rscale) {
-    const dim3 grid((rows + 3) / 4);   // wave per row
-    switch (K) {
-    case 2048: hipLaunchKernelGGL(qxp_pack<2048>, grid, dim3(256), 0, s, src, map, nrows, rows, nvalid, apk, rscale); break;
-    case 4096: hipLaunchKernelGGL(qxp_pack<4096>, grid, dim3(256), 0, s, src, map, nrows, rows, nvalid, apk, rscale); break;
-    default: hipLaunchKernelGGL(qxp_pack<768>, grid, dim3(256), 0, s, src, map, nrows, rows, nvalid, apk, rscale); break;
     }
 }
 }
