@@ -55,17 +55,19 @@ void qxl_head(hipStream_t, const float *, const float *, const QTensor *, uint32
               uint32_t *, bool, Timer = Timer());
 __global__ void qxp_embed(const uint8_t *, uint64_t, const uint32_t *, float *);
 __global__ void qxp_norm(const float *, const float *, uint32_t, float *);
-__global__ void qxp_ffn_norm(const float *, const float *, uint32_t, float *, uint8_t *, float *);
-__global__ void qxp_norm_pack(const float *, const float *, uint32_t, uint32_t, uint4 *, float *);
-__global__ void qxp_qk(const float *, const float *, const float *, Tables, int8_t *, int8_t *, float *, float *,
+__global__ void qxp_ffn_norm(const float *, const float *, uint32_t, const float *, uint32_t, float *, float *, uint8_t *, float *);
+__global__ void qxp_norm_pack(float *, const float *, const float *, const double *, const float *, uint8_t *, float *, float *);
+__global__ void qxp_qk(const float *, uint32_t, uint32_t, const float *, const float *, Tables, int8_t *, int8_t *, float *, float *,
                        uint32_t, uint32_t, uint32_t, float *);
 __global__ void qxp_attn(const float *, const int8_t *, const int8_t *, const float *, const float *, uint32_t, uint32_t,
                          uint32_t, uint32_t, float *);
 __global__ void qxp_router(const float *, const float *, uint32_t, uint32_t, double *, uint32_t *);
 __global__ void qxp_route(const double *, uint32_t, uint32_t, double *, uint32_t *, uint32_t *);
 __global__ void qxp_combine(const float *, const float *, const double *, float *, float *);
-__global__ void qxp_pack_ctx(const float *, uint32_t, uint32_t, uint4 *, float *);
-void qxp_launch_gemm(hipStream_t, int, const PfGemm &, const PfTables &, uint32_t, uint32_t, Timer);
+__global__ void qxp_pack_ctx(const float *, uint8_t *, float *, float *);
+__global__ void qxp_dense_plane(uint32_t, const uint8_t *, const uint8_t *, const uint8_t *, uint32_t, uint32_t, uint32_t, uint8_t *,
+                                float *, float *);
+void qxp_launch_dense(hipStream_t, const PfDense &, uint32_t, Timer);
 void qxp_launch_gate_up(hipStream_t, uint32_t, const PfExperts &, const PfTables &, uint32_t, Timer);
 void qxp_launch_down(hipStream_t, uint32_t, const PfExperts &, const PfTables &, uint32_t, Timer);
 }
@@ -166,13 +168,14 @@ struct qxg_ctx {
     // one decode step (embed .. head, top-1, step advance) recorded once and replayed
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    // the prefill's dense layout of every layer's Q/K/V and O matrices (qxg_pf_dense.hip)
+    uint8_t *dense = nullptr;
     // batched prefill: codebooks and work buffers for chunks of up to QXP_MAX tokens
     struct Prefill {
         bool ready = false;
         PfTables P{};
-        float *X = nullptr, *X1 = nullptr, *XN = nullptr, *QKV = nullptr, *QR = nullptr, *CTX = nullptr;
-        float *HS = nullptr, *Y = nullptr, *rscale = nullptr, *xscale = nullptr, *dump = nullptr;
-        uint4 *apk = nullptr;
+        float *X = nullptr, *X1 = nullptr, *XN = nullptr, *PART = nullptr, *QR = nullptr, *CTX = nullptr;
+        float *HS = nullptr, *Y = nullptr, *xscale = nullptr, *sums = nullptr, *dump = nullptr;
         uint8_t *XP = nullptr, *HP = nullptr;
         double *lg = nullptr, *w = nullptr;
         uint32_t *cnt = nullptr, *list = nullptr, *tokens = nullptr;
@@ -496,6 +499,45 @@ bool build_router_fold(qxg_ctx *c, char *err, uint64_t n) {
     return ok;
 }
 
+// Layer l's Q/K/V (stacked rows) or O matrix in the dense layout: codes, scales, offsets
+constexpr uint64_t DENSE_QKV = 5120ull * 2048, DENSE_O = 2048ull * 4096;
+constexpr uint64_t DENSE_LAYER = (DENSE_QKV + DENSE_O) * 10 / 8;   // a byte a weight and 2 floats per 32 weights
+PfDense dense_args(const qxg_ctx *c, uint32_t l, bool qkv) {
+    const LayerW &w = c->L[l];
+    PfDense g{};
+    uint8_t *base = c->dense + l * DENSE_LAYER + (qkv ? 0 : DENSE_QKV * 10 / 8);
+    const uint64_t n = qkv ? DENSE_QKV : DENSE_O;
+    g.codes = base;
+    g.scale = (const float *)(base + n);
+    g.ofs = g.scale + n / 32;
+    g.lines = qkv ? 64 : 128;
+    g.cols = qkv ? 5120 : 2048;
+    g.seg1 = qkv ? 128 : 0xffffffffu;
+    g.seg2 = qkv ? 144 : 0xffffffffu;
+    g.ofs_segs = qkv ? (uint32_t)(w.wq->type == 13) | (uint32_t)(w.wk->type == 13) << 1 | (uint32_t)(w.wv->type == 13) << 2
+                     : (uint32_t)(w.wo->type == 13);
+    return g;
+}
+
+// Every layer's Q/K/V and O matrices in the prefill's dense layout (1 GB for 48 layers)
+bool build_dense(qxg_ctx *c, char *err, uint64_t n) {
+    if (c->dense) (void)hipFree(c->dense);
+    c->dense = nullptr;
+    if (!hip_ok(hipMalloc(&c->dense, DENSE_LAYER * c->layers), err, n, "dense layout")) return false;
+    for (uint32_t l = 0; l < c->layers; ++l) {
+        const LayerW &w = c->L[l];
+        const QTensor *m[4] = {w.wq, w.wk, w.wv, w.wo};
+        const uint32_t rows[4] = {4096, 512, 512, 2048}, ct0[4] = {0, 128, 144, 0};
+        for (int i = 0; i < 4; ++i) {
+            const PfDense g = dense_args(c, l, i < 3);
+            hipLaunchKernelGGL(qxp_dense_plane, dim3(rows[i] * g.lines / 256), dim3(256), 0, c->s, (uint32_t)m[i]->type,
+                               (const uint8_t *)m[i]->p0, (const uint8_t *)m[i]->p1, (const uint8_t *)m[i]->p2, rows[i],
+                               g.lines, ct0[i], (uint8_t *)g.codes, (float *)g.scale, (float *)g.ofs);
+        }
+    }
+    return hip_ok(hipGetLastError(), err, n, "dense layout") && hip_ok(hipStreamSynchronize(c->s), err, n, "dense layout");
+}
+
 // The routed experts' rows of every layer in the persistent decode's interleaved layout
 // (QXD_GU_UNIT, QXD_DN_ROW in qxg_internal.h), copied from the IQ2_XS / IQ3_XXS planes.
 bool build_expert_interleave(qxg_ctx *c, char *err, uint64_t n) {
@@ -706,6 +748,20 @@ uint16_t f16_int(int v) {
 // prefills every prompt.
 bool batched_prefill(const qxg_ctx *c) { return !c->q8; }
 
+// Parts of K of a dense GEMM over T rows: about 320 workgroups (two fit a CU) of at least 8
+// lines each.  Fewer leave CUs idle (a 37-token O projection as one part took 44 us on 16
+// workgroups, 7 us in 16 parts); more only add parts to write and add up.
+uint32_t dense_parts(uint32_t T, uint32_t cols, uint32_t lines) {
+    const uint32_t wgs = (cols / 128) * (T > 32 ? (T + 63) / 64 : 1);
+    uint32_t p = 1;
+    while (2 * p * wgs <= 320 && 2 * p * 8 <= lines) p *= 2;
+    return p;
+}
+// floats of either GEMM's parts: one part is at most QXP_MAX x 5120; p parts of 5120 columns
+// have p * ceil(T / 64) <= 8 (p T <= 512), of 2048 columns <= 20 (p T 2048 <= 512 x 5120)
+constexpr uint64_t PF_PART_FLOATS = (uint64_t)QXP_MAX * 5120;
+static_assert(QXP_MAX >= 512, "the parts' buffer");
+
 bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
     auto &B = c->pf;
     if (B.ready) return true;
@@ -716,12 +772,11 @@ bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
     };
     const uint64_t T = QXP_MAX, PAIRS = T * QXG_TOPK;
     bool ok = alloc((void **)&B.X, T * 2048 * 4) && alloc((void **)&B.X1, T * 2048 * 4) &&
-              alloc((void **)&B.XN, T * 2048 * 4) && alloc((void **)&B.QKV, T * 5120 * 4) &&
+              alloc((void **)&B.XN, T * 2048 * 4) && alloc((void **)&B.PART, PF_PART_FLOATS * 4) &&
               alloc((void **)&B.QR, T * 4096 * 4) && alloc((void **)&B.CTX, T * 4096 * 4) &&
-              alloc((void **)&B.XP, T * 8192) && alloc((void **)&B.xscale, T * 4) && alloc((void **)&B.HP, PAIRS * 3072) &&
+              alloc((void **)&B.XP, T * PF_PITCH(4096)) && alloc((void **)&B.xscale, T * 4) && alloc((void **)&B.HP, PAIRS * PF_PITCH(768)) &&
               alloc((void **)&B.HS, PAIRS * 8 * 4) && alloc((void **)&B.Y, PAIRS * 2048 * 4) &&
-              alloc((void **)&B.rscale, T * 4) && alloc((void **)&B.dump, T * 2048 * 4) &&
-              alloc((void **)&B.apk, T * 4096 * 4) && alloc((void **)&B.lg, T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
+              alloc((void **)&B.sums, T * 128 * 4) && alloc((void **)&B.dump, T * 2048 * 4) && alloc((void **)&B.lg, T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
               alloc((void **)&B.cnt, 128 * 4) && alloc((void **)&B.list, 128ull * QXP_LIST * 4) &&
               alloc((void **)&B.tokens, T * 4);
     // codebooks: grids as magnitude bytes, sign bytes (0x80 where negative), the IQ4_XS byte table as fp16
@@ -759,53 +814,47 @@ PfMat pf_mat(const QTensor *t) { return PfMat{t->p0, t->p1, t->p2, t->d}; }
 
 // One layer over the T tokens of a chunk at positions p0..p0+T-1: pf.X -> pf.X (pf.X1
 // holds the attention half's result, the MoE input).  Asynchronous on c->s.
-void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, float *moe_dump) {
+// first: its input is pf.X; otherwise the previous layer's experts are combined into it.  last: the
+// layer's own experts are combined into pf.X (moe_dump, if any: their sum).
+void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, bool first, bool last, float *moe_dump) {
     auto &B = c->pf;
     const LayerW &w = c->L[l];
     hipStream_t s = c->s;
-    const uint32_t mt = (T + 31) / 32, E = c->experts;
-    const uint32_t none = 0xffffffffu;
-    // attention half: RMSNorm, Q/K/V GEMM, q/k norm + RoPE + INT8 append, attention, O GEMM + residual
-    hipLaunchKernelGGL(qxp_norm_pack, dim3(mt * 8), dim3(256), 0, s, (const float *)B.X, w.attn_norm, mt * 32, T, B.apk,
-                       B.rscale);
-    // per-layer formats of the real checkpoint: V and O in Q5_K or IQ4_XS, gate/up in IQ2_S or
-    // IQ2_XS, down in IQ3_XXS, IQ3_S or IQ4_XS (type ids of the QXF1 manifest)
-    const bool vo_q5 = w.wv->type == 13;
-    PfGemm g{};
-    g.w[0] = pf_mat(w.wq); g.w[1] = pf_mat(w.wk); g.w[2] = pf_mat(w.wv);
-    g.w_start[0] = 0; g.w_start[1] = 4096; g.w_start[2] = vo_q5 ? none : 4608;
-    g.kb = 8; g.apk = B.apk; g.rscale = B.rscale; g.mtiles = mt; g.nvalid = T; g.out = B.QKV; g.ld = 5120;
-    qxp_launch_gemm(s, QXP_QKV, g, B.P, (vo_q5 ? 4608 : 5120) / 128, mt, timer_for(c, 8));
-    if (vo_q5) {   // V (Q5_K) into columns 4608..5119
-        PfGemm gv = g;
-        gv.w[0] = pf_mat(w.wv); gv.w_start[1] = none; gv.w_start[2] = none; gv.out = B.QKV + 4608;
-        qxp_launch_gemm(s, QXP_V_Q5, gv, B.P, 512 / 128, mt, Timer{});
-    }
-    hipLaunchKernelGGL(qxp_qk, dim3(T), dim3(256), 0, s, (const float *)B.QKV, w.q_norm, w.k_norm, c->T, c->kc, c->vc,
-                       c->ks, c->vs, l, c->kv_ctx, p0, B.QR);
+    const uint32_t E = c->experts;
+    // attention half: RMSNorm, Q/K/V GEMM, q/k norm + RoPE + INT8 append, attention, O GEMM
+    hipLaunchKernelGGL(qxp_norm_pack, dim3(T), dim3(256), 0, s, B.X, (const float *)B.X1,
+                       first ? (const float *)nullptr : (const float *)B.Y, (const double *)B.w, w.attn_norm, B.XP, B.xscale,
+                       B.sums);
+    PfDense g = dense_args(c, l, true);
+    const uint32_t qkv_parts = dense_parts(T, g.cols, g.lines), o_parts = dense_parts(T, 2048, 128);
+    g.part_lines = g.lines / qkv_parts;
+    g.rows_packed = B.XP; g.rows = T; g.row_bytes = PF_PITCH(2048); g.rscale = B.xscale; g.sums = B.sums; g.out = B.PART;
+    qxp_launch_dense(s, g, qkv_parts, timer_for(c, 8));
+    hipLaunchKernelGGL(qxp_qk, dim3(T), dim3(256), 0, s, (const float *)B.PART, qkv_parts, T, w.q_norm, w.k_norm, c->T, c->kc,
+                       c->vc, c->ks, c->vs, l, c->kv_ctx, p0, B.QR);
     qx_launch(qxp_attn, dim3(4, (T + 3) / 4), dim3(256), 0, s, timer_for(c, 13), (const float *)B.QR,
               (const int8_t *)c->kc, (const int8_t *)c->vc, (const float *)c->ks, (const float *)c->vs, l, c->kv_ctx, p0, T,
               B.CTX);
-    hipLaunchKernelGGL(qxp_pack_ctx, dim3(mt * 8), dim3(256), 0, s, (const float *)B.CTX, mt * 32, T, B.apk, B.rscale);
-    g = PfGemm{};
-    g.w[0] = pf_mat(w.wo); g.w_start[1] = none; g.w_start[2] = none;
-    g.kb = 16; g.apk = B.apk; g.rscale = B.rscale; g.mtiles = mt; g.nvalid = T; g.out = B.X1; g.ld = 2048;
-    g.resid = B.X;
-    qxp_launch_gemm(s, vo_q5 ? QXP_O_Q5 : QXP_O, g, B.P, 2048 / 128, mt, timer_for(c, 9));
-    // MoE half: RMSNorm, router logits, top-8 and the experts' pair lists, gate/up + SwiGLU, down, combine
-    hipLaunchKernelGGL(qxp_ffn_norm, dim3((T + 3) / 4), dim3(256), 0, s, (const float *)B.X1, w.ffn_norm, T, B.XN, B.XP,
-                       B.xscale);
+    hipLaunchKernelGGL(qxp_pack_ctx, dim3(T), dim3(256), 0, s, (const float *)B.CTX, B.XP, B.xscale, B.sums);
+    g = dense_args(c, l, false);
+    g.part_lines = g.lines / o_parts;
+    g.rows_packed = B.XP; g.rows = T; g.row_bytes = PF_PITCH(4096); g.rscale = B.xscale; g.sums = B.sums; g.out = B.PART;
+    qxp_launch_dense(s, g, o_parts, timer_for(c, 9));
+    // MoE half: residual + RMSNorm, router logits, top-8 and the experts' pair lists, gate/up + SwiGLU, down, combine
+    hipLaunchKernelGGL(qxp_ffn_norm, dim3(T), dim3(256), 0, s, (const float *)B.X, (const float *)B.PART, o_parts,
+                       w.ffn_norm, T, B.X1, B.XN, B.XP, B.xscale);
     qx_launch(qxp_router, dim3((T + 15) / 16, (E + 15) / 16), dim3(512), 0, s, timer_for(c, 12), (const float *)B.XN,
               w.router, T, E, B.lg, B.cnt);
-    hipLaunchKernelGGL(qxp_route, dim3((T + 31) / 32), dim3(1024), 0, s, (const double *)B.lg, T, E, B.w, B.cnt, B.list);
+    hipLaunchKernelGGL(qxp_route, dim3((T + 15) / 16), dim3(1024), 0, s, (const double *)B.lg, T, E, B.w, B.cnt, B.list);
     PfExperts x{};
     x.w[0] = pf_mat(w.gate); x.w[1] = pf_mat(w.up); x.w[2] = pf_mat(w.down);
     x.experts = E; x.cnt = B.cnt; x.list = B.list; x.xp = B.XP; x.xs = B.xscale; x.hp = B.HP; x.hs = B.HS;
     x.h_pairs = w.down->type == 23; x.y = B.Y;
     qxp_launch_gate_up(s, w.gate->type, x, B.P, T, timer_for(c, 10));
     qxp_launch_down(s, w.down->type, x, B.P, T, timer_for(c, 11));
-    hipLaunchKernelGGL(qxp_combine, dim3(T), dim3(256), 0, s, (const float *)B.X1, (const float *)B.Y, (const double *)B.w,
-                       B.X, moe_dump);
+    if (last)
+        hipLaunchKernelGGL(qxp_combine, dim3(T), dim3(256), 0, s, (const float *)B.X1, (const float *)B.Y, (const double *)B.w,
+                           B.X, moe_dump);
 }
 // Token-step prefill: one decode step per prompt token (embedding, every layer), the head
 // on the last when run_head; residual_out row i is token i's final residual.
@@ -994,6 +1043,7 @@ void qxg_close(qxg_ctx *c) {
                     c->T.rope_cs, c->half_dump, c->wsum_dump};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : c->arenas) (void)hipFree(p);
+    if (c->dense) (void)hipFree(c->dense);
     for (void *p : c->pf.all) (void)hipFree(p);
     for (void *p : c->sg.all) (void)hipFree(p);
     for (hipEvent_t e : c->kt.ev) (void)hipEventDestroy(e);
@@ -1110,6 +1160,7 @@ int qxg_bind_model(qxg_ctx *c, uint32_t layers, int need_embedding, int need_hea
         if (!hip_ok(hipMalloc(bufs[i], sizes[i]), err, err_len, "work buffers")) return 0;
     if (!hip_ok(hipMemset(c->tokens, 0, sizes[15]), err, err_len, "work buffers")) return 0;
     if (layers && base && !build_arenas(c, err, err_len)) return 0;
+    if (layers && !build_dense(c, err, err_len)) return 0;
     if (c->mfold) { (void)hipFree(c->mfold); c->mfold = nullptr; }
     if (layers && base && !build_router_fold(c, err, err_len)) return 0;
     if (layers && base && !build_expert_interleave(c, err, err_len)) return 0;
@@ -1860,7 +1911,7 @@ int qxg_prefill(qxg_ctx *c, const uint32_t *tokens, uint32_t n, uint32_t positio
                 return 0;
         }
         hipLaunchKernelGGL(qxp_embed, dim3(T), dim3(256), 0, c->s, c->emb, c->emb_row, (const uint32_t *)B.tokens, B.X);
-        for (uint32_t l = 0; l < c->layers; ++l) prefill_layer(c, l, T, position0 + c0, nullptr);
+        for (uint32_t l = 0; l < c->layers; ++l) prefill_layer(c, l, T, position0 + c0, l == 0, l + 1 == c->layers, nullptr);
         if (residual_out &&
             !hip_ok(hipMemcpyAsync(residual_out + 2048ull * c0, B.X, 2048ull * 4 * T, hipMemcpyDeviceToHost, c->s), err, err_len, "read"))
             return 0;
@@ -1903,7 +1954,7 @@ int qxg_prefill_layer(qxg_ctx *c, uint32_t layer, uint32_t n, uint32_t position0
     if (!prefill_ready(c, err, err_len)) return 0;
     auto &B = c->pf;
     if (!hip_ok(hipMemcpyAsync(B.X, x_in, 2048ull * 4 * n, hipMemcpyHostToDevice, c->s), err, err_len, "upload")) return 0;
-    prefill_layer(c, layer, n, position0, moe_out ? B.dump : nullptr);
+    prefill_layer(c, layer, n, position0, true, true, moe_out ? B.dump : nullptr);
     if (!finish(c, err, err_len)) return 0;
     if (ffn_inp_out && !hip_ok(hipMemcpy(ffn_inp_out, B.X1, 2048ull * 4 * n, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
     if (moe_out && !hip_ok(hipMemcpy(moe_out, B.dump, 2048ull * 4 * n, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;

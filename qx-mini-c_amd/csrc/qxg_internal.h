@@ -203,6 +203,11 @@ struct QxDArgs {
 
 // ---- batched prefill (qxg_prefill.hip)
 #define QXP_MAX 512   // tokens per prefill chunk
+// Bytes from one packed activation row of K values (hi and lo, 4 bytes a value) to the next.  A
+// GEMM's workgroups read one 128-byte line of each of their rows at a time, all along K in step:
+// at a pitch of K * 4 alone (a multiple of 4 KB, or of 1 KB) those lines meet in one L2 channel
+// (or four); 256 bytes more spread them over all sixteen.
+#define PF_PITCH(K) (4u * (K) + 256u)
 // entries of one expert's pair list: every (token, rank) pair of a chunk (an expert takes a
 // token once, except where non-finite logits make the top-8 repeat it)
 #define QXP_LIST (QXP_MAX * QXG_TOPK)
@@ -220,28 +225,27 @@ struct PfTables {
 
 // One quantized matrix [rows x K] in the repacked layout (expert e's rows follow e*rows).
 struct PfMat {
-    const uint8_t *qs, *p1;   // qs plane; IQ4_XS / Q5_K meta, IQ2_XS / IQ2_S scales, IQ3_XXS aux, IQ3_S signs
-    const uint8_t *p2;        // Q5_K qh, IQ2_S qh, IQ3_S {qh, scales}
+    const uint8_t *qs, *p1;   // qs plane; IQ4_XS meta, IQ2_XS / IQ2_S scales, IQ3_XXS aux, IQ3_S signs
+    const uint8_t *p2;        // IQ2_S qh, IQ3_S {qh, scales}
     const uint16_t *d;        // fp16 d per block (IQ2_XS, IQ3_XXS, IQ2_S, IQ3_S)
 };
 
-// Arguments of one dense prefill GEMM launch: Y[row][col] = sum_k A[row][k] * W[col][k], A the
-// packed activations (rows = tokens), W up to three matrices stacked along the output
-// columns (Q, K, V).
-struct PfGemm {
-    PfMat w[3];
-    uint32_t w_start[3];       // first output column of each stacked matrix
-    uint32_t kb;               // 256-value blocks per matrix row (K / 256)
-    const uint4 *apk;          // packed activations
-    const float *rscale;       // per packed row: 1/s, 0 for a non-finite row
-    uint32_t mtiles, nvalid;   // m-tiles of 32 rows, valid rows
-    float *out;                // output rows of ld floats
-    uint32_t ld;
-    const float *resid;        // residual added by the O projection epilogue
-    uint32_t xcd_rows;         // row-tile classes across the 8 XCDs (1, 2, 4 or 8; the launcher sets it)
+// Arguments of one dense prefill GEMM (qxg_pf_dense.hip): rows of packed activations against a
+// matrix in the dense layout (Q, K and V stacked, or O), in parts of K.
+struct PfDense {
+    const uint8_t *codes;       // [32-row tile][line][lane][16]
+    const float *scale, *ofs;   // [tile][line / 4][row][line % 4]; ofs null without Q5_K
+    uint32_t lines;             // K / 32
+    uint32_t seg1, seg2;        // first tiles of the second and third stacked matrix
+    uint32_t ofs_segs;          // bit i: matrix i has offsets
+    uint32_t part_lines;        // lines of one part of K (a multiple of 4)
+    const uint8_t *rows_packed;
+    uint32_t rows, row_bytes;
+    const float *rscale;        // per row: 1 / its power-of-two scale, 0 for a non-finite row
+    const float *sums;          // [row][line] sums of the scaled values, for the offsets
+    float *out;                 // [part][row][cols]
+    uint32_t cols;
 };
-// GEMM kinds of qxp_launch_gemm (format and epilogue of the weight matrix)
-enum QxpGemmKind : int { QXP_QKV = 0, QXP_O = 1, QXP_V_Q5 = 4, QXP_O_Q5 = 5 };
 
 // Arguments of the routed-expert GEMMs (qxg_pf_experts.hip); pair p = 8 * token + rank.
 struct PfExperts {
@@ -249,9 +253,9 @@ struct PfExperts {
     uint32_t experts;
     const uint32_t *cnt;       // pairs of each expert
     const uint32_t *list;      // [expert][QXP_LIST] its pairs
-    const uint8_t *xp;         // packed normed activations, 8192 bytes a token
+    const uint8_t *xp;         // packed normed activations, PF_PITCH(2048) a token
     const float *xs;           // per token: 1 / the row's power-of-two scale, 0 for a non-finite row
-    uint8_t *hp;               // packed SwiGLU rows, 3072 bytes a pair
+    uint8_t *hp;               // packed SwiGLU rows, PF_PITCH(768) a pair
     float *hs;                 // [pair][8]: 1 / scale of each 128 values (6 used), NaN for non-finite ones
     uint32_t h_pairs;          // hp in the order of an IQ4_XS down matrix
     float *y;                  // [pair][2048] down rows

@@ -10,19 +10,11 @@
 // (gate/up, gathered through the list while they are staged) and per pair (down, written
 // by gate/up's epilogue); no copy of them is sorted or padded by expert.
 //
-// Tiles.  v_mfma_f32_32x32x16_f16: lane l holds, for A, row l%32 and, for B, column l%32,
-// each 8 values of K at lane half h = l/32; result register r of lane l is row
-// 8*(r/4) + 4*h + r%4, column l%32.  (With one wave on a SIMD the 16x16x32 form reaches 1.2
-// PFLOP/s here, this one 1.6.)  Which 8 values a lane half holds is free as long as A and B
-// agree: a lane takes its part of a weight block whole, and the rows are packed in lines of
-// 128 bytes, line k / 2 and in it [k % 2][hi, lo][h][8 fp16] for k-step k:
+// Order of K.  Which 8 values a lane half holds is free as long as A and B agree: a lane
+// takes its part of a weight block whole, and the rows are packed (qxg_pf.h) with
 //     gate/up: K = 256 b + 128 h + 8 s + j, k-step 16 b + s    (sub-blocks 4h .. 4h + 3)
 //     down:    K = 128 q + 64 h + 8 s + j, k-step 8 q + s      (two sub-blocks of a half block)
 //     down in IQ4_XS: K = 32 i + 8 h + 4 t + j / 2 + 16 (j % 2), k-step 2 i + t   (a scale per 32)
-//
-// Staging.  A stage is 128 values of K of the pass's rows, 4 lines a row, copied to LDS by
-// load-to-LDS instructions of 8 rows x one whole line; the 16-byte chunk c of row r lies at
-// place c ^ (r % 8) of its line, so the column-wise reads spread over all banks.
 //
 // Codes.  The codebooks are bytes in LDS, 8 or 4 magnitudes an entry, with a second table
 // of sign bytes (0x80 where negative).  A magnitude byte and its sign byte side by side are
@@ -34,37 +26,10 @@
 // What bounds them: the matrix cores at their sustained rate (about 1.4 PFLOP/s for tens of us,
 // power-limited), with twice the algorithmic work for hi and lo, where experts hold many pairs; the
 // weights' bytes and the about 20 vector instructions per 8 codes where they hold few.
-#include "qxg_dev.h"
+#include "qxg_pf.h"
 
 namespace {
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef float f4x __attribute__((ext_vector_type(4)));
-typedef float f16x __attribute__((ext_vector_type(16)));
-
 enum { FMT_IQ2 = 0, FMT_IQ2S = 1, FMT_IQ3 = 2, FMT_IQ3S = 3, FMT_IQ4 = 4 };
-
-DEV f16x mfma(uint4 a, uint4 b, f16x c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, a), __builtin_bit_cast(h8v, b), c, 0, 0, 0);
-}
-DEV f16x zero16() {
-    f16x z;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = 0.0f;
-    return z;
-}
-// lane i's 16 bytes at base + off land at lds + 16 i (lds the same in every lane)
-DEV void dma16(const void *base, uint32_t off, const void *lds) {
-    const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)lds);
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
-}
-// waits until at most N of the wave's loads (the youngest) are outstanding
-template <int N>
-DEV void wait_loads() {
-    static_assert(N < 16, "the wait's low counter bits");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | N);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 
 // two signed codes (sign byte over magnitude byte, a subnormal fp16) times m
 DEV uint32_t code2(uint32_t mag, uint32_t sgn, uint32_t sel, h2v m) {
@@ -87,40 +52,6 @@ DEV uint32_t ldu16(const void *p) { return *reinterpret_cast<const uint16_t *>(p
 DEV uint32_t ldu32(const void *p) { return *reinterpret_cast<const uint32_t *>(p); }
 DEV uint2 ldu64(const void *p) { return *reinterpret_cast<const uint2 *>(p); }
 DEV uint4 ldu128(const void *p) { return *reinterpret_cast<const uint4 *>(p); }
-
-constexpr int RT = 2;                    // 32-row tiles of a workgroup pass, at most
-constexpr int ROWS = 32 * RT;            // pairs per pass
-constexpr int STAGE = 4 * ROWS * 8;      // uint4 per stage: 4 lines of 8 chunks a row
-
-// The four lines from line0 on of the pass's rows: wave w copies line w, 8 rows an
-// instruction; off[i] is the lane's row 8 i + lane / 8 and its chunk of the line.
-template <int MT>
-DEV void stage_rows(const void *rows, const uint32_t (&off)[4 * MT], uint32_t line0, uint4 *buf, int wave) {
-#pragma unroll
-    for (int i = 0; i < 4 * MT; ++i) dma16(rows, off[i] + (line0 + wave) * 128, buf + (wave * ROWS + 8 * i) * 8);
-}
-template <int MT>
-DEV void stage_offsets(uint32_t (&off)[4 * MT], const uint32_t *s_row, uint32_t row_bytes, int lane) {
-#pragma unroll
-    for (int i = 0; i < 4 * MT; ++i) off[i] = s_row[8 * i + (lane >> 3)] * row_bytes + (((lane & 7) ^ (lane >> 3)) << 4);
-}
-// A fragments of k-step s of the stage: lane's row l%32 of each tile, lane half l/32
-struct ALane { uint32_t at[4]; };   // byte offset of chunk 2 i + h in the lane's row of line 0
-DEV ALane a_lane(int lane) {
-    ALane a;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a.at[i] = (lane & 31) * 128 + ((((2 * i + (lane >> 5)) ^ lane) & 7) << 4);
-    return a;
-}
-template <int MT>
-DEV void a_read(uint4 (&ah)[MT], uint4 (&al)[MT], const uint4 *buf, const ALane &a, int s) {
-    const uint8_t *p = reinterpret_cast<const uint8_t *>(buf) + (s >> 1) * (ROWS * 128);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        ah[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1)]);
-        al[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1) + 1]);
-    }
-}
 
 // ---------------------------------------------------------------- gate/up weights
 template <int F> struct GuBlk;                                               // the lane's half of a block
@@ -210,7 +141,7 @@ DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
     }
     __syncthreads();   // the rows' tokens, and the tables
     uint32_t off[4 * MT];
-    stage_offsets<MT>(off, s_row, 8192u, lane);   // 2048 values, 4 bytes each
+    stage_offsets<MT>(off, s_row, PF_PITCH(2048), lane);
     stage_rows<MT>(a.xp, off, 0, buf, wave);
     const ALane at = a_lane(lane);
     f16x acc[2][MT];
@@ -303,7 +234,7 @@ DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
                 hi[j] = t;
                 lo[j] = (_Float16)(y - (float)t);
             }
-            uint8_t *o = a.hp + (uint64_t)pr * 3072 + (ks >> 1) * 128 + (ks & 1) * 64 + hh * 16;
+            uint8_t *o = a.hp + (uint64_t)pr * PF_PITCH(768) + (ks >> 1) * 128 + (ks & 1) * 64 + hh * 16;
             *reinterpret_cast<uint4 *>(o) = __builtin_bit_cast(uint4, hi);
             *reinterpret_cast<uint4 *>(o + 32) = __builtin_bit_cast(uint4, lo);
             if (c == 0) a.hs[(uint64_t)pr * 8 + cg] = ok ? exp2i(-sh) : __builtin_nanf("");
@@ -375,7 +306,7 @@ DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
     if (tid < 32 * MT) s_row[tid] = list[min((uint32_t)tid, n - 1)];
     __syncthreads();   // the rows' pairs, and the tables
     uint32_t off[4 * MT];
-    stage_offsets<MT>(off, s_row, 3072u, lane);   // 768 values, 4 bytes each
+    stage_offsets<MT>(off, s_row, PF_PITCH(768), lane);
     stage_rows<MT>(a.hp, off, 0, buf, wave);
     const ALane at = a_lane(lane);
     for (int i = tid; i < 6 * 32 * MT; i += 256)   // the rows' scales of each 128 values

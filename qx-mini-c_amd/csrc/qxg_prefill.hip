@@ -15,257 +15,9 @@
 // lo fp16, |e| <= 2^-22 |x*s|.  A code times an fp16 value is exact in f32; the matrix
 // cores sum the products in f32 over one block (IQ2_XS, IQ3_XXS: 256 values) or one
 // group (IQ4_XS: 32 values), that partial sum is multiplied by its f32 scale once, and
-// the row result is divided by s.  The routed experts' GEMMs are in qxg_pf_experts.hip.
-//
-// Dense GEMMs (Q/K/V, O): MFMA operand layout of v_mfma_f32_32x32x16_f16: lane l holds,
-// for A, row l%32 and k = 8*(l/32) + j (j < 8); for B, column l%32 and the same k; result
-// register r of lane l is (row 8*(r/4) + 4*(l/32) + r%4, column l%32).  Rows are tokens,
-// columns are weight rows, so each lane's results share one weight row and its scale.
-// Activations are packed once per GEMM in exactly this fragment order:
-//     apk[((mtile * KS + kstep) * 2 + piece) * 64 + lane] = 8 fp16 values (uint4).
-#include "qxg_dev.h"
-
-namespace {
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef float f16x __attribute__((ext_vector_type(16)));
-
-enum { FMT_IQ4 = 0, FMT_Q5 = 3 };
-enum { EPI_STORE = 0, EPI_RESID = 1 };
-
-DEV f16x mfma(uint4 a, uint4 b, f16x c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, a), __builtin_bit_cast(h8v, b), c, 0, 0, 0);
-}
-
-DEV uint32_t comp(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
-
-// ---------------------------------------------------------------- weight blocks per lane
-// The lane's share of one 256-value block of its weight row: lane half h = l/32 takes
-// k = 16*s + 8*h + j of every k-step s (16 per block).
-template <int F> struct Blk;
-template <> struct Blk<FMT_IQ4> { uint2 q[8]; uint2 m; };                 // qs bytes 16ib+8h..+8, meta
-template <> struct Blk<FMT_Q5> { uint2 q[8]; uint2 qh[2]; uint4 m; };     // qs 32p+16t+8h..+8, qh 16t+8h..+8, meta
-
-DEV void blk_load(Blk<FMT_IQ4> &b, const PfMat &w, uint64_t bi, int h) {
-    const uint8_t *q = w.qs + bi * 128 + 8 * h;
-#pragma unroll
-    for (int ib = 0; ib < 8; ++ib) b.q[ib] = *reinterpret_cast<const uint2 *>(q + 16 * ib);
-    b.m = *reinterpret_cast<const uint2 *>(w.p1 + bi * 8);
-}
-
-DEV void blk_load(Blk<FMT_Q5> &b, const PfMat &w, uint64_t bi, int h) {
-    const uint8_t *q = w.qs + bi * 128 + 8 * h;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) b.q[i] = *reinterpret_cast<const uint2 *>(q + 32 * (i >> 1) + 16 * (i & 1));
-    b.qh[0] = *reinterpret_cast<const uint2 *>(w.p2 + bi * 32 + 8 * h);
-    b.qh[1] = *reinterpret_cast<const uint2 *>(w.p2 + bi * 32 + 16 + 8 * h);
-    b.m = *reinterpret_cast<const uint4 *>(w.p1 + bi * 16);
-}
-// B fragment of k-step s (8 fp16 codes).
-// IQ4_XS (src/qx_format.c:2032-2053): element 32ib+j = kvalue[qs[16ib+j] & 15],
-// 32ib+16+j = kvalue[qs[16ib+j] >> 4]; k-step 2ib takes the low nibbles of the lane's
-// 8 bytes, 2ib+1 the high nibbles.
-DEV uint4 frag(const Blk<FMT_IQ4> &b, int s, const uint32_t *KV2) {
-    const uint2 q = b.q[s >> 1];
-    uint32_t p[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        p[j] = KV2[(q.x >> (8 * j)) & 255u];
-        p[4 + j] = KV2[(q.y >> (8 * j)) & 255u];
-    }
-    const uint32_t sel = (s & 1) ? 0x07060302u : 0x05040100u;
-    return make_uint4(perm(p[1], p[0], sel), perm(p[3], p[2], sel), perm(p[5], p[4], sel), perm(p[7], p[6], sel));
-}
-// Q5_K (src/qx_format.c:2112-2145): element 32ib+l has the 5-bit code (nibble ib&1 of
-// qs[32(ib/2)+l]) | (bit ib of qh[l]) << 4 and w = d*sc*code - dmin*m; k-step s = 2ib + t
-// takes l = 16t + 8h + j.  Codes 0..31 go to fp16 exactly as bits(1024 + c) - 1024.
-DEV uint32_t u8pair_h2(uint32_t w4, bool hi) {
-    const h2v v = __builtin_bit_cast(h2v, perm(0u, w4, hi ? 0x0c030c02u : 0x0c010c00u) | 0x64006400u);
-    const h2v k = {(_Float16)1024.0f, (_Float16)1024.0f};
-    return __builtin_bit_cast(uint32_t, v - k);
-}
-DEV uint4 frag(const Blk<FMT_Q5> &b, int s, const uint32_t *) {
-    const int ib = s >> 1, t = s & 1;
-    const uint2 q = b.q[2 * (ib >> 1) + t], qh = b.qh[t];
-    const uint32_t nsh = 4 * (ib & 1);
-    const uint32_t c0 = ((q.x >> nsh) & 0x0f0f0f0fu) | (((qh.x >> ib) & 0x01010101u) << 4);
-    const uint32_t c1 = ((q.y >> nsh) & 0x0f0f0f0fu) | (((qh.y >> ib) & 0x01010101u) << 4);
-    return make_uint4(u8pair_h2(c0, false), u8pair_h2(c0, true), u8pair_h2(c1, false), u8pair_h2(c1, true));
-}
-// f32 scale of the partial sums: group ib's d*(ls-32)
-DEV float blk_scale(const Blk<FMT_IQ4> &b, int ib) {
-    const uint32_t sh = b.m.x >> 16, sl = (b.m.y >> (8 * (ib >> 1))) & 255u;
-    const int ls = (int)(((sl >> (4 * (ib & 1))) & 15u) | (((sh >> (2 * ib)) & 3u) << 4));
-    return fp16_exact(b.m.x & 0xffffu) * (float)(ls - 32);
-}
-// Q5_K sub-block ib: scale d*sc and offset dmin*m (6-bit sc, m: get_scale_min_k4,
-// src/qx_format.c:2079-2087); meta = {d, dmin, scales[12]}
-DEV uint32_t q5_scale_byte(const uint4 &m, int i) { return (comp(m, 1 + (i >> 2)) >> (8 * (i & 3))) & 255u; }
-DEV void q5_sc_m(const Blk<FMT_Q5> &b, int ib, uint32_t &sc, uint32_t &mn) {
-    if (ib < 4) {
-        sc = q5_scale_byte(b.m, ib) & 63u;
-        mn = q5_scale_byte(b.m, ib + 4) & 63u;
-    } else {
-        sc = (q5_scale_byte(b.m, ib + 4) & 15u) | ((q5_scale_byte(b.m, ib - 4) >> 6) << 4);
-        mn = (q5_scale_byte(b.m, ib + 4) >> 4) | ((q5_scale_byte(b.m, ib) >> 6) << 4);
-    }
-}
-DEV float blk_scale(const Blk<FMT_Q5> &b, int ib) {
-    uint32_t sc, mn;
-    q5_sc_m(b, ib, sc, mn);
-    return fp16_exact(b.m.x & 0xffffu) * (float)sc;
-}
-template <int F> DEV float blk_offset(const Blk<F> &, int) { return 0.0f; }
-DEV float blk_offset(const Blk<FMT_Q5> &b, int ib) {
-    uint32_t sc, mn;
-    q5_sc_m(b, ib, sc, mn);
-    return fp16_exact(b.m.x >> 16) * (float)mn;
-}
-
-DEV f16x zero16() {
-    f16x z;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = 0.0f;
-    return z;
-}
-}  // namespace
-
-// ================================================================= GEMM
-// One wave: a column tile of 32 weight rows x a row tile of 32 tokens, over all of K.
-// Workgroup = 4 waves on 4 consecutive column tiles of the same row tile.  The row tile's
-// fragments of one 256-value block (32 KiB) are copied by the whole workgroup into one of
-// two LDS stages while the previous block is multiplied, and the next block's weights are
-// loaded into registers at the same time, so each block's loads have one block of matrix
-// work to arrive.  The loop has no data-dependent branches: the last iteration re-loads the
-// last block (never used).
-// A fragments of block kb: thread tid holds uint4 tid + 256*i (i < 8), kept in native
-// 4-dword vectors (register-promoted; the uint4 struct array is not)
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-DEV void a_load(v4u (&ra)[8], const uint4 *A, uint32_t kb) {
-    const v4u *a = reinterpret_cast<const v4u *>(A);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ra[i] = a[(uint64_t)kb * 16 * 128 + 256 * i];
-}
-DEV void a_store(const v4u (&ra)[8], uint4 *stage, int tid) {
-    v4u *st = reinterpret_cast<v4u *>(stage);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) st[tid + 256 * i] = ra[i];
-}
-
-// the 16 k-steps of one block: partial sums per group of two k-steps, each scaled once into acc
-template <int F>
-DEV void block_mma(const Blk<F> &bk, const uint4 *sa, f16x &acc, const uint32_t *t, int lane) {
-    float scl[8], ofs[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        scl[q] = blk_scale(bk, q);
-        ofs[q] = F == FMT_Q5 ? blk_offset(bk, q) : 0.0f;
-    }
-    f16x G = zero16(), S = zero16();   // S, Q5_K: sums of the activations over the group (B = all ones), for the dmin term
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const uint4 ah = sa[s * 128 + lane], al = sa[s * 128 + 64 + lane];
-        if (F == FMT_Q5) {
-            const uint4 ones = make_uint4(0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u);   // fp16 1.0
-            S = mfma(ah, ones, S);
-            S = mfma(al, ones, S);
-        }
-        const uint4 b = frag(bk, s, t);
-        G = mfma(ah, b, G);
-        G = mfma(al, b, G);
-        if (s & 1) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[r] = fmaf(scl[s >> 1], G[r], acc[r]);
-                if (F == FMT_Q5) acc[r] = fmaf(-ofs[s >> 1], S[r], acc[r]);
-            }
-            G = zero16();
-            if (F == FMT_Q5) S = zero16();
-        }
-        // LDS reads of later k-steps stay behind this point: the unrolled loop would
-        // otherwise hoist all of them into registers
-        if (s & 1) asm volatile("" ::: "memory");
-    }
-}
-
-// XCD-aware tile order.  Workgroups go to the 8 XCDs round-robin by linear index, and each
-// XCD has its own L2, so a row tile's packed activations are fetched once into every L2
-// whose XCD runs one of its column workgroups, and a weight column group once into every
-// L2 that runs one of its row tiles.  Workgroup L (on XCD r = L % 8) takes the tile
-// (x, y) with y % a == r / b and x % b == r % b, a = xcd_rows row classes, b = 8 / a column
-// classes: each XCD then reads 1/a of the activations and 1/b of the weights.  The
-// launcher makes gridDim.x a multiple of b and gridDim.y of a (extra rows return).
-DEV void xcd_tile(uint32_t a, uint32_t &bx, uint32_t &by) {
-    const uint32_t L = blockIdx.x + gridDim.x * blockIdx.y, r = L & 7u, j = L >> 3;
-    const uint32_t b = 8u / a, nxb = gridDim.x / b;
-    bx = (j % nxb) * b + r % b;
-    by = (j / nxb) * a + r / b;
-}
-
-template <int F, int EPI>
-__global__ __launch_bounds__(256, 2) void qxp_gemm(PfGemm g, PfTables P) {
-    uint32_t bx, mt0;
-    xcd_tile(g.xcd_rows, bx, mt0);
-    if (mt0 >= g.mtiles) return;   // whole workgroup: a padding row
-    __shared__ uint32_t s_t[F == FMT_IQ4 ? 256 : 1];
-    __shared__ uint4 s_a[2 * 2048];   // [stage][(kstep*2 + piece)*64 + lane]
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
-    if (F == FMT_IQ4) s_t[tid] = P.kv2[tid];
-    const uint32_t KB = g.kb, KS = 16 * KB;
-    const uint32_t c = 32 * (bx * 4 + wave);   // first output column
-    const int mi = c >= g.w_start[2] ? 2 : c >= g.w_start[1] ? 1 : 0;
-    const PfMat W = g.w[mi];
-    const uint64_t rowblk = (uint64_t)(c - g.w_start[mi] + col) * KB;
-    const uint4 *A = g.apk + (uint64_t)mt0 * KS * 128 + tid;
-    uint4 *stage0 = s_a, *stage1 = s_a + 2048;
-
-    f16x acc = zero16();
-    // weights of even blocks in b0, odd blocks in b1; A of block kb in stage kb&1
-    Blk<F> b0, b1;
-    v4u ra[8];
-    const uint32_t k1 = KB > 1 ? 1 : 0;
-    blk_load(b0, W, rowblk, h);
-    a_load(ra, A, 0);
-    a_store(ra, stage0, tid);
-    a_load(ra, A, k1);
-    blk_load(b1, W, rowblk + k1, h);
-    __syncthreads();   // tables and stage 0
-
-    // per block: multiply, stage the next block's A (its stage was last read two blocks
-    // back, before the barrier that ended the previous block), then start the loads of
-    // the block after it (clamped to the last block: always in bounds, never used)
-#pragma unroll 1
-    for (uint32_t kb = 0; kb < KB; kb += 2) {
-        block_mma<F>(b0, stage0, acc, s_t, lane);
-        a_store(ra, stage1, tid);
-        {
-            const uint32_t kn = kb + 2 < KB ? kb + 2 : KB - 1;
-            a_load(ra, A, kn);
-            blk_load(b0, W, rowblk + kn, h);
-        }
-        __syncthreads();
-        if (kb + 1 >= KB) break;
-        block_mma<F>(b1, stage1, acc, s_t, lane);
-        a_store(ra, stage0, tid);
-        {
-            const uint32_t kn = kb + 3 < KB ? kb + 3 : KB - 1;
-            a_load(ra, A, kn);
-            blk_load(b1, W, rowblk + kn, h);
-        }
-        __syncthreads();
-    }
-
-    // epilogue: lane's column c + col, rows 8*(r/4) + 4h + r%4 of the row tile
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t row = mt0 * 32 + 4 * h + 8 * (r >> 2) + (r & 3);
-        if (row >= g.nvalid) continue;
-        float y = acc[r] * g.rscale[row];
-        y = isfinite(y) ? y : 0.0f;   // non-finite projection outputs -> 0 (src/qx_format.c:4284)
-        const uint64_t o = (uint64_t)row * g.ld + c + col;
-        g.out[o] = EPI == EPI_RESID ? g.resid[o] + y : y;
-    }
-}
+// the row result is divided by s.  The GEMMs are in qxg_pf_dense.hip (Q/K/V, O) and
+// qxg_pf_experts.hip; here are the stages between them.
+#include "qxg_pf.h"
 
 // ================================================================= element-wise stages
 // Q4_K embedding rows of tokens[0..T) (src/qx_format.c:3759-3793); block per token.
@@ -289,172 +41,217 @@ extern "C" __global__ __launch_bounds__(256) void qxp_norm(const float *x, const
     for (int i = 0; i < 8; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 }
 
-// shift of the power-of-two scale 2^sh that takes a row's largest magnitude (mx: the lane's)
-// into [2^13, 2^14); every lane gets it
-DEV int row_shift(float mx, bool ok) {
-    mx = fmaxf(mx, dppf<DPP_XOR1>(mx)); mx = fmaxf(mx, dppf<DPP_XOR2>(mx));
-    mx = fmaxf(mx, dppf<DPP_ROR4>(mx)); mx = fmaxf(mx, dppf<DPP_ROR8>(mx));
-    mx = fmaxf(fmaxf(rdlanef(mx, 0), rdlanef(mx, 16)), fmaxf(rdlanef(mx, 32), rdlanef(mx, 48)));
-    int ex = 0;
-    if (mx > 0.0f && ok) (void)frexpf(mx, &ex);   // mx = f * 2^ex, f in [0.5, 1)
-    const int sh = 14 - ex;
-    return sh > 100 ? 100 : sh < -100 ? -100 : sh;
+// ---- rows of a token, block per token: thread tid holds values 8 tid .. 8 tid + 7.  (A wave per
+// token with 32 values a lane left these stages waiting on one chain of loads after another:
+// adding up 8 parts of Q/K/V took 45 us for 8 tokens.)
+namespace {
+DEV void load8(const float *p, float (&v)[8]) {
+    const float4 a = reinterpret_cast<const float4 *>(p)[0], b = reinterpret_cast<const float4 *>(p)[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
-
-// Packs one row of the A operand held by a wave, NC chunks of 8 values per lane (chunk
-// index c[i]): scaled by a power of two and split into fp16 hi/lo fragments; rscale[r]
-// = 1/s, or 0 (and zeros) when the row has a non-finite value.
-template <int NC, int K>
-DEV void pack_row(const float (&v)[NC][8], const int (&c)[NC], uint32_t r, uint4 *apk, float *rscale) {
-    constexpr int CH = K / 8, KS = K / 16;
-    const int lane = threadIdx.x & 63;
+DEV void store8(float *p, const float (&v)[8]) {
+    reinterpret_cast<float4 *>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<float4 *>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+// RMSNorm of the block's 2048 values (qx_apply_f32_rmsnorm, src/qx_format.c:3358-3371; rmsnorm32's
+// arithmetic, the squares summed in another order, in double)
+DEV void block_rmsnorm(float (&v)[8], const float (&w)[8], double *red) {
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += (double)v[i] * (double)v[i];
+    ss = wave_total_d(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    const double inv = 1.0 / sqrt(((red[0] + red[1]) + (red[2] + red[3])) / 2048.0 + 1.0e-6);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (float)((double)v[i] * inv) * w[i];
+}
+// shift sh of the power-of-two scale that takes the block's largest magnitude into [2^13, 2^14);
+// false when a value is not finite (the row then packs zeros under a scale of 0)
+template <int N>
+DEV bool block_shift(const float (&v)[N], float *red, int &sh) {
     float mx = 0.0f;
     bool fin = true;
 #pragma unroll
-    for (int i = 0; i < NC; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            fin = fin && isfinite(v[i][j]);
-            mx = fmaxf(mx, fabsf(v[i][j]));
-        }
-    const bool ok = __ballot(!fin) == 0;
-    const int sh = row_shift(mx, ok);
-    const float sc = ldexpf(1.0f, sh);
-    if (lane == 0) rscale[r] = ok ? ldexpf(1.0f, -sh) : 0.0f;
-    const uint32_t mt = r >> 5, i32 = r & 31;
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        if (c[i] >= CH) continue;
-        h8v hi, lo;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float y = ok ? v[i][j] * sc : 0.0f;
-            const _Float16 a = (_Float16)y;
-            hi[j] = a;
-            lo[j] = (_Float16)(y - (float)a);
-        }
-        const uint64_t base = ((uint64_t)mt * KS + (c[i] >> 1)) * 128 + i32 + 32 * (c[i] & 1);
-        apk[base] = __builtin_bit_cast(uint4, hi);
-        apk[base + 64] = __builtin_bit_cast(uint4, lo);
-    }
-}
-
-// Packs row r < rows of the O GEMM's A operand from the 4096-value rows of src; rows r >=
-// nvalid pack zeros.  Wave per row, chunks lane + 64 i, no workgroup barriers.
-extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src, uint32_t rows, uint32_t nvalid, uint4 *apk,
-                                                               float *rscale) {
-    constexpr int PL = 8;
-    const int lane = threadIdx.x & 63;
-    const uint32_t r = blockIdx.x * 4 + wave_id();
-    if (r >= rows) return;   // whole wave
-    float v[PL][8];
-    int c[PL];
-#pragma unroll
-    for (int i = 0; i < PL; ++i) {
-        c[i] = lane + 64 * i;
-        if (r < nvalid) {
-            const float4 *p = reinterpret_cast<const float4 *>(src + (uint64_t)r * 4096 + 8 * c[i]);
-            const float4 a = p[0], b = p[1];
-            v[i][0] = a.x; v[i][1] = a.y; v[i][2] = a.z; v[i][3] = a.w;
-            v[i][4] = b.x; v[i][5] = b.y; v[i][6] = b.z; v[i][7] = b.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
-        }
-    }
-    pack_row<PL, 4096>(v, c, r, apk, rscale);
-}
-
-// RMSNorm of each token's 2048-vector (qx_apply_f32_rmsnorm, src/qx_format.c:3358-3371) as
-// f32 rows for the router and as the gate/up GEMM's packed rows (lines of two k-steps,
-// [hi, lo][h][8] each; k-step 16 b + s and lane half h hold K = 256 b + 128 h + 8 s + j);
-// rscale[t] = 1/s, or 0 (and zeros) when the row has a non-finite value.  Wave per token, 32
-// values a lane.
-extern "C" __global__ __launch_bounds__(256) void qxp_ffn_norm(const float *x, const float *w, uint32_t T, float *y,
-                                                               uint8_t *xp, float *rscale) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t t = blockIdx.x * 4 + wave_id();
-    if (t >= T) return;   // whole wave
-    float v[32], ww[32];
-    load32(x + (uint64_t)t * 2048 + 32 * lane, v);
-    load32(w + 32 * lane, ww);
-    rmsnorm32(v, ww);
-    float4 *o = reinterpret_cast<float4 *>(y + (uint64_t)t * 2048 + 32 * lane);
-    float mx = 0.0f;
-    bool fin = true;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < N; ++i) {
         fin = fin && isfinite(v[i]);
         mx = fmaxf(mx, fabsf(v[i]));
     }
+    mx = block_max256(fin ? mx : INFINITY, red);
+    sh = 140 - (int)(__float_as_uint(mx) >> 23);
+    sh = sh > 100 ? 100 : sh < -100 ? -100 : sh;
+    return mx < INFINITY;
+}
+// 8 values as fp16 hi + lo at their chunk's place; returns the scaled values' sum
+DEV float pack8(const float *v, float sc, bool ok, uint8_t *at) {
+    h8v hi, lo;
+    float t = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    const bool ok = __ballot(!fin) == 0;
-    const int sh = row_shift(mx, ok);
-    const float sc = ldexpf(1.0f, sh);
-    if (lane == 0) rscale[t] = ok ? ldexpf(1.0f, -sh) : 0.0f;
+    for (int j = 0; j < 8; ++j) {
+        const float y = ok ? v[j] * sc : 0.0f;
+        const _Float16 a = (_Float16)y;
+        hi[j] = a;
+        lo[j] = (_Float16)(y - (float)a);
+        t += y;
+    }
+    *reinterpret_cast<uint4 *>(at) = __builtin_bit_cast(uint4, hi);
+    *reinterpret_cast<uint4 *>(at + 32) = __builtin_bit_cast(uint4, lo);
+    return t;
+}
+// chunk c (8 values) of a dense row (k-steps of 16 consecutive values) and its line's sum
+DEV void pack_dense8(const float *v, float sc, bool ok, uint8_t *row, float *sums, uint32_t c) {
+    float t = pack8(v, sc, ok, row + (c >> 2) * 128 + 64 * ((c >> 1) & 1) + 16 * (c & 1));
+    t += dppf<DPP_XOR1>(t);
+    t += dppf<DPP_XOR2>(t);
+    if ((c & 3) == 0) sums[c >> 2] = t;
+}
+// v = the sum of `parts` rows of 8 values, stride floats apart, in order
+DEV void sum_parts(const float *p, uint64_t stride, uint32_t parts, float (&v)[8]) {
+    load8(p, v);
+    uint32_t k = 1;
+    for (; k + 4 <= parts; k += 4) {
+        float q[4][8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t c = 4 * lane + i, at = (16 * (c >> 5) + (c & 15)) * 64 + ((c >> 4) & 1) * 16;
-        h8v hi, lo;
+        for (int u = 0; u < 4; ++u) load8(p + (k + u) * stride, q[u]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float q = ok ? v[8 * i + j] * sc : 0.0f;
-            const _Float16 a = (_Float16)q;
-            hi[j] = a;
-            lo[j] = (_Float16)(q - (float)a);
-        }
-        *reinterpret_cast<uint4 *>(xp + (uint64_t)t * 8192 + at) = __builtin_bit_cast(uint4, hi);
-        *reinterpret_cast<uint4 *>(xp + (uint64_t)t * 8192 + at + 32) = __builtin_bit_cast(uint4, lo);
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] += q[u][i];
+    }
+    for (; k < parts; ++k) {
+        float q[8];
+        load8(p + k * stride, q);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += q[i];
     }
 }
-
-// RMSNorm of token r (32 consecutive values per lane) fused with
-// its packing as the Q/K/V GEMM's A operand; rows r >= nvalid pack zeros.
-extern "C" __global__ __launch_bounds__(256) void qxp_norm_pack(const float *x, const float *w, uint32_t rows,
-                                                                uint32_t nvalid, uint4 *apk, float *rscale) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t r = blockIdx.x * 4 + wave_id();
-    if (r >= rows) return;   // whole wave
-    float v[4][8];
-    const int c[4] = {4 * lane, 4 * lane + 1, 4 * lane + 2, 4 * lane + 3};
-    if (r < nvalid) {
-        float t[32], ww[32];
-        load32(x + (uint64_t)r * 2048 + 32 * lane, t);
-        load32(w + 32 * lane, ww);
-        rmsnorm32(t, ww);
+// x1 + sum_r (float)(w_r * (double)y[8 t + r]), ranks in order (src/qx_format.c:5296-5309)
+DEV void combine8(const float *x1, const float *y, const double *wts, uint32_t t, int tid, float (&v)[8], float *moe) {
+    float q[QXG_TOPK][8];
+    double w[QXG_TOPK];
 #pragma unroll
-        for (int i = 0; i < 32; ++i) v[i >> 3][i & 7] = t[i];
+    for (int r = 0; r < QXG_TOPK; ++r) {
+        load8(y + ((uint64_t)t * 8 + r) * 2048 + 8 * tid, q[r]);
+        w[r] = wts[t * 8 + r];
+    }
+    load8(x1 + (uint64_t)t * 2048 + 8 * tid, v);
+    float m[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        m[i] = 0.0f;
+#pragma unroll
+        for (int r = 0; r < QXG_TOPK; ++r) m[i] += (float)(w[r] * (double)q[r][i]);
+        v[i] += m[i];
+    }
+    if (moe) store8(moe + (uint64_t)t * 2048 + 8 * tid, m);
+}
+}  // namespace
+
+// The layer's input and its RMSNorm packed as the Q/K/V GEMM's rows.  With y, the input is the
+// layer before's combined experts (combine8 on its x1, y and weights), stored to x.
+extern "C" __global__ __launch_bounds__(256) void qxp_norm_pack(float *x, const float *x1, const float *y, const double *wts,
+        const float *w, uint8_t *xp, float *rscale, float *sums) {
+    __shared__ double red[4];
+    __shared__ float redf[4];
+    const int tid = threadIdx.x;
+    const uint32_t t = blockIdx.x;
+    float v[8], ww[8];
+    load8(w + 8 * tid, ww);
+    if (y) {
+        combine8(x1, y, wts, t, tid, v, nullptr);
+        store8(x + (uint64_t)t * 2048 + 8 * tid, v);
     } else {
-#pragma unroll
-        for (int i = 0; i < 32; ++i) v[i >> 3][i & 7] = 0.0f;
+        load8(x + (uint64_t)t * 2048 + 8 * tid, v);
     }
-    pack_row<4, 2048>(v, c, r, apk, rscale);
+    block_rmsnorm(v, ww, red);
+    int sh;
+    const bool ok = block_shift<8>(v, redf, sh);
+    if (tid == 0) rscale[t] = ok ? ldexpf(1.0f, -sh) : 0.0f;
+    pack_dense8(v, ldexpf(1.0f, sh), ok, xp + (uint64_t)t * PF_PITCH(2048), sums + (uint64_t)t * 64, tid);
 }
 
-// Per token (block): q/k head RMSNorm (src/qx_format.c:3740-3757) and RoPE at position
+// The O projection's rows from the 4096-value context rows
+extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src, uint8_t *xp, float *rscale, float *sums) {
+    __shared__ float redf[4];
+    const int tid = threadIdx.x;
+    const uint32_t t = blockIdx.x;
+    float v[16], a[8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        load8(src + (uint64_t)t * 4096 + 2048 * i + 8 * tid, a);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[8 * i + j] = a[j];
+    }
+    int sh;
+    const bool ok = block_shift<16>(v, redf, sh);
+    if (tid == 0) rscale[t] = ok ? ldexpf(1.0f, -sh) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        pack_dense8(v + 8 * i, ldexpf(1.0f, sh), ok, xp + (uint64_t)t * PF_PITCH(4096), sums + (uint64_t)t * 128, tid + 256 * i);
+}
+
+// The attention half's residual x1 = x + O (the O projection's parts of K added in order, a
+// non-finite result 0, src/qx_format.c:4284) and its RMSNorm as f32 rows for the router and
+// as the gate/up GEMM's packed rows (k-step 16 b + s and lane half h hold K = 256 b + 128 h +
+// 8 s + j).
+extern "C" __global__ __launch_bounds__(256) void qxp_ffn_norm(const float *x, const float *parts, uint32_t nparts,
+        const float *w, uint32_t T, float *x1, float *y, uint8_t *xp, float *rscale) {
+    __shared__ double red[4];
+    __shared__ float redf[4];
+    const int tid = threadIdx.x;
+    const uint32_t t = blockIdx.x;
+    const uint64_t at = (uint64_t)t * 2048 + 8 * tid;
+    float v[8], r[8], ww[8];
+    load8(x + at, r);
+    load8(w + 8 * tid, ww);
+    sum_parts(parts + at, (uint64_t)T * 2048, nparts, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = r[i] + (isfinite(v[i]) ? v[i] : 0.0f);
+    store8(x1 + at, v);
+    block_rmsnorm(v, ww, red);
+    store8(y + at, v);
+    int sh;
+    const bool ok = block_shift<8>(v, redf, sh);
+    if (tid == 0) rscale[t] = ok ? ldexpf(1.0f, -sh) : 0.0f;
+    const uint32_t c = tid;
+    pack8(v, ldexpf(1.0f, sh), ok, xp + (uint64_t)t * PF_PITCH(2048) + (16 * (c >> 5) + (c & 15)) * 64 + ((c >> 4) & 1) * 16);
+}
+
+// Per token (block): the Q/K/V GEMM's parts of K added in order (non-finite results 0,
+// src/qx_format.c:4284), q/k head RMSNorm (src/qx_format.c:3740-3757) and RoPE at position
 // p0+t (4625-4641), INT8 quantization of K and V over all 512 values (4449-4463) into
 // the cache row [layer][p0+t]; the roped q (f32) goes to qr for attention.
-extern "C" __global__ __launch_bounds__(256) void qxp_qk(const float *qkv, const float *q_norm, const float *k_norm,
-        Tables T, int8_t *kc, int8_t *vc, float *ks, float *vs, uint32_t layer, uint32_t ctx, uint32_t p0, float *qr) {
-    __shared__ float s_k[512], s_v[512];
+extern "C" __global__ __launch_bounds__(256) void qxp_qk(const float *parts, uint32_t nparts, uint32_t rows, const float *q_norm,
+        const float *k_norm, Tables T, int8_t *kc, int8_t *vc, float *ks, float *vs, uint32_t layer, uint32_t ctx, uint32_t p0,
+        float *qr) {
+    __shared__ float s_row[5120], s_k[512];
     __shared__ float red[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const uint32_t t = blockIdx.x, pos = p0 + t;
-    const float *row = qkv + (uint64_t)t * 5120;
-    float k0 = row[4096 + 128 * wave + lane], k1 = row[4096 + 128 * wave + 64 + lane];
-    const float v0 = row[4608 + tid], v1 = row[4608 + 256 + tid];
     const float kw0 = k_norm[lane], kw1 = k_norm[64 + lane], qw0 = q_norm[lane], qw1 = q_norm[64 + lane];
     const double c = T.rope_cos[pos * 64 + lane], s = T.rope_sin[pos * 64 + lane];
+    float v[3][8];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        if (i < 2 || tid < 128) sum_parts(parts + (uint64_t)t * 5120 + 2048 * i + 8 * tid, (uint64_t)rows * 5120, nparts, v[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        if (i < 2 || tid < 128) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[i][j] = isfinite(v[i][j]) ? v[i][j] : 0.0f;
+            store8(s_row + 2048 * i + 8 * tid, v[i]);
+        }
+    __syncthreads();
+    float k0 = s_row[4096 + 128 * wave + lane], k1 = s_row[4096 + 128 * wave + 64 + lane];
+    const float v0 = s_row[4608 + tid], v1 = s_row[4608 + 256 + tid];
     head_norm_rope_wave(k0, k1, kw0, kw1, c, s);
     s_k[128 * wave + lane] = k0;
     s_k[128 * wave + 64 + lane] = k1;
-    s_v[tid] = v0;
-    s_v[256 + tid] = v1;
-#pragma unroll 1
+#pragma unroll 2
     for (int hh = 0; hh < 8; ++hh) {
         const int qh = 8 * wave + hh;
-        float q0 = row[128 * qh + lane], q1 = row[128 * qh + 64 + lane];
+        float q0 = s_row[128 * qh + lane], q1 = s_row[128 * qh + 64 + lane];
         head_norm_rope_wave(q0, q1, qw0, qw1, c, s);
         qr[(uint64_t)t * 4096 + 128 * qh + lane] = q0;
         qr[(uint64_t)t * 4096 + 128 * qh + 64 + lane] = q1;
@@ -466,7 +263,7 @@ extern "C" __global__ __launch_bounds__(256) void qxp_qk(const float *qkv, const
     const uint64_t slot = (uint64_t)layer * ctx + pos;
     for (int i = tid; i < 512; i += 256) {
         kc[slot * 512 + i] = int8_code(s_k[i], kscale);
-        vc[slot * 512 + i] = int8_code(s_v[i], vscale);
+        vc[slot * 512 + i] = int8_code(i < 256 ? v0 : v1, vscale);
     }
     if (tid == 0) { ks[slot] = kscale; vs[slot] = vscale; }
 }
@@ -743,7 +540,7 @@ extern "C" __global__ __launch_bounds__(512) void qxp_router(const float *xn, co
 // Top-8 experts and renormalised weights per token (the decode path's selection,
 // src/qx_format.c:5265-5285), and the experts' pair lists: pair p = 8 t + rank joins list e at
 // the next free place.  The order within a list varies from run to run; a pair's row of the
-// expert GEMMs does not depend on its place.  A workgroup takes 32 tokens, two a wave, counts
+// expert GEMMs does not depend on its place.  A workgroup takes 16 tokens, one a wave, counts
 // its pairs by expert in LDS and claims the list places with one atomic per expert (pairs that
 // each took their place themselves waited on the crowded experts' counters: 20 us).
 extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logits, uint32_t T, uint32_t experts,
@@ -753,76 +550,36 @@ extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logit
     if (tid < 128) s_n[tid] = 0u;
     __syncthreads();
     const int E = (int)experts;
-    uint32_t e[2] = {0, 0}, place[2] = {0, 0};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t t = blockIdx.x * 32 + 2 * wave_id() + i;
-        if (t >= T) break;   // whole wave
+    const uint32_t t = blockIdx.x * 16 + wave_id();
+    uint32_t e = 0, place = 0;
+    if (t < T) {   // whole wave
         const double l0 = lane < E ? logits[(uint64_t)t * 128 + lane] : 0.0;
         const double l1 = lane + 64 < E ? logits[(uint64_t)t * 128 + lane + 64] : 0.0;
         uint32_t id[QXG_TOPK];
         double w[QXG_TOPK];
         wave_top8(l0, l1, E, id, w);
+        double wl = 0.0;
 #pragma unroll
         for (int q = 0; q < QXG_TOPK; ++q)
             if (lane == q) {
-                e[i] = id[q] < experts ? id[q] : 0u;
-                wts[t * 8 + q] = w[q];
-                place[i] = atomicAdd(&s_n[e[i]], 1u);
+                e = id[q] < experts ? id[q] : 0u;
+                wl = w[q];
             }
+        if (lane < QXG_TOPK) {
+            wts[t * 8 + lane] = wl;
+            place = atomicAdd(&s_n[e], 1u);
+        }
     }
     __syncthreads();
     if (tid < 128 && s_n[tid]) s_at[tid] = atomicAdd(&cnt[tid], s_n[tid]);
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t t = blockIdx.x * 32 + 2 * wave_id() + i;
-        if (t < T && lane < QXG_TOPK) list[(uint64_t)e[i] * QXP_LIST + s_at[e[i]] + place[i]] = t * 8 + lane;
-    }
+    if (t < T && lane < QXG_TOPK) list[(uint64_t)e * QXP_LIST + s_at[e] + place] = t * 8 + lane;
 }
 
-// x[t][i] = x1[t][i] + sum_r (float)(w_r * (double)y[8 t + r][i]), ranks in order
-// (src/qx_format.c:5296-5309); block per token.
+// The last layer's output x = x1 + its combined experts (moe_dump: the expert sum alone)
 extern "C" __global__ __launch_bounds__(256) void qxp_combine(const float *x1, const float *y, const double *wts, float *x,
                                                               float *moe_dump) {
-    const uint32_t t = blockIdx.x;
-    double w[QXG_TOPK];
-#pragma unroll
-    for (int r = 0; r < QXG_TOPK; ++r) w[r] = wts[t * 8 + r];
-    for (int i = threadIdx.x; i < 2048; i += 256) {
-        float m = 0.0f;
-#pragma unroll
-        for (int r = 0; r < QXG_TOPK; ++r) m += (float)(w[r] * (double)y[((uint64_t)t * 8 + r) * 2048 + i]);
-        if (moe_dump) moe_dump[(uint64_t)t * 2048 + i] = m;
-        x[(uint64_t)t * 2048 + i] = x1[(uint64_t)t * 2048 + i] + m;
-    }
-}
-
-// ================================================================= launch wrappers
-extern "C" {
-void qxp_launch_gemm(hipStream_t s, int kind, const PfGemm &g0, const PfTables &P, uint32_t grid_x, uint32_t grid_y,
-                     Timer tm) {
-    // row classes per kind (xcd_tile): Q/K/V 2 (4 MB of activations, 5.6 MB of weights),
-    // O 4 (8 MB, 4.5 MB)
-    PfGemm g = g0;
-    g.xcd_rows = kind == QXP_QKV || kind == QXP_V_Q5 ? 2u : 4u;
-    const uint32_t b = 8u / g.xcd_rows;
-    if (grid_x % b) g.xcd_rows = 8u;   // (the column counts here are multiples of 8 workgroups)
-    grid_y = (grid_y + g.xcd_rows - 1) / g.xcd_rows * g.xcd_rows;
-    const dim3 grid(grid_x, grid_y);
-    switch (kind) {
-    case QXP_QKV:       // Q/K/V (or Q/K): IQ4_XS
-        qx_launch(qxp_gemm<FMT_IQ4, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    case QXP_O:         // O projection + residual: IQ4_XS
-        qx_launch(qxp_gemm<FMT_IQ4, EPI_RESID>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    case QXP_V_Q5:      // V alone: Q5_K
-        qx_launch(qxp_gemm<FMT_Q5, EPI_STORE>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    default:            // O projection + residual: Q5_K
-        qx_launch(qxp_gemm<FMT_Q5, EPI_RESID>, grid, dim3(256), 0, s, tm, g, P);
-        break;
-    }
-}
+    float v[8];
+    combine8(x1, y, wts, blockIdx.x, threadIdx.x, v, moe_dump);
+    store8(x + (uint64_t)blockIdx.x * 2048 + 8 * threadIdx.x, v);
 }

@@ -44,3 +44,27 @@ def test_expert_row_tiles(ctx, models, mix, layer, n):
         assert rel_l2(moe[t], m) <= REL_L2, (t, rel_l2(moe[t], m))
         assert rel_l2(out[t], y) <= REL_L2, (t, rel_l2(out[t], y))
     om.close()
+
+
+@pytest.mark.parametrize("mix,layer", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("n", [1, 8, 32, 33, 64, 65, 128, 129, 257])
+def test_dense_row_tiles_and_parts(ctx, models, mix, layer, n):
+    """Q/K/V and O at the edges of their row tiles, which are also where the number of parts of K
+    changes (8 and 16 parts up to 64 rows, 4 and 8 up to 128, ...): the attention half of the
+    edge rows against the oracle over the GPU's own cache rows, IQ4_XS and Q5_K V and O."""
+    p = models / f"m{mix}.qxf"
+    ctx.load(p)
+    layers = 4 if mix else 1
+    ctx.kv_create(layers, 300)
+    x = np.random.default_rng(70 + n).standard_normal((n, 2048)).astype(np.float32)
+    x[n // 2] *= 1e3
+    fi, _, _ = ctx.prefill_layer(layer, 0, x)
+    okv = qxo.KV(layers, 300)
+    okv.k[layer, :n], okv.v[layer, :n], okv.ks[layer, :n], okv.vs[layer, :n] = ctx.kv_read(layer, 0, n)
+    om = qxo.Model(p)
+    for t in sorted({0, 31, 32, 63, 64, 127, 128, 255, 256, n // 2, n - 1} & set(range(n))):
+        a, _, _, rk, rv, (sk, sv) = qxo.attention_layer_given_row(om, layer, t, okv, x[t])
+        assert rel_l2(fi[t], x[t] + a) <= REL_L2, (t, rel_l2(fi[t], x[t] + a))
+        assert np.abs(okv.k[layer, t].astype(int) - rk.astype(int)).max() <= 1, t
+        assert np.abs(okv.v[layer, t].astype(int) - rv.astype(int)).max() <= 1, t
+    om.close()
