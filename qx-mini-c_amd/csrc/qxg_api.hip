@@ -60,11 +60,11 @@ __global__ void qxp_norm_pack(float *, const float *, const float *, const doubl
 __global__ void qxp_qk(const float *, uint32_t, uint32_t, const float *, const float *, Tables, int8_t *, int8_t *, float *, float *,
                        uint32_t, uint32_t, uint32_t, float *);
 __global__ void qxp_attn(const float *, const int8_t *, const int8_t *, const float *, const float *, uint32_t, uint32_t,
-                         uint32_t, uint32_t, float *);
+                         uint32_t, uint32_t, float *, float2 *);
 __global__ void qxp_router(const float *, const float *, uint32_t, uint32_t, double *, uint32_t *);
 __global__ void qxp_route(const double *, uint32_t, uint32_t, double *, uint32_t *, uint32_t *);
 __global__ void qxp_combine(const float *, const float *, const double *, float *, float *);
-__global__ void qxp_pack_ctx(const float *, uint8_t *, float *, float *);
+__global__ void qxp_pack_ctx(const float *, const float2 *, uint32_t, uint32_t, uint8_t *, float *, float *);
 __global__ void qxp_dense_plane(uint32_t, const uint8_t *, const uint8_t *, const uint8_t *, uint32_t, uint32_t, uint32_t, uint8_t *,
                                 float *, float *);
 void qxp_launch_dense(hipStream_t, const PfDense &, uint32_t, Timer);
@@ -177,6 +177,7 @@ struct qxg_ctx {
         float *X = nullptr, *X1 = nullptr, *XN = nullptr, *PART = nullptr, *QR = nullptr, *CTX = nullptr;
         float *HS = nullptr, *Y = nullptr, *xscale = nullptr, *sums = nullptr, *dump = nullptr;
         uint8_t *XP = nullptr, *HP = nullptr;
+        float2 *md = nullptr;
         double *lg = nullptr, *w = nullptr;
         uint32_t *cnt = nullptr, *list = nullptr, *tokens = nullptr;
         std::vector<void *> all;
@@ -762,6 +763,17 @@ uint32_t dense_parts(uint32_t T, uint32_t cols, uint32_t lines) {
 constexpr uint64_t PF_PART_FLOATS = (uint64_t)QXP_MAX * 5120;
 static_assert(QXP_MAX >= 512, "the parts' buffer");
 
+// Runs of positions of the attention over T tokens and n positions: about 512 workgroups (two fit
+// a CU) of at least four 32-position chunks (one a wave) each.  37 tokens at position 2100 took
+// 60 us as one run (40 workgroups of 67 chunks).
+uint32_t attn_runs(uint32_t T, uint32_t n) {
+    const uint32_t wgs = 4 * ((T + 3) / 4), most = std::max<uint32_t>(1, n / 128);
+    return std::max<uint32_t>(1, std::min<uint32_t>(512 / wgs, most));
+}
+// rows of all runs: runs * T <= 512 / 4 * 4 (T a multiple of 4) and T otherwise no more than that
+constexpr uint64_t PF_CTX_ROWS = QXP_MAX;
+static_assert(QXP_MAX >= 512, "the runs' rows");
+
 bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
     auto &B = c->pf;
     if (B.ready) return true;
@@ -773,7 +785,7 @@ bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
     const uint64_t T = QXP_MAX, PAIRS = T * QXG_TOPK;
     bool ok = alloc((void **)&B.X, T * 2048 * 4) && alloc((void **)&B.X1, T * 2048 * 4) &&
               alloc((void **)&B.XN, T * 2048 * 4) && alloc((void **)&B.PART, PF_PART_FLOATS * 4) &&
-              alloc((void **)&B.QR, T * 4096 * 4) && alloc((void **)&B.CTX, T * 4096 * 4) &&
+              alloc((void **)&B.QR, T * 4096 * 4) && alloc((void **)&B.CTX, PF_CTX_ROWS * 4096 * 4) && alloc((void **)&B.md, PF_CTX_ROWS * 32 * 8) &&
               alloc((void **)&B.XP, T * PF_PITCH(4096)) && alloc((void **)&B.xscale, T * 4) && alloc((void **)&B.HP, PAIRS * PF_PITCH(768)) &&
               alloc((void **)&B.HS, PAIRS * 8 * 4) && alloc((void **)&B.Y, PAIRS * 2048 * 4) &&
               alloc((void **)&B.sums, T * 128 * 4) && alloc((void **)&B.dump, T * 2048 * 4) && alloc((void **)&B.lg, T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
@@ -832,10 +844,12 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, bool first, 
     qxp_launch_dense(s, g, qkv_parts, timer_for(c, 8));
     hipLaunchKernelGGL(qxp_qk, dim3(T), dim3(256), 0, s, (const float *)B.PART, qkv_parts, T, w.q_norm, w.k_norm, c->T, c->kc,
                        c->vc, c->ks, c->vs, l, c->kv_ctx, p0, B.QR);
-    qx_launch(qxp_attn, dim3(4, (T + 3) / 4), dim3(256), 0, s, timer_for(c, 13), (const float *)B.QR,
+    const uint32_t runs = attn_runs(T, p0 + T);
+    qx_launch(qxp_attn, dim3(4, (T + 3) / 4, runs), dim3(256), 0, s, timer_for(c, 13), (const float *)B.QR,
               (const int8_t *)c->kc, (const int8_t *)c->vc, (const float *)c->ks, (const float *)c->vs, l, c->kv_ctx, p0, T,
-              B.CTX);
-    hipLaunchKernelGGL(qxp_pack_ctx, dim3(T), dim3(256), 0, s, (const float *)B.CTX, B.XP, B.xscale, B.sums);
+              B.CTX, B.md);
+    hipLaunchKernelGGL(qxp_pack_ctx, dim3(T), dim3(256), 0, s, (const float *)B.CTX, (const float2 *)B.md, runs, T,
+                       B.XP, B.xscale, B.sums);
     g = dense_args(c, l, false);
     g.part_lines = g.lines / o_parts;
     g.rows_packed = B.XP; g.rows = T; g.row_bytes = PF_PITCH(4096); g.rscale = B.xscale; g.sums = B.sums; g.out = B.PART;

@@ -45,6 +45,7 @@ extern "C" __global__ __launch_bounds__(256) void qxp_norm(const float *x, const
 // token with 32 values a lane left these stages waiting on one chain of loads after another:
 // adding up 8 parts of Q/K/V took 45 us for 8 tokens.)
 namespace {
+DEV float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 DEV void load8(const float *p, float (&v)[8]) {
     const float4 a = reinterpret_cast<const float4 *>(p)[0], b = reinterpret_cast<const float4 *>(p)[1];
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
@@ -171,15 +172,39 @@ extern "C" __global__ __launch_bounds__(256) void qxp_norm_pack(float *x, const 
     pack_dense8(v, ldexpf(1.0f, sh), ok, xp + (uint64_t)t * PF_PITCH(2048), sums + (uint64_t)t * 64, tid);
 }
 
-// The O projection's rows from the 4096-value context rows
-extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src, uint8_t *xp, float *rscale, float *sums) {
+// The O projection's rows from the 4096-value context rows; with several runs of positions,
+// the context is sum_r 2^(m_r - M) acc_r over sum_r 2^(m_r - M) den_r, runs in order.
+extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src, const float2 *md, uint32_t runs, uint32_t T,
+                                                               uint8_t *xp, float *rscale, float *sums) {
     __shared__ float redf[4];
     const int tid = threadIdx.x;
     const uint32_t t = blockIdx.x;
-    float v[16], a[8];
+    float v[16];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        load8(src + (uint64_t)t * 4096 + 2048 * i + 8 * tid, a);
+        const uint32_t d = 2048 * i + 8 * tid, head = d >> 7;
+        float a[8];
+        if (runs == 1) {
+            load8(src + (uint64_t)t * 4096 + d, a);
+        } else {
+            float M = -INFINITY, L = 0.0f;
+            for (uint32_t r = 0; r < runs; ++r) M = fmaxf(M, md[((uint64_t)r * T + t) * 32 + head].x);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] = 0.0f;
+#pragma unroll 4
+            for (uint32_t r = 0; r < runs; ++r) {
+                const float2 s = md[((uint64_t)r * T + t) * 32 + head];
+                const float f = s.x == -INFINITY ? 0.0f : exp2_fast(s.x - M);
+                float b[8];
+                load8(src + ((uint64_t)r * T + t) * 4096 + d, b);
+                L = fmaf(f, s.y, L);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] = fmaf(f, b[j], a[j]);
+            }
+            const float inv = 1.0f / L;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] *= inv;
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[8 * i + j] = a[j];
     }
@@ -269,130 +294,147 @@ extern "C" __global__ __launch_bounds__(256) void qxp_qk(const float *parts, uin
 }
 
 // Causal GQA attention of the chunk on the matrix cores (qx_rope_gqa_attention_partial,
-// src/qx_format.c:5051-5196, for every token of the chunk at once).  A workgroup takes
-// one KV head and 4 consecutive tokens: the 8 q heads of the KV head x 4 tokens are the
-// 32 columns of v_mfma_f32_32x32x16_f16 (column c: head c/4, token c%4).  Its 4 waves
-// take the 32-position chunks ci = wave, wave+4, ... of positions 0..p0+t and keep, per
-// column, a running maximum, denominator and context (online softmax; the reference
-// normalises with the global maximum, the same quantity up to rounding).  Per chunk:
-//   scores  S^T[pos][col] = K8[pos][:] . q[col][:]: A = the chunk's INT8 K codes
-//           (exact in fp16), B = q split hi + lo in fp16 after a power-of-two row
-//           scale (max |q| in [2^13, 2^14)); f32 accumulation; times ks[pos] /
-//           sqrt(128) and the row scale; positions past the token masked;
-//   weights p = exp(s - m) (f32), pv = p * vs[pos], split hi + lo after a power-of-two
-//           scale per column and chunk;
-//   context C[dim][col] += V8^T[dim][pos] . pv[pos][col] (A = V codes from a transposed
-//           LDS copy of the chunk), rescaled by exp(m_old - m_new) per column.
-// The result registers of the score product are exactly the k layout the context
-// product's B operand needs (lane l: column l%32, positions 8(r/4) + 4(l/32) + r%4 of
-// register r), so the weights never leave the lane.  The waves' states are merged in
-// LDS at the end and the context is divided by the denominator.
+// src/qx_format.c:5051-5196, for every token of the chunk at once).  A workgroup takes one KV
+// head, 4 consecutive tokens and a run of 32-position chunks (gridDim.z of them, so that few
+// tokens over a long cache still fill the GPU); the 8 q heads of the KV head x 4 tokens are
+// the 32 columns of v_mfma_f32_32x32x16_f16 (column c: head c/4, token c%4).  Its 4 waves
+// take every fourth chunk and keep, per column, a running maximum, denominator and context.
+// Per chunk:
+//   scores  S^T[pos][col] = K8[pos][:] . q[col][:]: A = the chunk's INT8 K codes (exact in
+//           fp16; lane half h holds dims 64h .. 64h + 63 of a position), B = q split hi + lo
+//           in fp16 after a power-of-two row scale (in LDS, the same for the four waves),
+//           the hi and the lo products summed apart (two chains of matrix instructions);
+//           times ks[pos]; positions past the token masked in the chunks that hold any;
+//   weights e = 2^(score * scale - m), pv = e * vs[pos] split hi + lo under a power-of-two
+//           scale of the column;
+//   context C[dim][col] += V8^T[dim][pos] . pv[pos][col] (A = V codes from a transposed LDS copy
+//           of the chunk), accumulated by the matrix cores.
+// The result registers of the score product are exactly the k layout the context product's B
+// operand needs (lane l: column l%32, positions 8(r/4) + 4(l/32) + r%4 of register r), so the
+// weights never leave the lane.  The softmax's vector work bounds this kernel, about 17 issue
+// slots a score against 64 matrix cycles per 32 of them, so: m is the running maximum only to
+// within a factor 2^8 and the column's scale only to within 2^5 of its largest weight, and the
+// context is rescaled (64 multiplies) only in the chunks that leave those; the exponent is base
+// 2; the next chunk's K and V rows are loaded while the current one is worked on.  The
+// waves' states are merged in LDS, the runs' by qxp_pack_ctx.
 namespace {
 constexpr int PA_TT = 4;   // tokens per workgroup
 
-DEV uint4 i8x8_to_f16(uint2 v) {   // 8 int8 -> 8 exact fp16 (bias 0x64 trick: 1024 + (b ^ 0x80) - 1152)
+DEV uint4 i8x8_to_f16(uint32_t vx, uint32_t vy) {   // 8 int8 -> 8 exact fp16 (bias 0x64 trick: 1024 + (b ^ 0x80) - 1152)
     const h2v bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-    const uint32_t x = v.x ^ 0x80808080u, y = v.y ^ 0x80808080u;
+    const uint32_t x = vx ^ 0x80808080u, y = vy ^ 0x80808080u;
     const uint32_t c = 0x64646464u;
     auto cv = [&](uint32_t w) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, w) - bias); };
     return make_uint4(cv(perm(c, x, 0x04010400u)), cv(perm(c, x, 0x04030402u)), cv(perm(c, y, 0x04010400u)),
                       cv(perm(c, y, 0x04030402u)));
 }
-DEV void split8(const float (&v)[8], float sc, uint4 &hi, uint4 &lo) {   // v * sc = hi + lo (+ 2^-22 rel)
-    uint32_t h[4], l[4];
+DEV void split8(const float *v, float sc, uint4 &hi, uint4 &lo) {   // v * sc = hi + lo (+ 2^-22 rel)
+    h8v h, l;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = v[2 * i] * sc, b = v[2 * i + 1] * sc;
-        const _Float16 ha = (_Float16)a, hb = (_Float16)b;
-        const _Float16 la = (_Float16)(a - (float)ha), lb = (_Float16)(b - (float)hb);
-        const h2v hh = {ha, hb}, ll = {la, lb};
-        h[i] = __builtin_bit_cast(uint32_t, hh);
-        l[i] = __builtin_bit_cast(uint32_t, ll);
+    for (int i = 0; i < 8; ++i) {
+        const float a = v[i] * sc;
+        const _Float16 t = (_Float16)a;
+        h[i] = t;
+        l[i] = (_Float16)(a - (float)t);
     }
-    hi = make_uint4(h[0], h[1], h[2], h[3]);
-    lo = make_uint4(l[0], l[1], l[2], l[3]);
+    hi = __builtin_bit_cast(uint4, h);
+    lo = __builtin_bit_cast(uint4, l);
 }
-DEV float pow2_scale(float mx) {   // 2^(14-e) with mx = m * 2^e, m in [0.5, 1): mx * scale in [2^13, 2^14)
-    int e = 0;
-    if (mx > 0.0f && isfinite(mx)) (void)frexpf(mx, &e);
-    return mx > 0.0f && isfinite(mx) ? ldexpf(1.0f, 14 - e) : 1.0f;
+// 2^(k - e) with |v| = f * 2^e, f in [0.5, 1); 1 for zero, subnormal and non-finite v
+DEV float pow2_scale(float v, int k) {
+    const int e = (int)((__float_as_uint(v) >> 23) & 255u);
+    const int s = 127 + k + 126 - e;   // exponent field of the result
+    return e == 0 || e == 255 ? 1.0f : __uint_as_float((uint32_t)(s < 1 ? 1 : s > 254 ? 254 : s) << 23);
 }
+struct PaRows { uint4 k[4]; uint32_t v[16]; float ks, vs; };   // a chunk's rows as one lane loads them
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(256) void qxp_attn(const float *qr, const int8_t *kc, const int8_t *vc,
-        const float *ks, const float *vs, uint32_t layer, uint32_t ctx, uint32_t p0, uint32_t T, float *ctx_out) {
-    __shared__ uint32_t s_vt[4][128 * 9];   // per wave: V^T of its chunk, rows of 36 bytes (32 positions)
+extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, const int8_t *kc, const int8_t *vc,
+        const float *ks, const float *vs, uint32_t layer, uint32_t ctx, uint32_t p0, uint32_t T, float *ctx_out, float2 *md) {
+    __shared__ uint4 s_q[8 * 2 * 64];           // [k-step][hi, lo][lane] q fragments
+    __shared__ float s_sf[32];                  // per column: 1 / (q scale * sqrt(128)) * log2(e)
     __shared__ float s_ks[4][32], s_vs[4][32];
-    __shared__ float s_acc[2][32][129];
     __shared__ float s_m[2][32], s_den[2][32];
+    __shared__ union { uint32_t vt[4][128 * 9]; float acc[2][32][129]; } u;   // per wave V^T rows of 36 bytes; the merge
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int col = lane & 31, h = lane >> 5;
     const uint32_t kh = blockIdx.x, t0 = blockIdx.y * PA_TT;
     const uint32_t tt = t0 + (col & 3), qh = kh * 8 + (col >> 2);
     const bool tok_ok = tt < T;
     const uint32_t limit = p0 + (tok_ok ? tt : 0);              // last position of the column's token
-    const uint32_t last_t = min(t0 + PA_TT, T) - 1;
-    const uint32_t npos = p0 + last_t + 1;                      // positions the workgroup needs
-    const uint64_t base = (uint64_t)layer * ctx;
-    // q fragments: k-step s holds dims 16s + 8h + j of the column's q row
-    float qv[8][8];
-    bool fin = true;
-    float qmx = 0.0f;
-    const float *qrow = qr + (uint64_t)(tok_ok ? tt : 0) * 4096 + qh * 128 + 8 * h;
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) {
-        const float4 a = *reinterpret_cast<const float4 *>(qrow + 16 * s8);
-        const float4 b = *reinterpret_cast<const float4 *>(qrow + 16 * s8 + 4);
-        qv[s8][0] = a.x; qv[s8][1] = a.y; qv[s8][2] = a.z; qv[s8][3] = a.w;
-        qv[s8][4] = b.x; qv[s8][5] = b.y; qv[s8][6] = b.z; qv[s8][7] = b.w;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { fin = fin && isfinite(qv[s8][j]); qmx = fmaxf(qmx, fabsf(qv[s8][j])); }
-    }
-    fin = fin && (__shfl_xor((int)fin, 32) != 0);
-    qmx = fmaxf(qmx, __shfl_xor(qmx, 32));
-    // a non-finite q makes every score non-finite, which the reference stores as 0
-    const bool qz = !fin || !tok_ok;
-    const float qsc = pow2_scale(qz ? 0.0f : qmx);
-    uint4 qhi[8], qlo[8];
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) {
-        if (qz) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) qv[s8][j] = 0.0f;
-        }
-        split8(qv[s8], qsc, qhi[s8], qlo[s8]);
-    }
-    const float sfac = (float)(1.0 / ((double)qsc * sqrt(128.0)));   // exact power of two over sqrt(128)
-    float m_run = -INFINITY, den = 0.0f;
-    f16x acc[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d) acc[d] = zero16();
+    const uint32_t npos = p0 + min(t0 + PA_TT, T);              // positions the workgroup's tokens need
     const uint32_t nchunk = (npos + 31) / 32;
-    uint32_t *vt = s_vt[wave];
-#pragma unroll 1
-    for (uint32_t ci = wave; ci < nchunk; ci += 4) {
-        const uint32_t pb = ci * 32;
-        // K fragments of position pb + col (clamped inside the workgroup's range)
-        const uint32_t pk = min(pb + col, npos - 1);
-        const int8_t *krow = kc + (base + pk) * 512 + kh * 128 + 8 * h;
-        uint2 kq[8];
+    const uint32_t c_lo = nchunk * blockIdx.z / gridDim.z, c_hi = nchunk * (blockIdx.z + 1) / gridDim.z;
+    const uint64_t base = (uint64_t)layer * ctx;
+    PaRows nx;
+    auto load = [&](uint32_t ci) {   // (rows past the last position read it again)
+        const uint32_t pb = ci * 32, pk = min(pb + col, npos - 1);
+        const uint4 *krow = reinterpret_cast<const uint4 *>(kc + (base + pk) * 512 + kh * 128 + 64 * h);
 #pragma unroll
-        for (int s8 = 0; s8 < 8; ++s8) kq[s8] = *reinterpret_cast<const uint2 *>(krow + 16 * s8);
-        if (lane < 32) {
-            const uint32_t pp = min(pb + lane, npos - 1);
-            s_ks[wave][lane] = ks[base + pp];
-            s_vs[wave][lane] = vs[base + pp];
-        }
-        // V^T of the chunk: lane takes 4 blocks of 4 positions x 4 dims and transposes them
+        for (int i = 0; i < 4; ++i) nx.k[i] = krow[i];
+        nx.ks = ks[base + pk];
+        nx.vs = vs[base + pk];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int bq = lane + 64 * i, pq = bq & 7, dq = bq >> 3;
-            uint32_t w[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t pp = min(pb + 4 * pq + r, npos - 1);
-                w[r] = *reinterpret_cast<const uint32_t *>(vc + (base + pp) * 512 + kh * 128 + 4 * dq);
-            }
+            for (int r = 0; r < 4; ++r)
+                nx.v[4 * i + r] = *reinterpret_cast<const uint32_t *>(vc + (base + min(pb + 4 * pq + r, npos - 1)) * 512 + kh * 128 + 4 * dq);
+        }
+    };
+    if (c_lo + wave < c_hi) load(c_lo + wave);
+    // q: thread takes 16 dims of a column; k-step s of lane half hh holds dims 64 hh + 8 s + j
+    {
+        const int c = tid >> 3, seg = tid & 7;
+        const uint32_t ct = t0 + (c & 3);
+        float v[16], mx = 0.0f;
+        bool fin = true;
+        const float4 *qrow = reinterpret_cast<const float4 *>(qr + (uint64_t)(ct < T ? ct : 0) * 4096 + (kh * 8 + (c >> 2)) * 128 + 16 * seg);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 a = qrow[i];
+            v[4 * i] = a.x; v[4 * i + 1] = a.y; v[4 * i + 2] = a.z; v[4 * i + 3] = a.w;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { fin = fin && isfinite(v[i]); mx = fmaxf(mx, fabsf(v[i])); }
+        mx = fin && ct < T ? mx : INFINITY;
+        mx = fmaxf(mx, dppf<DPP_XOR1>(mx)); mx = fmaxf(mx, dppf<DPP_XOR2>(mx)); mx = fmaxf(mx, dppf<DPP_HALF_MIRROR>(mx));
+        // a non-finite q makes every score non-finite, which the reference stores as 0
+        const bool zero = !(mx < INFINITY);
+        const float sc = pow2_scale(zero ? 0.0f : mx, 14);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = zero ? 0.0f : v[i];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            uint4 hi, lo;
+            split8(v + 8 * i, sc, hi, lo);
+            const int s = 2 * (seg & 3) + i, l = c + 32 * (seg >> 2);
+            s_q[(s * 2 + 0) * 64 + l] = hi;
+            s_q[(s * 2 + 1) * 64 + l] = lo;
+        }
+        if (seg == 0) s_sf[c] = (float)(1.4426950408889634 / ((double)sc * sqrt(128.0)));
+    }
+    __syncthreads();
+    const float sf = s_sf[col];
+    float m = -INFINITY, den = 0.0f, psc = 1.0f, top = 0.0f;   // top: the largest weight * vs so far, at the current m
+    f16x acc[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) acc[d] = zero16();
+    uint32_t *vt = u.vt[wave];
+#pragma unroll 1
+    for (uint32_t ci = c_lo + wave; ci < c_hi; ci += 4) {
+        const uint32_t pb = ci * 32;
+        // this chunk's rows: scales and V^T to LDS (a wave's own), K stays in registers
+        const uint4 kq[4] = {nx.k[0], nx.k[1], nx.k[2], nx.k[3]};
+        const bool big = __ballot(!(fabsf(nx.ks) < 1.1529215e18f)) != 0;   // 2^60: a score could overflow
+        if (lane < 32) {
+            s_ks[wave][lane] = nx.ks;
+            s_vs[wave][lane] = nx.vs;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int bq = lane + 64 * i, pq = bq & 7, dq = bq >> 3;
+            const uint32_t *w = nx.v + 4 * i;
             const uint32_t a0 = perm(w[1], w[0], 0x05010400u), a1 = perm(w[3], w[2], 0x05010400u);
             const uint32_t a2 = perm(w[1], w[0], 0x07030602u), a3 = perm(w[3], w[2], 0x07030602u);
             vt[(4 * dq + 0) * 9 + pq] = perm(a1, a0, 0x05040100u);
@@ -400,65 +442,100 @@ extern "C" __global__ __launch_bounds__(256) void qxp_attn(const float *qr, cons
             vt[(4 * dq + 2) * 9 + pq] = perm(a3, a2, 0x05040100u);
             vt[(4 * dq + 3) * 9 + pq] = perm(a3, a2, 0x07060302u);
         }
+        if (ci + 4 < c_hi) load(ci + 4);
         // scores: S^T = K8 . q
-        f16x sacc = zero16();
+        f16x sh = zero16(), sl = zero16();
 #pragma unroll
-        for (int s8 = 0; s8 < 8; ++s8) {
-            const uint4 kf = i8x8_to_f16(kq[s8]);
-            sacc = mfma(kf, qhi[s8], sacc);
-            sacc = mfma(kf, qlo[s8], sacc);
+        for (int s = 0; s < 8; ++s) {
+            const uint4 kw = kq[s >> 1];
+            const uint4 kf = s & 1 ? i8x8_to_f16(kw.z, kw.w) : i8x8_to_f16(kw.x, kw.y);
+            sh = mfma(kf, s_q[(s * 2 + 0) * 64 + lane], sh);
+            sl = mfma(kf, s_q[(s * 2 + 1) * 64 + lane], sl);
+            if (s & 1) asm volatile("" ::: "memory");   // later q reads stay below: hoisted together they spill
         }
         // register r: position pb + 8(r/4) + 4h + r%4
         float sc[16], cmax = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t pr = 8 * (r >> 2) + 4 * h + (r & 3), p = pb + pr;
-            float v = sacc[r] * (s_ks[wave][pr] * sfac);
-            v = isfinite(v) ? v : 0.0f;
-            sc[r] = p <= limit ? v : -INFINITY;
-            cmax = fmaxf(cmax, sc[r]);
-        }
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
-        const float m_new = fmaxf(m_run, cmax);
-        const float alpha = m_new == -INFINITY ? 1.0f : __expf(m_run - m_new);
-        float pv[16], psum = 0.0f, pmx = 0.0f;
+        for (int q = 0; q < 4; ++q) {
+            const f4x k4 = *reinterpret_cast<const f4x *>(&s_ks[wave][8 * q + 4 * h]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t pr = 8 * (r >> 2) + 4 * h + (r & 3);
-            const float e = sc[r] == -INFINITY ? 0.0f : __expf(sc[r] - m_new);
-            psum += e;
-            pv[r] = e * s_vs[wave][pr];
-            pmx = fmaxf(pmx, pv[r]);
+            for (int r = 0; r < 4; ++r) sc[4 * q + r] = (sh[4 * q + r] + sl[4 * q + r]) * k4[r];
         }
-        pmx = fmaxf(pmx, __shfl_xor(pmx, 32));
-        den = den * alpha + psum;
-        m_run = m_new;
-        const float psc = pow2_scale(pmx), pinv = 1.0f / psc;   // powers of two: exact
+        if (big) {   // non-finite scores are 0 (src/qx_format.c:5137-5139)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = isfinite(sc[r] * sf) ? sc[r] : 0.0f;
+        }
+        const bool tail = pb + 31 > p0 + t0;   // the chunk holds positions past the first token
+        if (tail) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = pb + 8 * (r >> 2) + 4 * h + (r & 3) <= limit ? sc[r] : -INFINITY;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) cmax = fmaxf(cmax, sc[r]);
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32)) * sf;
+        f4x v4[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v4[q] = *reinterpret_cast<const f4x *>(&s_vs[wave][8 * q + 4 * h]);
+        float e[16], pv[16], pmx = 0.0f;
+        auto weigh = [&]() {
+            const float mm = m == -INFINITY ? 0.0f : m;
+            pmx = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                e[r] = exp2_fast(fmaf(sc[r], sf, -mm));
+                pv[r] = e[r] * v4[r >> 2][r & 3];
+                pmx = fmaxf(pmx, pv[r]);
+            }
+            if (tail) {   // (a masked position's V scale does not count, whatever it is)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) pv[r] = sc[r] == -INFINITY ? 0.0f : pv[r];
+            }
+            pmx = fmaxf(pmx, __shfl_xor(pmx, 32));
+        };
+        const bool grow = cmax > m + 8.0f;
+        if (__ballot(grow) == 0) weigh();
+        if (__ballot(grow || pmx * psc > 32768.0f) != 0) {   // (whole wave)
+            const float mn = fmaxf(m, cmax);
+            const float alpha = mn == -INFINITY || m == -INFINITY ? (m == mn ? 1.0f : 0.0f) : exp2_fast(m - mn);
+            m = mn;
+            weigh();
+            top = fmaxf(top * alpha, pmx);
+            const float pn = pow2_scale(top, 10), f = alpha * (pn / psc);   // a power of two times alpha
+            psc = pn;
+            den *= alpha;
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[d][r] *= f;
+        }
+        top = fmaxf(top, pmx);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) den += e[r];
         uint4 phi[2], plo[2];
-        {
-            float a8[8], b8[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) { a8[j] = pv[j]; b8[j] = pv[8 + j]; }
-            split8(a8, psc, phi[0], plo[0]);
-            split8(b8, psc, phi[1], plo[1]);
-        }
-        // context: per 32-dim tile, C[dim][col] = V8^T . pv, merged into the running sums
+        split8(pv, psc, phi[0], plo[0]);
+        split8(pv + 8, psc, phi[1], plo[1]);
+        // context: per 32-dim tile, C[dim][col] += V8^T . pv
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            f16x cacc = zero16();
             const uint32_t *row = vt + (32 * d + col) * 9;
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) {
-                const uint4 vf = i8x8_to_f16(make_uint2(row[4 * s2 + h], row[4 * s2 + 2 + h]));
-                cacc = mfma(vf, phi[s2], cacc);
-                cacc = mfma(vf, plo[s2], cacc);
+                const uint4 vf = i8x8_to_f16(row[4 * s2 + h], row[4 * s2 + 2 + h]);
+                acc[d] = mfma(vf, phi[s2], acc[d]);
+                acc[d] = mfma(vf, plo[s2], acc[d]);
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[d][r] = fmaf(acc[d][r], alpha, cacc[r] * pinv);
         }
+    }
+    {
+        const float inv = 1.0f / psc;   // (a power of two: exact)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[d][r] *= inv;
     }
     // merge the 4 waves' (max, denominator, context) per column: 2+3 into 0+1, then 1 into 0
     den += __shfl_xor(den, 32);
+    __syncthreads();   // the V^T rows are read: their space takes the merge
 #pragma unroll 1
     for (int round = 0; round < 2; ++round) {
         const int nw = round == 0 ? 2 : 1;   // waves [nw, 2nw) hand over to [0, nw)
@@ -467,32 +544,37 @@ extern "C" __global__ __launch_bounds__(256) void qxp_attn(const float *qr, cons
 #pragma unroll
             for (int d = 0; d < 4; ++d)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s_acc[slot][col][32 * d + 8 * (r >> 2) + 4 * h + (r & 3)] = acc[d][r];
-            if (h == 0) { s_m[slot][col] = m_run; s_den[slot][col] = den; }
+                for (int r = 0; r < 16; ++r) u.acc[slot][col][32 * d + 8 * (r >> 2) + 4 * h + (r & 3)] = acc[d][r];
+            if (h == 0) { s_m[slot][col] = m; s_den[slot][col] = den; }
         }
         __syncthreads();
         if (wave < nw) {
             const float mo = s_m[wave][col], dn = s_den[wave][col];
-            const float m_new = fmaxf(m_run, mo);
-            const float fa = m_run == -INFINITY ? 0.0f : __expf(m_run - m_new);
-            const float fb = mo == -INFINITY ? 0.0f : __expf(mo - m_new);
+            const float m_new = fmaxf(m, mo);
+            const float fa = m == -INFINITY ? 0.0f : exp2_fast(m - m_new);
+            const float fb = mo == -INFINITY ? 0.0f : exp2_fast(mo - m_new);
 #pragma unroll
             for (int d = 0; d < 4; ++d)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    acc[d][r] = acc[d][r] * fa + s_acc[wave][col][32 * d + 8 * (r >> 2) + 4 * h + (r & 3)] * fb;
+                    acc[d][r] = acc[d][r] * fa + u.acc[wave][col][32 * d + 8 * (r >> 2) + 4 * h + (r & 3)] * fb;
             den = den * fa + dn * fb;
-            m_run = m_new;
+            m = m_new;
         }
         __syncthreads();
     }
     if (wave == 0 && tok_ok) {
-        const float inv = 1.0f / den;
-        float *out = ctx_out + (uint64_t)tt * 4096 + qh * 128;
+        // one run: the context itself; several: its sums, with their maximum and denominator
+        const float inv = gridDim.z == 1 ? 1.0f / den : 1.0f;
+        const uint64_t row = (uint64_t)blockIdx.z * T + tt;
+        float *out = ctx_out + row * 4096 + qh * 128;
 #pragma unroll
         for (int d = 0; d < 4; ++d)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) out[32 * d + 8 * (r >> 2) + 4 * h + (r & 3)] = acc[d][r] * inv;
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<float4 *>(out + 32 * d + 8 * q + 4 * h) =
+                    make_float4(acc[d][4 * q] * inv, acc[d][4 * q + 1] * inv, acc[d][4 * q + 2] * inv, acc[d][4 * q + 3] * inv);
+        if (h == 0) md[row * 32 + qh] = make_float2(m, den);
     }
 }
 

@@ -5,7 +5,7 @@ import pytest
 
 import qxo
 import qxg
-from helpers import REL_L2, rel_l2
+from helpers import REL_L2, rel_l2, seeded_kv
 
 pytestmark = pytest.mark.gpu
 
@@ -67,4 +67,32 @@ def test_dense_row_tiles_and_parts(ctx, models, mix, layer, n):
         assert rel_l2(fi[t], x[t] + a) <= REL_L2, (t, rel_l2(fi[t], x[t] + a))
         assert np.abs(okv.k[layer, t].astype(int) - rk.astype(int)).max() <= 1, t
         assert np.abs(okv.v[layer, t].astype(int) - rv.astype(int)).max() <= 1, t
+    om.close()
+
+
+@pytest.mark.parametrize("n,p0,odd", [(1, 0, 0), (1, 31, 0), (3, 127, 0), (5, 128, 0), (4, 290, 0), (13, 260, 1), (66, 70, 1)])
+def test_attention_runs_and_scales(ctx, models, n, p0, odd):
+    """Attention over one and several runs of positions (several from 256 positions on while the
+    tokens are few), chunks that hold only masked positions for some token, and, with odd, V
+    scales 1e6 apart inside a chunk and between chunks and a NaN K scale (the reference's scores
+    of that position are 0): every row against the oracle over the same cache rows."""
+    p = models / "m0.qxf"
+    ctx.load(p)
+    ctx.kv_create(1, 400)
+    okv = qxo.KV(1, 400)
+    if p0:
+        k, v, ks, vs = seeded_kv(300 + p0, p0)
+        if odd:
+            vs[::7] *= 1e-6
+            vs[40:44] *= 1e3
+            ks[11] = np.nan
+        ctx.kv_write(0, 0, k, v, ks, vs)
+        okv.k[0, :p0], okv.v[0, :p0], okv.ks[0, :p0], okv.vs[0, :p0] = k, v, ks, vs
+    x = np.random.default_rng(31 + n).standard_normal((n, 2048)).astype(np.float32)
+    fi, _, _ = ctx.prefill_layer(0, p0, x)
+    okv.k[0, p0:p0 + n], okv.v[0, p0:p0 + n], okv.ks[0, p0:p0 + n], okv.vs[0, p0:p0 + n] = ctx.kv_read(0, p0, n)
+    om = qxo.Model(p)
+    for t in range(n):
+        a = qxo.attention_layer_given_row(om, 0, p0 + t, okv, x[t])[0]
+        assert rel_l2(fi[t], x[t] + a) <= REL_L2, (t, rel_l2(fi[t], x[t] + a))
     om.close()
