@@ -23,6 +23,9 @@ __global__ void qxk_stage_ctx(const float *, uint32_t, float *);
 __global__ void qxk_router(const float *, const float *, const float *, uint32_t, double *);
 __global__ void qxk_topk(const float *, uint32_t, uint32_t, float *, uint32_t *, float *, uint32_t *, uint32_t *,
                          DevState *);
+__global__ void qxk_begin(DevState *, uint32_t, uint32_t, uint32_t, uint32_t, const double *, const double *, const uint4 *, uint4 *,
+                          uint32_t);
+__global__ void qxk_gather(QxGather);
 __global__ void qxk_advance(DevState *, const double *, const double *);
 __global__ void qxk_topk_merge(const float *, const uint32_t *, uint32_t, uint32_t, float *, uint32_t *, uint32_t *,
                                DevState *);
@@ -164,6 +167,7 @@ struct qxg_ctx {
     uint32_t next_ep = 0;            // epoch base of the next persistent launch
     bool coop_held = false;          // another process holds the GPU's cooperative launches: launch plainly
     uint32_t *abort = nullptr;
+    uint8_t *io = nullptr;           // pinned host memory: IO_IN bytes of a call's input, then IO_OUT of its outputs
     uint8_t *scratch = nullptr;      // device address of this GPU's static workspace (qxg_dequant_blocks_static)
     // one decode step (embed .. head, top-1, step advance) recorded once and replayed
     hipGraph_t graph = nullptr;
@@ -312,14 +316,17 @@ void build_tables(std::vector<uint4> &g2, std::vector<uint2> &g3, std::vector<ui
     }
 }
 
-void write_state(qxg_ctx *c, uint32_t pos0, uint32_t step, uint32_t n_prompt, uint32_t force_head) {
-    DevState h{};
-    h.pos0 = pos0; h.step = step; h.n_prompt = n_prompt; h.force_head = force_head;
-    (void)hipMemcpyAsync(c->st, &h, offsetof(DevState, moe_ids), hipMemcpyHostToDevice, c->s);
-    // the position's RoPE row, read by the attention kernel without waiting for the position
-    const uint64_t p = std::min<uint64_t>((uint64_t)pos0 + step, QXG_MAX_CTX - 1);
-    (void)hipMemcpyAsync(c->st->rope_c, c->T.rope_cos + p * 64, 64 * sizeof(double), hipMemcpyDeviceToDevice, c->s);
-    (void)hipMemcpyAsync(c->st->rope_s, c->T.rope_sin + p * 64, 64 * sizeof(double), hipMemcpyDeviceToDevice, c->s);
+// Writes the step state and the position's RoPE row; with in, also `bytes` of input (at most
+// IO_IN) to dst, through the context's pinned buffer.  The buffer is free for the next call: every
+// call ends by waiting for its stream.
+constexpr uint64_t IO_IN = 512 << 10, IO_OUT = 2 << 20;
+void write_state(qxg_ctx *c, uint32_t pos0, uint32_t step, uint32_t n_prompt, uint32_t force_head, const void *in = nullptr,
+                 void *dst = nullptr, uint64_t bytes = 0) {
+    if (in) memcpy(c->io, in, bytes);
+    const uint32_t n4 = in ? (uint32_t)((bytes + 15) / 16) : 0u;
+    hipLaunchKernelGGL(qxk_begin, dim3(std::max<uint32_t>(1, std::min<uint32_t>(128, n4 / 512))), dim3(256), 0, c->s, c->st, pos0,
+                       step, n_prompt, force_head, (const double *)c->T.rope_cos, (const double *)c->T.rope_sin,
+                       (const uint4 *)c->io, (uint4 *)dst, n4);
 }
 
 const QTensor *find(qxg_ctx *c, const std::string &name) {
@@ -636,6 +643,54 @@ bool finish(qxg_ctx *c, char *err, uint64_t n) {
     return !c->abort || check_abort(c, err, n);
 }
 
+// Waits for the call's work and reads its outputs (and the step state, if asked for).  The
+// outputs, the state and the abort flag leave the device in one launch into the pinned buffer
+// and the stream is waited for once; a wait and a pageable copy for each took 10 us apiece.
+// Outputs beyond the buffer or QX_GATHER - 2 are copied one by one.
+struct HostOut { void *dst; const void *src; uint64_t bytes; };   // bytes: a multiple of 4; dst null: not wanted
+bool finish_read(qxg_ctx *c, std::initializer_list<HostOut> outs, DevState *state, char *err, uint64_t n) {
+    uint64_t total = 0;
+    uint32_t count = 0;
+    for (const HostOut &o : outs)
+        if (o.dst && o.bytes) { total += (o.bytes + 15) & ~15ull; ++count; }
+    const uint64_t st_bytes = offsetof(DevState, rope_c);
+    if (total + st_bytes + 64 > IO_OUT || count > QX_GATHER - 2) {
+        if (!finish(c, err, n)) return false;
+        for (const HostOut &o : outs)
+            if (o.dst && o.bytes && !hip_ok(hipMemcpy(o.dst, o.src, o.bytes, hipMemcpyDeviceToHost), err, n, "read")) return false;
+        return !state || hip_ok(hipMemcpy(state, c->st, sizeof(*state), hipMemcpyDeviceToHost), err, n, "state read");
+    }
+    QxGather g{};
+    uint32_t k = 0, most = 0;
+    uint8_t *at = c->io + IO_IN;
+    auto add = [&](const void *src, uint64_t bytes) {
+        g.src[k] = (const uint32_t *)src;
+        g.dst[k] = (uint32_t *)at;
+        g.words[k] = (uint32_t)(bytes / 4);
+        most = std::max(most, g.words[k++]);
+        uint8_t *p = at;
+        at += (bytes + 15) & ~15ull;
+        return p;
+    };
+    const uint8_t *st = add(c->st, st_bytes), *ab = c->abort ? add(c->abort, 4) : nullptr;
+    const uint8_t *first = at;
+    for (const HostOut &o : outs)
+        if (o.dst && o.bytes) (void)add(o.src, o.bytes);
+    hipLaunchKernelGGL(qxk_gather, dim3(std::max<uint32_t>(1, std::min<uint32_t>(128, most / 2048)), k), dim3(256), 0, c->s, g);
+    if (!hip_ok(hipGetLastError(), err, n, "launch") || !hip_ok(hipStreamSynchronize(c->s), err, n, "stream")) return false;
+    DevState h;
+    memcpy(&h, st, st_bytes);
+    if (c->q8 && h.q8_fault && !check_q8(c, err, n)) return false;
+    if (ab && *(const uint32_t *)ab && !check_abort(c, err, n)) return false;
+    if (state) memcpy(state, &h, st_bytes);
+    for (const HostOut &o : outs)
+        if (o.dst && o.bytes) {
+            memcpy(o.dst, first, o.bytes);
+            first += (o.bytes + 15) & ~15ull;
+        }
+    return true;
+}
+
 bool read_state(qxg_ctx *c, DevState &h, char *err, uint64_t n) {
     return hip_ok(hipMemcpyAsync(&h, c->st, sizeof(h), hipMemcpyDeviceToHost, c->s), err, n, "state read") &&
            hip_ok(hipStreamSynchronize(c->s), err, n, "stream");
@@ -895,16 +950,13 @@ int prefill_steps(qxg_ctx *c, const uint32_t *tokens, uint32_t n, uint32_t posit
 // Waits for the prefill's work and reads the head's outputs of the last token.
 int prefill_finish(qxg_ctx *c, int run_head, float *logits, uint32_t top_n, uint32_t *top_ids, double *top_logits,
                    float *elapsed_ms, char *err, uint64_t err_len) {
-    if (!finish(c, err, err_len)) return 0;
-    if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, c->e0, c->e1);
-    if (!run_head) return 1;
     DevState h;
-    if (!read_state(c, h, err, err_len)) return 0;
-    if (logits && !hip_ok(hipMemcpy(logits, c->logits, (uint64_t)c->vocab * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
     float tv[QXG_MAX_TOPN];
     uint32_t ti[QXG_MAX_TOPN];
-    if (!hip_ok(hipMemcpy(tv, c->top_v, top_n * 4, hipMemcpyDeviceToHost), err, err_len, "read") ||
-        !hip_ok(hipMemcpy(ti, c->top_i, top_n * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+    if (!finish_read(c, {{run_head ? logits : nullptr, c->logits, (uint64_t)c->vocab * 4}, {run_head ? tv : nullptr, c->top_v, top_n * 4},
+                         {run_head ? ti : nullptr, c->top_i, top_n * 4}}, &h, err, err_len)) return 0;
+    if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, c->e0, c->e1);
+    if (!run_head) return 1;
     for (uint32_t i = 0; i < top_n; ++i) {
         if (top_ids) top_ids[i] = ti[i];
         if (top_logits) top_logits[i] = (double)tv[i];
@@ -990,7 +1042,8 @@ int qxg_open(int device, qxg_ctx **out, char *err, uint64_t err_len) {
         const char *ev = getenv("QXG_EAGER");
         c->eager = ev && ev[0] == '1';
     }
-    bool ok = hip_ok(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking), err, err_len, "stream");
+    bool ok = hip_ok(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking), err, err_len, "stream") &&
+              hip_ok(hipHostMalloc((void **)&c->io, IO_IN + IO_OUT, hipHostMallocDefault), err, err_len, "pinned buffer");
     std::vector<uint4> g2, g2s;
     std::vector<uint2> g3, sel, g3s, sel8;
     build_tables(g2, g3, sel);
@@ -1058,6 +1111,7 @@ void qxg_close(qxg_ctx *c) {
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : c->arenas) (void)hipFree(p);
     if (c->dense) (void)hipFree(c->dense);
+    if (c->io) (void)hipHostFree(c->io);
     for (void *p : c->pf.all) (void)hipFree(p);
     for (void *p : c->sg.all) (void)hipFree(p);
     for (hipEvent_t e : c->kt.ev) (void)hipEventDestroy(e);
@@ -1262,8 +1316,8 @@ int qxg_decode_token(qxg_ctx *c, uint32_t token, uint32_t position, int run_head
     if (top_n == 0) top_n = 1;
     if (top_n > QXG_MAX_TOPN) top_n = QXG_MAX_TOPN;
     (void)hipSetDevice(c->device);
-    (void)hipMemcpyAsync(c->tokens, &token, 4, hipMemcpyHostToDevice, c->s);
-    write_state(c, position, 0, run_head ? 1 : 2, 0);
+    const uint32_t word[4] = {token};   // (tokens holds at least 16 bytes)
+    write_state(c, position, 0, run_head ? 1 : 2, 0, word, c->tokens, 16);
     if (persistent(c) && c->layers) {
         // one step of the persistent decode (its head writes every logit), then the top-N
         // of those logits by the per-phase selection kernels
@@ -1289,17 +1343,14 @@ int qxg_decode_token(qxg_ctx *c, uint32_t token, uint32_t position, int run_head
         }
         if (run_head) launch_head(c, top_n, c->norm);
     }
-    if (!finish(c, err, err_len)) return 0;
-    if (residual_out && !hip_ok(hipMemcpy(residual_out, c->x, 2048 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (layer_out && !hip_ok(hipMemcpy(layer_out, c->layer_dump, 2048ull * 4 * c->layers, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (!run_head) return 1;
     DevState h;
-    if (!read_state(c, h, err, err_len)) return 0;
-    if (logits && !hip_ok(hipMemcpy(logits, c->logits, (uint64_t)c->vocab * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
     float tv[QXG_MAX_TOPN];
     uint32_t ti[QXG_MAX_TOPN];
-    if (!hip_ok(hipMemcpy(tv, c->top_v, top_n * 4, hipMemcpyDeviceToHost), err, err_len, "read") ||
-        !hip_ok(hipMemcpy(ti, c->top_i, top_n * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+    if (!finish_read(c, {{residual_out, c->x, 2048 * 4}, {layer_out, c->layer_dump, 2048ull * 4 * c->layers},
+                         {run_head ? logits : nullptr, c->logits, (uint64_t)c->vocab * 4},
+                         {run_head ? tv : nullptr, c->top_v, top_n * 4}, {run_head ? ti : nullptr, c->top_i, top_n * 4}},
+                     &h, err, err_len)) return 0;
+    if (!run_head) return 1;
     for (uint32_t i = 0; i < top_n; ++i) {
         if (top_ids) top_ids[i] = ti[i];
         if (top_logits) top_logits[i] = (double)tv[i];
@@ -1325,11 +1376,9 @@ int qxg_generate(qxg_ctx *c, const uint32_t *prompt, uint32_t n_prompt, uint32_t
         (void)hipEventRecord(c->e0, c->s);
         if (!launch_decode(c, (uint32_t)steps, n_prompt, pos0, false, DecodeDumps(), err, err_len)) return 0;
         (void)hipEventRecord(c->e1, c->s);
-        if (!finish(c, err, err_len)) return 0;
-        if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, c->e0, c->e1);
         DevState h;
-        if (!read_state(c, h, err, err_len)) return 0;
-        if (tokens_out && !hip_ok(hipMemcpy(tokens_out, c->tokens + n_prompt, (uint64_t)n_gen * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+        if (!finish_read(c, {{tokens_out, c->tokens + n_prompt, (uint64_t)n_gen * 4}}, &h, err, err_len)) return 0;
+        if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, c->e0, c->e1);
         if (h.nonfinite) { write_state(c, 0, 0, 0, 0); set_err(err, err_len, "non-finite final logit"); return 0; }
         return 1;
     }
@@ -1373,11 +1422,9 @@ int qxg_generate(qxg_ctx *c, const uint32_t *prompt, uint32_t n_prompt, uint32_t
         }
     }
     (void)hipEventRecord(c->e1, c->s);
-    if (!finish(c, err, err_len)) return 0;
-    if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, c->e0, c->e1);
     DevState h;
-    if (!read_state(c, h, err, err_len)) return 0;
-    if (tokens_out && !hip_ok(hipMemcpy(tokens_out, c->tokens + n_prompt, (uint64_t)n_gen * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+    if (!finish_read(c, {{tokens_out, c->tokens + n_prompt, (uint64_t)n_gen * 4}}, &h, err, err_len)) return 0;
+    if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, c->e0, c->e1);
     if (h.nonfinite) { write_state(c, 0, 0, 0, 0); set_err(err, err_len, "non-finite final logit"); return 0; }
     return 1;
 }
@@ -1484,11 +1531,10 @@ int qxg_embed_token(qxg_ctx *c, uint32_t token, float *x_out, char *err, uint64_
     if (!c->emb) { set_err(err, err_len, "token_embd.weight not bound"); return 0; }
     if (token >= c->vocab || !x_out) { set_err(err, err_len, "token id out of range"); return 0; }
     (void)hipSetDevice(c->device);
-    (void)hipMemcpyAsync(c->tokens, &token, 4, hipMemcpyHostToDevice, c->s);
-    write_state(c, 0, 0, 1, 1);
+    const uint32_t word[4] = {token};
+    write_state(c, 0, 0, 1, 1, word, c->tokens, 16);
     hipLaunchKernelGGL(qxk_embed, dim3(1), dim3(256), 0, c->s, c->emb, c->emb_row, c->tokens, c->st, c->x);
-    if (!finish(c, err, err_len)) return 0;
-    return hip_ok(hipMemcpy(x_out, c->x, 2048 * 4, hipMemcpyDeviceToHost), err, err_len, "read");
+    return finish_read(c, {{x_out, c->x, 2048 * 4}}, nullptr, err, err_len);
 }
 
 namespace {
@@ -1517,15 +1563,10 @@ int qxg_attention_layer_ex(qxg_ctx *c, uint32_t layer, uint32_t position, const 
     if (!x_in || layer >= c->layers || layer >= c->kv_layers || position >= c->kv_ctx) { set_err(err, err_len, "invalid attention layer argument"); return 0; }
     (void)hipSetDevice(c->device);
     if (head_weight_sums && !stage_buffers(c, err, err_len)) return 0;
-    (void)hipMemcpyAsync(c->x, x_in, 2048 * 4, hipMemcpyHostToDevice, c->s);
-    write_state(c, position, 0, 1, 1);
+    write_state(c, position, 0, 1, 1, x_in, c->x, 2048 * 4);
     launch_attention(c, layer, c->x, c->attn, c->vcur, head_weight_sums ? c->sg.wsum : nullptr);
-    if (!finish(c, err, err_len)) return 0;
-    if (head_weight_sums && !hip_ok(hipMemcpy(head_weight_sums, c->sg.wsum, 32 * 8, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (attn_out && !hip_ok(hipMemcpy(attn_out, c->attn, 2048 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (kqv_out && !hip_ok(hipMemcpy(kqv_out, c->ctxv, 4096 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (vcur_out && !hip_ok(hipMemcpy(vcur_out, c->vcur, 512 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    return 1;
+    return finish_read(c, {{head_weight_sums, c->sg.wsum, 32 * 8}, {attn_out, c->attn, 2048 * 4}, {kqv_out, c->ctxv, 4096 * 4},
+                           {vcur_out, c->vcur, 512 * 4}}, nullptr, err, err_len);
 }
 
 int qxg_moe_layer(qxg_ctx *c, uint32_t layer, const float *ffn_inp, float *layer_out, float *moe_out, uint32_t ids[8],
@@ -1533,14 +1574,10 @@ int qxg_moe_layer(qxg_ctx *c, uint32_t layer, const float *ffn_inp, float *layer
     if (!check_ready(c, false, err, err_len)) return 0;
     if (!ffn_inp || layer >= c->layers) { set_err(err, err_len, "invalid MoE layer argument"); return 0; }
     (void)hipSetDevice(c->device);
-    (void)hipMemcpyAsync(c->x, ffn_inp, 2048 * 4, hipMemcpyHostToDevice, c->s);
-    write_state(c, 0, 0, 1, 1);
+    write_state(c, 0, 0, 1, 1, ffn_inp, c->x, 2048 * 4);
     launch_moe(c, layer, c->x, c->moe);
-    if (!finish(c, err, err_len)) return 0;
     DevState h;
-    if (!read_state(c, h, err, err_len)) return 0;
-    if (layer_out && !hip_ok(hipMemcpy(layer_out, c->x, 2048 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (moe_out && !hip_ok(hipMemcpy(moe_out, c->moe, 2048 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+    if (!finish_read(c, {{layer_out, c->x, 2048 * 4}, {moe_out, c->moe, 2048 * 4}}, &h, err, err_len)) return 0;
     for (int r = 0; r < 8; ++r) {
         if (ids) ids[r] = h.moe_ids[r];
         if (weights) weights[r] = h.moe_w[r];
@@ -1628,18 +1665,13 @@ int qxg_final_head(qxg_ctx *c, const float *residual, float *norm_out, float *lo
     if (top_n == 0) top_n = 1;
     if (top_n > QXG_MAX_TOPN) top_n = QXG_MAX_TOPN;
     (void)hipSetDevice(c->device);
-    (void)hipMemcpyAsync(c->x, residual, 2048 * 4, hipMemcpyHostToDevice, c->s);
-    write_state(c, 0, 0, 1, 1);
+    write_state(c, 0, 0, 1, 1, residual, c->x, 2048 * 4);
     launch_head(c, top_n, c->norm);
-    if (!finish(c, err, err_len)) return 0;
     DevState h;
-    if (!read_state(c, h, err, err_len)) return 0;
-    if (norm_out && !hip_ok(hipMemcpy(norm_out, c->norm, 2048 * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (logits && !hip_ok(hipMemcpy(logits, c->logits, (uint64_t)c->vocab * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
     float tv[QXG_MAX_TOPN];
     uint32_t ti[QXG_MAX_TOPN];
-    if (!hip_ok(hipMemcpy(tv, c->top_v, top_n * 4, hipMemcpyDeviceToHost), err, err_len, "read") ||
-        !hip_ok(hipMemcpy(ti, c->top_i, top_n * 4, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+    if (!finish_read(c, {{norm_out, c->norm, 2048 * 4}, {logits, c->logits, (uint64_t)c->vocab * 4}, {tv, c->top_v, top_n * 4},
+                         {ti, c->top_i, top_n * 4}}, &h, err, err_len)) return 0;
     for (uint32_t i = 0; i < top_n; ++i) {
         if (top_ids) top_ids[i] = ti[i];
         if (top_logits) top_logits[i] = (double)tv[i];
@@ -1967,12 +1999,12 @@ int qxg_prefill_layer(qxg_ctx *c, uint32_t layer, uint32_t n, uint32_t position0
     }
     if (!prefill_ready(c, err, err_len)) return 0;
     auto &B = c->pf;
-    if (!hip_ok(hipMemcpyAsync(B.X, x_in, 2048ull * 4 * n, hipMemcpyHostToDevice, c->s), err, err_len, "upload")) return 0;
+    const uint64_t bytes = 2048ull * 4 * n;
+    if (bytes <= IO_IN)   // (few rows: one launch each way; many go faster as the runtime's own copies)
+        write_state(c, position0, 0, 1, 1, x_in, B.X, bytes);
+    else if (!hip_ok(hipMemcpyAsync(B.X, x_in, bytes, hipMemcpyHostToDevice, c->s), err, err_len, "upload")) return 0;
     prefill_layer(c, layer, n, position0, true, true, moe_out ? B.dump : nullptr);
-    if (!finish(c, err, err_len)) return 0;
-    if (ffn_inp_out && !hip_ok(hipMemcpy(ffn_inp_out, B.X1, 2048ull * 4 * n, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (moe_out && !hip_ok(hipMemcpy(moe_out, B.dump, 2048ull * 4 * n, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
-    if (x_out && !hip_ok(hipMemcpy(x_out, B.X, 2048ull * 4 * n, hipMemcpyDeviceToHost), err, err_len, "read")) return 0;
+    if (!finish_read(c, {{ffn_inp_out, B.X1, bytes}, {moe_out, B.dump, bytes}, {x_out, B.X, bytes}}, nullptr, err, err_len)) return 0;
     return 1;
 }
 

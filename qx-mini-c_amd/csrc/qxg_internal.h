@@ -59,6 +59,14 @@ struct DevState {
     double rope_s[64];      // with the position by the host and by qxk_advance
 };
 
+// Arguments of qxk_gather: up to QX_GATHER outputs
+#define QX_GATHER 8
+struct QxGather {
+    const uint32_t *src[QX_GATHER];
+    uint32_t *dst[QX_GATHER];
+    uint32_t words[QX_GATHER];
+};
+
 // q8_k_compat failures, reported as the reference reports them (src/qx_format.c:3906, 4771)
 #define QXG_Q8_NONFINITE_INPUT 1u    // "Q8_K activation contains NaN or Inf"
 #define QXG_Q8_NONFINITE_EXPERT 2u   // "non-finite packed expert Q8_K output"

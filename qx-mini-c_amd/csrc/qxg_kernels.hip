@@ -839,6 +839,37 @@ extern "C" __global__ __launch_bounds__(256) void qxk_topk_merge(const float *ca
     if (threadIdx.x == 0 && st->step + 1 >= st->n_prompt) tokens[st->step + 1] = top_i[0];
 }
 
+// Starts a call: the host-written prefix of the state, the position's RoPE row, and, with src
+// (host memory the device can read), n4 16-byte words of the call's input to dst.  One launch
+// in place of a copy each.
+extern "C" __global__ __launch_bounds__(256) void qxk_begin(DevState *st, uint32_t pos0, uint32_t step, uint32_t n_prompt,
+        uint32_t force_head, const double *rope_cos, const double *rope_sin, const uint4 *src, uint4 *dst, uint32_t n4) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n4; i += gridDim.x * 256) dst[i] = src[i];
+    if (blockIdx.x) return;
+    const uint32_t p = min(pos0 + step, (uint32_t)QXG_MAX_CTX - 1);
+    const int i = threadIdx.x;
+    if (i < 64) {
+        st->rope_c[i] = rope_cos[p * 64 + i];
+        st->rope_s[i] = rope_sin[p * 64 + i];
+    }
+    if (i == 0) {
+        st->pos0 = pos0; st->step = step; st->n_prompt = n_prompt; st->nonfinite = 0;
+        st->spare = 0; st->spare2 = 0; st->force_head = force_head; st->pad = 0;
+    }
+}
+
+// Ends a call: copies its outputs (4-byte words) to host memory the device can write, one
+// launch for all of them; blockIdx.y is the output.
+extern "C" __global__ __launch_bounds__(256) void qxk_gather(QxGather g) {
+    const uint32_t *src = g.src[blockIdx.y];
+    uint32_t *dst = g.dst[blockIdx.y];
+    const uint32_t n = g.words[blockIdx.y], n4 = n / 4;
+    const bool wide = ((uintptr_t)src & 15) == 0;   // (outputs inside larger buffers may start anywhere)
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < (wide ? n4 : 0u); i += gridDim.x * 256)
+        reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    for (uint32_t i = (wide ? 4 * n4 : 0u) + blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
 // Next step: step + 1, and the RoPE row of its position (64 threads)
 extern "C" __global__ void qxk_advance(DevState *st, const double *rope_cos, const double *rope_sin) {
     const uint32_t step = st->step + 1, p = min(st->pos0 + step, (uint32_t)QXG_MAX_CTX - 1);
