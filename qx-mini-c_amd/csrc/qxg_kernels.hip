@@ -761,82 +761,85 @@ __global__ __launch_bounds__(256) void qxk_head(const uint32_t *dig, const uint8
 
 // top-N (N <= 32) over logits by (value desc, index asc): each block of qxk_topk
 // reduces a slice to N candidates, qxk_topk_merge (one block, the next launch) merges
-// them and writes tokens[step+1] = argmax on generate steps.  Round r picks the best element strictly below pick r-1 in that
-// total order, so equal values are taken in index order.
+// them and writes tokens[step+1] = argmax on generate steps.  A value and its index are one
+// 64-bit key, unique, 0 for none (NaN).  Each wave keeps its keys in registers and takes the
+// largest N times (lane r keeps the r-th), the block's four lists are taken together in wave
+// 0: about 0.2 us a round and one barrier.  (Rounds of the whole block, each scanning the slice
+// again with two barriers: 15 + 15 us for N = 8, now 5 + 5.)
 namespace {
-DEV bool better(float v, uint32_t i, float bv, uint32_t bi) { return v > bv || (v == bv && i < bi); }
-
-DEV void block_best(float &v, uint32_t &i, float *sv, uint32_t *si) {
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(v, o);
-        const uint32_t oi = __shfl_xor(i, o);
-        if (better(ov, oi, v, i)) { v = ov; i = oi; }
-    }
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = v; si[threadIdx.x >> 6] = i; }
-    __syncthreads();
-    v = sv[0]; i = si[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
-        if (better(sv[w], si[w], v, i)) { v = sv[w]; i = si[w]; }
+DEV uint64_t topn_key(float v, uint32_t i) {
+    if (v != v) return 0;
+    const uint32_t b = __float_as_uint(v + 0.0f);   // (-0 as +0: equal values go by index)
+    return ((uint64_t)((b >> 31) ? ~b : (b | 0x80000000u)) << 32) | (0xffffffffu - i);
 }
-
-DEV void select_topn(const float *vals, const uint32_t *idx, uint32_t n, uint32_t topn, float *ov, uint32_t *oi,
-                     float *sv, uint32_t *si) {
-    float pv = INFINITY;
-    uint32_t pi = 0;
-    bool first = true;
-    for (uint32_t r = 0; r < topn; ++r) {
-        float bv = -INFINITY;
-        uint32_t bi = 0xffffffffu;
-        for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
-            const float v = vals[t];
-            const uint32_t i = idx ? idx[t] : t;
-            if (i == 0xffffffffu) continue;
-            const bool below = first || better(pv, pi, v, i);
-            if (below && better(v, i, bv, bi)) { bv = v; bi = i; }
-        }
-        block_best(bv, bi, sv, si);
-        if (threadIdx.x == 0) { ov[r] = bv; oi[r] = bi; }
-        pv = bv; pi = bi; first = false;
+DEV void topn_out(uint64_t k, float &v, uint32_t &i) {
+    const uint32_t b = (uint32_t)(k >> 32);
+    v = k ? __uint_as_float((b >> 31) ? (b & 0x7fffffffu) : ~b) : -INFINITY;
+    i = k ? 0xffffffffu - (uint32_t)k : 0xffffffffu;
+}
+// the wave's n largest of its lanes' R keys: lane r (< n <= 32) returns the r-th
+template <int R>
+DEV uint64_t wave_topn(uint64_t (&k)[R], uint32_t n) {
+    const int lane = threadIdx.x & 63;
+    uint64_t mine = 0;
+    for (uint32_t r = 0; r < n; ++r) {
+        uint64_t m = k[0];
+#pragma unroll
+        for (int i = 1; i < R; ++i) m = umax64(m, k[i]);
+        m = wave_max_u64(m);
+#pragma unroll
+        for (int i = 0; i < R; ++i) k[i] = k[i] == m ? 0 : k[i];
+        if (lane == (int)r) mine = m;
     }
+    return mine;
+}
+// the block's n largest: fetch(t) is the key of element t < count; wave 0's lane r returns the
+// r-th.  256 threads; s_k holds 4 * 32 keys.
+template <typename F>
+DEV uint64_t block_topn(F fetch, uint32_t count, uint32_t n, uint64_t *s_k) {
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    uint64_t mine = 0;
+    for (uint32_t t0 = 0; t0 < count; t0 += 8 * 256) {   // (once, for up to 2048 elements)
+        uint64_t k[9];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t t = t0 + 256 * i + threadIdx.x;
+            k[i] = t < count ? fetch(t) : 0;
+        }
+        k[8] = mine;
+        mine = wave_topn<9>(k, n);
+    }
+    if (lane < 32) s_k[32 * wave + lane] = mine;
+    __syncthreads();
+    uint64_t k[2] = {s_k[lane], s_k[64 + lane]};
+    return wave == 0 ? wave_topn<2>(k, n) : 0;
 }
 }  // namespace
 
 extern "C" __global__ __launch_bounds__(256) void qxk_topk(const float *logits, uint32_t vocab, uint32_t topn,
         float *cand_v, uint32_t *cand_i, float *top_v, uint32_t *top_i, uint32_t *tokens, DevState *st) {
     if (prompt_step(st)) return;
-    __shared__ float sv[4];
-    __shared__ uint32_t si[4];
+    __shared__ uint64_t s_k[128];
     const uint32_t chunk = (vocab + gridDim.x - 1) / gridDim.x;
     const uint32_t s0 = blockIdx.x * chunk, s1 = min(vocab, s0 + chunk);
-    const uint32_t n = s1 > s0 ? s1 - s0 : 0;
-    // local candidates (indices are global)
-    {
-        float pv = INFINITY;
-        uint32_t pi = 0;
-        for (uint32_t r = 0; r < topn; ++r) {
-            float bv = -INFINITY;
-            uint32_t bi = 0xffffffffu;
-            for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
-                const float v = logits[s0 + t];
-                const uint32_t i = s0 + t;
-                if ((r == 0 || better(pv, pi, v, i)) && better(v, i, bv, bi)) { bv = v; bi = i; }
-            }
-            block_best(bv, bi, sv, si);
-            if (threadIdx.x == 0) { cand_v[blockIdx.x * topn + r] = bv; cand_i[blockIdx.x * topn + r] = bi; }
-            pv = bv; pi = bi;
-        }
-    }
+    const uint64_t k = block_topn([&](uint32_t t) { return topn_key(logits[s0 + t], s0 + t); }, s1 > s0 ? s1 - s0 : 0, topn, s_k);
+    if (threadIdx.x < topn) topn_out(k, cand_v[blockIdx.x * topn + threadIdx.x], cand_i[blockIdx.x * topn + threadIdx.x]);
 }
 // the merge of qxk_topk's per-block candidates (one block; the kernel boundary makes
 // them visible without fences), and tokens[step+1] = argmax on generate steps
 extern "C" __global__ __launch_bounds__(256) void qxk_topk_merge(const float *cand_v, const uint32_t *cand_i,
         uint32_t blocks, uint32_t topn, float *top_v, uint32_t *top_i, uint32_t *tokens, DevState *st) {
     if (prompt_step(st)) return;
-    __shared__ float sv[4];
-    __shared__ uint32_t si[4];
-    select_topn(cand_v, cand_i, blocks * topn, topn, top_v, top_i, sv, si);
-    if (threadIdx.x == 0 && st->step + 1 >= st->n_prompt) tokens[st->step + 1] = top_i[0];
+    __shared__ uint64_t s_k[128];
+    const uint64_t k = block_topn([&](uint32_t t) { return cand_i[t] == 0xffffffffu ? 0 : topn_key(cand_v[t], cand_i[t]); },
+                                  blocks * topn, topn, s_k);
+    if (threadIdx.x < topn) topn_out(k, top_v[threadIdx.x], top_i[threadIdx.x]);
+    if (threadIdx.x == 0 && st->step + 1 >= st->n_prompt) {
+        float v;
+        uint32_t i;
+        topn_out(k, v, i);
+        tokens[st->step + 1] = i;
+    }
 }
 
 // Starts a call: the host-written prefix of the state, the position's RoPE row, and, with src
