@@ -765,7 +765,7 @@ __global__ __launch_bounds__(256) void qxk_head(const uint32_t *dig, const uint8
 // 64-bit key, unique, 0 for none (NaN).  Each wave keeps its keys in registers and takes the
 // largest N times (lane r keeps the r-th), the block's four lists are taken together in wave
 // 0: about 0.2 us a round and one barrier.  (Rounds of the whole block, each scanning the slice
-// again with two barriers: 15 + 15 us for N = 8, now 5 + 5.)
+// again with two barriers: 15 + 15 us for N = 8, now 8 + 8.)
 namespace {
 DEV uint64_t topn_key(float v, uint32_t i) {
     if (v != v) return 0;
