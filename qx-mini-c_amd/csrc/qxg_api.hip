@@ -843,7 +843,7 @@ bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
               alloc((void **)&B.QR, T * 4096 * 4) && alloc((void **)&B.CTX, PF_CTX_ROWS * 4096 * 4) && alloc((void **)&B.md, PF_CTX_ROWS * 32 * 8) &&
               alloc((void **)&B.XP, T * PF_PITCH(4096)) && alloc((void **)&B.xscale, T * 4) && alloc((void **)&B.HP, PAIRS * PF_PITCH(768)) &&
               alloc((void **)&B.HS, PAIRS * 8 * 4) && alloc((void **)&B.Y, PAIRS * 2048 * 4) &&
-              alloc((void **)&B.sums, T * 128 * 4) && alloc((void **)&B.dump, T * 2048 * 4) && alloc((void **)&B.lg, T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
+              alloc((void **)&B.sums, T * 128 * 4) && alloc((void **)&B.dump, T * 2048 * 4) && alloc((void **)&B.lg, 4 * T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
               alloc((void **)&B.cnt, 128 * 4) && alloc((void **)&B.list, 128ull * QXP_LIST * 4) &&
               alloc((void **)&B.tokens, T * 4);
     // codebooks: grids as magnitude bytes, sign bytes (0x80 where negative), the IQ4_XS byte table as fp16
@@ -897,7 +897,7 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, bool first, 
     g.part_lines = g.lines / qkv_parts;
     g.rows_packed = B.XP; g.rows = T; g.row_bytes = PF_PITCH(2048); g.rscale = B.xscale; g.sums = B.sums; g.out = B.PART;
     qxp_launch_dense(s, g, qkv_parts, timer_for(c, 8));
-    hipLaunchKernelGGL(qxp_qk, dim3(T), dim3(256), 0, s, (const float *)B.PART, qkv_parts, T, w.q_norm, w.k_norm, c->T, c->kc,
+    hipLaunchKernelGGL(qxp_qk, dim3(T), dim3(640), 0, s, (const float *)B.PART, qkv_parts, T, w.q_norm, w.k_norm, c->T, c->kc,
                        c->vc, c->ks, c->vs, l, c->kv_ctx, p0, B.QR);
     const uint32_t runs = attn_runs(T, p0 + T);
     qx_launch(qxp_attn, dim3(4, (T + 3) / 4, runs), dim3(256), 0, s, timer_for(c, 13), (const float *)B.QR,
@@ -912,7 +912,7 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, bool first, 
     // MoE half: residual + RMSNorm, router logits, top-8 and the experts' pair lists, gate/up + SwiGLU, down, combine
     hipLaunchKernelGGL(qxp_ffn_norm, dim3(T), dim3(256), 0, s, (const float *)B.X, (const float *)B.PART, o_parts,
                        w.ffn_norm, T, B.X1, B.XN, B.XP, B.xscale);
-    qx_launch(qxp_router, dim3((T + 15) / 16, (E + 15) / 16), dim3(512), 0, s, timer_for(c, 12), (const float *)B.XN,
+    qx_launch(qxp_router, dim3((T + 15) / 16, (E + 15) / 16, 4), dim3(256), 0, s, timer_for(c, 12), (const float *)B.XN,
               w.router, T, E, B.lg, B.cnt);
     hipLaunchKernelGGL(qxp_route, dim3((T + 15) / 16), dim3(1024), 0, s, (const double *)B.lg, T, E, B.w, B.cnt, B.list);
     PfExperts x{};

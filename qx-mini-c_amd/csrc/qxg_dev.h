@@ -711,10 +711,13 @@ DEV void rows_reduce(float (&v)[R], float (&out)[R], int lane) {
 }
 
 
-DEV float block_max256(float v, float *red) {
+DEV float wave_max_f(float v) {
     v = fmaxf(v, dppf<DPP_XOR1>(v)); v = fmaxf(v, dppf<DPP_XOR2>(v));
     v = fmaxf(v, dppf<DPP_ROR4>(v)); v = fmaxf(v, dppf<DPP_ROR8>(v));
-    v = fmaxf(fmaxf(rdlanef(v, 0), rdlanef(v, 16)), fmaxf(rdlanef(v, 32), rdlanef(v, 48)));
+    return fmaxf(fmaxf(rdlanef(v, 0), rdlanef(v, 16)), fmaxf(rdlanef(v, 32), rdlanef(v, 48)));
+}
+DEV float block_max256(float v, float *red) {
+    v = wave_max_f(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();

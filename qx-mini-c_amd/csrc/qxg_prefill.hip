@@ -107,25 +107,25 @@ DEV void pack_dense8(const float *v, float sc, bool ok, uint8_t *row, float *sum
     t += dppf<DPP_XOR2>(t);
     if ((c & 3) == 0) sums[c >> 2] = t;
 }
-// v = the sum of `parts` rows of 8 values, stride floats apart, in order
+// v += rows k .. k + N - 1 of 8 values, stride floats apart, in order, all loaded at once
+template <int N>
+DEV void add_parts(const float *p, uint64_t stride, float (&v)[8]) {
+    float q[N][8];
+#pragma unroll
+    for (int u = 0; u < N; ++u) load8(p + u * stride, q[u]);
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += q[u][i];
+}
+// v = the sum of `parts` (a power of two) rows of 8 values, stride floats apart, in order
 DEV void sum_parts(const float *p, uint64_t stride, uint32_t parts, float (&v)[8]) {
-    load8(p, v);
-    uint32_t k = 1;
-    for (; k + 4 <= parts; k += 4) {
-        float q[4][8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) load8(p + (k + u) * stride, q[u]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] += q[u][i];
-    }
-    for (; k < parts; ++k) {
-        float q[8];
-        load8(p + k * stride, q);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] += q[i];
-    }
+    for (int i = 0; i < 8; ++i) v[i] = -0.0f;
+    if (parts == 1) add_parts<1>(p, stride, v);
+    else if (parts == 2) add_parts<2>(p, stride, v);
+    else if (parts == 4) add_parts<4>(p, stride, v);
+    else for (uint32_t k = 0; k < parts; k += 8) add_parts<8>(p + k * stride, stride, v);
 }
 // x1 + sum_r (float)(w_r * (double)y[8 t + r]), ranks in order (src/qx_format.c:5296-5309)
 DEV void combine8(const float *x1, const float *y, const double *wts, uint32_t t, int tid, float (&v)[8], float *moe) {
@@ -180,33 +180,53 @@ extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src,
     const int tid = threadIdx.x;
     const uint32_t t = blockIdx.x;
     float v[16];
+    const float *p = src + (uint64_t)t * 4096 + 8 * tid;
+    if (runs == 1) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t d = 2048 * i + 8 * tid, head = d >> 7;
-        float a[8];
-        if (runs == 1) {
-            load8(src + (uint64_t)t * 4096 + d, a);
-        } else {
-            float M = -INFINITY, L = 0.0f;
-            for (uint32_t r = 0; r < runs; ++r) M = fmaxf(M, md[((uint64_t)r * T + t) * 32 + head].x);
+        for (int i = 0; i < 2; ++i) load8(p + 2048 * i, *reinterpret_cast<float(*)[8]>(v + 8 * i));
+    } else {
+        // four runs' values and states at a time, so that one load latency covers them (37 tokens
+        // over 12 runs: 11.8 us a run at a time, now 8)
+        constexpr int N = 4;
+        const float2 *s = md + (uint64_t)t * 32 + (tid >> 4);   // heads tid / 16 and 16 + tid / 16
+        float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.0f, 0.0f};
 #pragma unroll
-            for (int j = 0; j < 8; ++j) a[j] = 0.0f;
-#pragma unroll 4
-            for (uint32_t r = 0; r < runs; ++r) {
-                const float2 s = md[((uint64_t)r * T + t) * 32 + head];
-                const float f = s.x == -INFINITY ? 0.0f : exp2_fast(s.x - M);
-                float b[8];
-                load8(src + ((uint64_t)r * T + t) * 4096 + d, b);
-                L = fmaf(f, s.y, L);
+        for (int j = 0; j < 16; ++j) v[j] = 0.0f;
+        for (uint32_t r0 = 0; r0 < runs; r0 += N) {
+            float b[N][2][8];
+            float2 st[N][2];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) a[j] = fmaf(f, b[j], a[j]);
+            for (int u = 0; u < N; ++u) {
+                const uint32_t r = min(r0 + u, runs - 1);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    st[u][i] = s[(uint64_t)r * T * 32 + 16 * i];
+                    load8(p + (uint64_t)r * T * 4096 + 2048 * i, b[u][i]);
+                }
             }
-            const float inv = 1.0f / L;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) a[j] *= inv;
+            for (int i = 0; i < 2; ++i) {
+                float m = M[i];
+#pragma unroll
+                for (int u = 0; u < N; ++u) m = fmaxf(m, st[u][i].x);   // (a repeated last run changes nothing)
+                const float f0 = M[i] == -INFINITY ? 0.0f : exp2_fast(M[i] - m);
+                L[i] *= f0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[8 * i + j] *= f0;
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    const float f = r0 + u >= runs || st[u][i].x == -INFINITY ? 0.0f : exp2_fast(st[u][i].x - m);
+                    L[i] = fmaf(f, st[u][i].y, L[i]);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) v[8 * i + j] = fmaf(f, b[u][i][j], v[8 * i + j]);
+                }
+                M[i] = m;
+            }
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[8 * i + j] = a[j];
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[8 * i + j] *= 1.0f / L[i];
     }
     int sh;
     const bool ok = block_shift<16>(v, redf, sh);
@@ -246,51 +266,54 @@ extern "C" __global__ __launch_bounds__(256) void qxp_ffn_norm(const float *x, c
 // Per token (block): the Q/K/V GEMM's parts of K added in order (non-finite results 0,
 // src/qx_format.c:4284), q/k head RMSNorm (src/qx_format.c:3740-3757) and RoPE at position
 // p0+t (4625-4641), INT8 quantization of K and V over all 512 values (4449-4463) into
-// the cache row [layer][p0+t]; the roped q (f32) goes to qr for attention.
-extern "C" __global__ __launch_bounds__(256) void qxp_qk(const float *parts, uint32_t nparts, uint32_t rows, const float *q_norm,
+// the cache row [layer][p0+t]; the roped q (f32) goes to qr for attention.  Ten waves: each
+// thread adds 8 columns, then waves 0 to 7 take four q heads each, wave 8 K and wave 9 V.
+// Latency bounds it.  (Four waves with three runs of adds and eight q heads each: 8.9 us for
+// 37 tokens, now 6.8.)
+extern "C" __global__ __launch_bounds__(640) void qxp_qk(const float *parts, uint32_t nparts, uint32_t rows, const float *q_norm,
         const float *k_norm, Tables T, int8_t *kc, int8_t *vc, float *ks, float *vs, uint32_t layer, uint32_t ctx, uint32_t p0,
         float *qr) {
-    __shared__ float s_row[5120], s_k[512];
-    __shared__ float red[4];
+    __shared__ float s_row[5120];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const uint32_t t = blockIdx.x, pos = p0 + t;
-    const float kw0 = k_norm[lane], kw1 = k_norm[64 + lane], qw0 = q_norm[lane], qw1 = q_norm[64 + lane];
+    const float *nw = wave == 8 ? k_norm : q_norm;
+    const float w0 = nw[lane], w1 = nw[64 + lane];
     const double c = T.rope_cos[pos * 64 + lane], s = T.rope_sin[pos * 64 + lane];
-    float v[3][8];
+    float v[8];
+    sum_parts(parts + (uint64_t)t * 5120 + 8 * tid, (uint64_t)rows * 5120, nparts, v);
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-        if (i < 2 || tid < 128) sum_parts(parts + (uint64_t)t * 5120 + 2048 * i + 8 * tid, (uint64_t)rows * 5120, nparts, v[i]);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-        if (i < 2 || tid < 128) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[i][j] = isfinite(v[i][j]) ? v[i][j] : 0.0f;
-            store8(s_row + 2048 * i + 8 * tid, v[i]);
-        }
+    for (int j = 0; j < 8; ++j) v[j] = isfinite(v[j]) ? v[j] : 0.0f;
+    store8(s_row + 8 * tid, v);
     __syncthreads();
-    float k0 = s_row[4096 + 128 * wave + lane], k1 = s_row[4096 + 128 * wave + 64 + lane];
-    const float v0 = s_row[4608 + tid], v1 = s_row[4608 + 256 + tid];
-    head_norm_rope_wave(k0, k1, kw0, kw1, c, s);
-    s_k[128 * wave + lane] = k0;
-    s_k[128 * wave + 64 + lane] = k1;
-#pragma unroll 2
-    for (int hh = 0; hh < 8; ++hh) {
-        const int qh = 8 * wave + hh;
-        float q0 = s_row[128 * qh + lane], q1 = s_row[128 * qh + 64 + lane];
-        head_norm_rope_wave(q0, q1, qw0, qw1, c, s);
-        qr[(uint64_t)t * 4096 + 128 * qh + lane] = q0;
-        qr[(uint64_t)t * 4096 + 128 * qh + 64 + lane] = q1;
+    const float *own = s_row + 512 * wave + lane;   // the wave's four heads
+    float a[4][2];
+#pragma unroll
+    for (int hh = 0; hh < 4; ++hh) {
+        a[hh][0] = own[128 * hh];
+        a[hh][1] = own[128 * hh + 64];
+        if (wave < 9) head_norm_rope_wave(a[hh][0], a[hh][1], w0, w1, c, s);
     }
-    float ka = fmaxf(int8_mag(k0), int8_mag(k1)), va = fmaxf(int8_mag(v0), int8_mag(v1));
-    ka = block_max256(ka, red);
-    va = block_max256(va, red);
-    const float kscale = int8_scale(ka), vscale = int8_scale(va);
+    if (wave < 8) {
+#pragma unroll
+        for (int hh = 0; hh < 4; ++hh) {
+            float *q = qr + (uint64_t)t * 4096 + 512 * wave + 128 * hh + lane;
+            q[0] = a[hh][0];
+            q[64] = a[hh][1];
+        }
+        return;
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int hh = 0; hh < 4; ++hh) mx = fmaxf(mx, fmaxf(int8_mag(a[hh][0]), int8_mag(a[hh][1])));
+    const float scale = int8_scale(wave_max_f(mx));
     const uint64_t slot = (uint64_t)layer * ctx + pos;
-    for (int i = tid; i < 512; i += 256) {
-        kc[slot * 512 + i] = int8_code(s_k[i], kscale);
-        vc[slot * 512 + i] = int8_code(i < 256 ? v0 : v1, vscale);
+    int8_t *code = (wave == 8 ? kc : vc) + slot * 512 + lane;
+#pragma unroll
+    for (int hh = 0; hh < 4; ++hh) {
+        code[128 * hh] = int8_code(a[hh][0], scale);
+        code[128 * hh + 64] = int8_code(a[hh][1], scale);
     }
-    if (tid == 0) { ks[slot] = kscale; vs[slot] = vscale; }
+    if (lane == 0) (wave == 8 ? ks : vs)[slot] = scale;
 }
 
 // Causal GQA attention of the chunk on the matrix cores (qx_rope_gqa_attention_partial,
@@ -581,42 +604,47 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
 // Router logits on the FP64 matrix cores: logit[t][e] = sum_i (double)W[e][i] *
 // (double)xn[t][i] (src/qx_format.c:5254-5264: the same exact double products, summed in
 // another order, within ~1e-15 relative of the reference's sequential sum; equal router
-// rows still give equal logits).  A workgroup owns a 16 x 16 (token x expert) tile; its 8
-// waves split K = 2048 in eighths and lane group g = lane / 16 of a wave feeds k-slot g
-// of v_mfma_f64_16x16x4 with 64 consecutive k of the wave's 256.  The 8 partial tiles
-// are added in LDS in a fixed order.
+// rows still give equal logits).  A workgroup owns a 16 x 16 (token x expert) tile of one
+// quarter of K; its 4 waves split that in 128s, and lane group g = lane / 16 of a wave feeds
+// k-slot g of v_mfma_f64_16x16x4 with float4 g of each 16 k.  The waves' tiles are added in
+// LDS in a fixed order, the quarters (planes of `logits`) by qxp_route.  Latency bounds it: a
+// wave's loads are all in flight before its first product, and a row's four lane groups
+// read one 64-byte piece.  (A workgroup over all of K, loads four iterations at a time: 11.4 us
+// for 37 tokens and 12.6 for 512; now 4.9 and 10.2.)
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-extern "C" __global__ __launch_bounds__(512) void qxp_router(const float *xn, const float *router, uint32_t T,
+extern "C" __global__ __launch_bounds__(256) void qxp_router(const float *xn, const float *router, uint32_t T,
                                                              uint32_t experts, double *logits, uint32_t *cnt) {
-    __shared__ double part[8][16][17];
+    __shared__ double part[4][16][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int i = lane & 15, g = lane >> 4;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid < 128) cnt[tid] = 0u;   // for qxp_route, the next launch
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid < 128) cnt[tid] = 0u;   // for qxp_route, the next launch
     const uint32_t t = blockIdx.x * 16 + i;   // < 512: xn holds QXP_MAX rows
     const uint32_t e = blockIdx.y * 16 + i, er = e < experts ? e : 0u;
-    const float4 *xa = reinterpret_cast<const float4 *>(xn + (uint64_t)t * 2048 + wave * 256 + g * 64);
-    const float4 *wb = reinterpret_cast<const float4 *>(router + (uint64_t)er * 2048 + wave * 256 + g * 64);
+    const uint32_t k0 = blockIdx.z * 512 + wave * 128 + g * 4;
+    const float *xa = xn + (uint64_t)t * 2048 + k0, *wb = router + (uint64_t)er * 2048 + k0;
+    float4 a[8], b[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        a[j] = *reinterpret_cast<const float4 *>(xa + 16 * j);
+        b[j] = *reinterpret_cast<const float4 *>(wb + 16 * j);
+    }
     f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (int j = 0; j < 16; ++j) {
-        const float4 a = xa[j], b = wb[j];
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.x, (double)b.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.y, (double)b.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.z, (double)b.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a.w, (double)b.w, acc, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[j].x, (double)b[j].x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[j].y, (double)b[j].y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[j].z, (double)b[j].z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[j].w, (double)b[j].w, acc, 0, 0, 0);
     }
     // result r of lane l: token row l / 16 + 4 * r, expert column l % 16 (the f64 16x16
     // layout, unlike the f32 ones' 4 * (l / 16) + r)
 #pragma unroll
     for (int r = 0; r < 4; ++r) part[wave][g + 4 * r][i] = acc[r];
     __syncthreads();
-    if (tid < 256) {
-        const int row = tid >> 4, col = tid & 15;
-        const double v = ((part[0][row][col] + part[1][row][col]) + (part[2][row][col] + part[3][row][col])) +
-                         ((part[4][row][col] + part[5][row][col]) + (part[6][row][col] + part[7][row][col]));
-        const uint32_t tt = blockIdx.x * 16 + row, ee = blockIdx.y * 16 + col;
-        if (tt < T && ee < experts) logits[(uint64_t)tt * 128 + ee] = v;
-    }
+    const int row = tid >> 4, col = tid & 15;
+    const double v = (part[0][row][col] + part[1][row][col]) + (part[2][row][col] + part[3][row][col]);
+    const uint32_t tt = blockIdx.x * 16 + row, ee = blockIdx.y * 16 + col;
+    if (tt < T && ee < experts) logits[((uint64_t)blockIdx.z * QXP_MAX + tt) * 128 + ee] = v;
 }
 
 // Top-8 experts and renormalised weights per token (the decode path's selection,
@@ -635,8 +663,14 @@ extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logit
     const uint32_t t = blockIdx.x * 16 + wave_id();
     uint32_t e = 0, place = 0;
     if (t < T) {   // whole wave
-        const double l0 = lane < E ? logits[(uint64_t)t * 128 + lane] : 0.0;
-        const double l1 = lane + 64 < E ? logits[(uint64_t)t * 128 + lane + 64] : 0.0;
+        double q[4][2];   // the quarters of K
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double *lg = logits + ((uint64_t)k * QXP_MAX + t) * 128;
+            q[k][0] = lane < E ? lg[lane] : 0.0;
+            q[k][1] = lane + 64 < E ? lg[lane + 64] : 0.0;
+        }
+        const double l0 = (q[0][0] + q[1][0]) + (q[2][0] + q[3][0]), l1 = (q[0][1] + q[1][1]) + (q[2][1] + q[3][1]);
         uint32_t id[QXG_TOPK];
         double w[QXG_TOPK];
         wave_top8(l0, l1, E, id, w);
