@@ -211,10 +211,9 @@ struct QxDArgs {
 
 // ---- batched prefill (qxg_prefill.hip)
 #define QXP_MAX 512   // tokens per prefill chunk
-// Bytes from one packed activation row of K values (hi and lo, 4 bytes a value) to the next.  A
-// GEMM's workgroups read one 128-byte line of each of their rows at a time, all along K in step:
-// at a pitch of K * 4 alone (a multiple of 4 KB, or of 1 KB) those lines meet in one L2 channel
-// (or four); 256 bytes more spread them over all sixteen.
+// Bytes from one packed activation row of K values (hi and lo, 4 bytes a value) to the next: two
+// lines more than the values, so that rows do not lie at a power-of-two stride (measured neutral:
+// Q/K/V of 512 tokens 40.0 us without and 39.9 with them)
 #define PF_PITCH(K) (4u * (K) + 256u)
 // entries of one expert's pair list: every (token, rank) pair of a chunk (an expert takes a
 // token once, except where non-finite logits make the top-8 repeat it)

@@ -46,37 +46,41 @@ DEV void wait_loads() {
 
 constexpr int RT = 2;                    // 32-row tiles of a workgroup, at most
 constexpr int ROWS = 32 * RT;
-constexpr int STAGE = 4 * ROWS * 8;      // uint4 per stage: 4 lines of 8 chunks a row
+template <int R> constexpr int STAGE = 4 * R * 8;   // uint4 per stage of R rows: 4 lines of 8 chunks a row
 
 // The four lines from line0 on of the workgroup's rows: wave w copies line w, 8 rows an
 // instruction; off[i] is the lane's row 8 i + lane / 8 and its chunk of the line.
-template <int MT>
-DEV void stage_rows(const void *rows, const uint32_t (&off)[4 * MT], uint32_t line0, uint4 *buf, int wave) {
+template <int R>
+DEV void stage_rows(const void *rows, const uint32_t (&off)[R / 8], uint32_t line0, uint4 *buf, int wave) {
 #pragma unroll
-    for (int i = 0; i < 4 * MT; ++i) dma16(rows, off[i] + (line0 + wave) * 128, buf + (wave * ROWS + 8 * i) * 8);
+    for (int i = 0; i < R / 8; ++i) dma16(rows, off[i] + (line0 + wave) * 128, buf + (wave * R + 8 * i) * 8);
 }
 // byte offset in its line of the chunk that lane copies in instruction i
 DEV uint32_t stage_chunk(int i, int lane) { return ((lane ^ (4 * i + (lane >> 4))) & 7) << 4; }
-template <int MT>
-DEV void stage_offsets(uint32_t (&off)[4 * MT], const uint32_t *s_row, uint32_t row_bytes, int lane) {
+template <int R>
+DEV void stage_offsets(uint32_t (&off)[R / 8], const uint32_t *s_row, uint32_t row_bytes, int lane) {
 #pragma unroll
-    for (int i = 0; i < 4 * MT; ++i) off[i] = s_row[8 * i + (lane >> 3)] * row_bytes + stage_chunk(i, lane);
+    for (int i = 0; i < R / 8; ++i) off[i] = s_row[8 * i + (lane >> 3)] * row_bytes + stage_chunk(i, lane);
 }
-// A fragments of k-step s of the stage: lane's row l%32 of each tile, lane half l/32
+// A fragments of k-step s of the stage: lane's row l%32 of each tile, lane half l/32.  Of 16
+// rows there is one fragment, tile rows 0 .. 15 their hi and 16 .. 31 their lo halves: one
+// matrix instruction does both products, and register r + 8 of a result is the lo part of r's.
 struct ALane { uint32_t at[4]; };   // byte offset of chunk 2 i + h in the lane's row of line 0
+template <int R>
 DEV ALane a_lane(int lane) {
     ALane a;
+    const int row = lane & (R == 16 ? 15 : 31), lo = R == 16 ? (lane >> 4) & 1 : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a.at[i] = (lane & 31) * 128 + ((((2 * i + (lane >> 5)) ^ (lane >> 1)) & 7) << 4);
+    for (int i = 0; i < 4; ++i) a.at[i] = row * 128 + ((((2 * (i | lo) + (lane >> 5)) ^ (row >> 1)) & 7) << 4);
     return a;
 }
-template <int MT>
+template <int R, int MT>
 DEV void a_read(uint4 (&ah)[MT], uint4 (&al)[MT], const uint4 *buf, const ALane &a, int s) {
-    const uint8_t *p = reinterpret_cast<const uint8_t *>(buf) + (s >> 1) * (ROWS * 128);
+    const uint8_t *p = reinterpret_cast<const uint8_t *>(buf) + (s >> 1) * (R * 128);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         ah[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1)]);
-        al[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1) + 1]);
+        if (R > 16) al[mt] = *reinterpret_cast<const uint4 *>(p + mt * 4096 + a.at[2 * (s & 1) + 1]);
     }
 }
 }  // namespace

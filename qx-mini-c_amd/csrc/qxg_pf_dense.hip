@@ -6,7 +6,8 @@
 // the f32 scale (d * (ls - 32) or d * sc) and, for Q5_K, the offset dmin * m: 1.13 bytes a
 // weight, 21 MB a layer.  A code becomes fp16 as bits(1024 + byte) - 1152, two a v_perm and
 // v_pk_add.  From the file's nibbles the same codes took a random LDS read per byte, for every
-// row tile again, which bounded the kernel (57 us for Q/K/V of 512 tokens, 20 now).
+// row tile again, which bounded the kernel (56 us for Q/K/V and 49 for O of 512 tokens, now 36 and 27; 25 and
+// 48 of 37, now 10 and 9).  The matrix instructions bound it, about 20 us of the 36.
 //
 // Tiles.  A workgroup takes up to 64 rows x 128 columns (4 waves of 32 columns) over a run of K;
 // the rows are staged in LDS, the codes go straight to registers.  The matrix cores sum 32
@@ -48,7 +49,7 @@ DEV void dns_tile(const PfDense &g, uint4 *buf, float *s_sum) {
         off[i] = min(row0 + 8 * i + (lane >> 3), g.rows - 1) * g.row_bytes + stage_chunk(i, lane);
     const uint32_t srow = min(row0 + (uint32_t)(tid & (32 * MT - 1)), g.rows - 1);
     auto stage = [&](uint32_t st) {
-        stage_rows<MT>(g.rows_packed, off, l0 + 4 * st, buf + (st & 1) * STAGE, wave);
+        stage_rows<32 * MT>(g.rows_packed, off, l0 + 4 * st, buf + (st & 1) * STAGE<32 * MT>, wave);
     };
     // the rows' sums of the stage's four lines, for the offsets
     auto load_sum = [&](uint32_t st) {
@@ -58,7 +59,7 @@ DEV void dns_tile(const PfDense &g, uint4 *buf, float *s_sum) {
     dns_load<OFS>(cur, g, ct, l0, lane, ofs);
     stage(0);
     float sum = OFS ? load_sum(0) : 0.0f;
-    const ALane at = a_lane(lane);
+    const ALane at = a_lane<32 * MT>(lane);
     f16x acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] = zero16();
@@ -71,7 +72,7 @@ DEV void dns_tile(const PfDense &g, uint4 *buf, float *s_sum) {
         if (sn != st) stage(sn);
         dns_load<OFS>(nxt, g, ct, l0 + 4 * sn, lane, ofs);
         if (OFS) sum = load_sum(sn);
-        const uint4 *sb = buf + (st & 1) * STAGE;
+        const uint4 *sb = buf + (st & 1) * STAGE<32 * MT>;
         // line l's sums times the column's scale, less its offset times the rows' sums
         auto add = [&](f16x (&acc)[MT], const f16x (&G)[MT], int l) {
             const float sc = l == 0 ? cur.sc.x : l == 1 ? cur.sc.y : l == 2 ? cur.sc.z : cur.sc.w;
@@ -94,14 +95,14 @@ DEV void dns_tile(const PfDense &g, uint4 *buf, float *s_sum) {
         // a line's rows are read while the line before is multiplied, and a line's sums join the
         // accumulators behind the next line's products: one wave a SIMD has to overlap both itself
         uint4 ah[2][MT], al[2][MT], nh[2][MT], nl[2][MT];
-        a_read<MT>(ah[0], al[0], sb, at, 0);
-        a_read<MT>(ah[1], al[1], sb, at, 1);
+        a_read<32 * MT, MT>(ah[0], al[0], sb, at, 0);
+        a_read<32 * MT, MT>(ah[1], al[1], sb, at, 1);
         f16x P[MT];   // the previous line's sums, still unscaled
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             if (l < 3) {
-                a_read<MT>(nh[0], nl[0], sb, at, 2 * l + 2);
-                a_read<MT>(nh[1], nl[1], sb, at, 2 * l + 3);
+                a_read<32 * MT, MT>(nh[0], nl[0], sb, at, 2 * l + 2);
+                a_read<32 * MT, MT>(nh[1], nl[1], sb, at, 2 * l + 3);
             }
             __builtin_amdgcn_sched_barrier(0);
             const uint4 b0 = biased8(cur.q[l].x, cur.q[l].y), b1 = biased8(cur.q[l].z, cur.q[l].w);
@@ -149,7 +150,7 @@ DEV void dns_tile(const PfDense &g, uint4 *buf, float *s_sum) {
 
 template <int MT, bool OFS>
 __global__ __launch_bounds__(256, 2) void qxp_dense(PfDense g) {
-    __shared__ uint4 s_buf[2 * STAGE];
+    __shared__ uint4 s_buf[2 * STAGE<32 * MT>];
     __shared__ float s_sum[OFS ? 2 * 4 * ROWS : 1];
     dns_tile<MT, OFS>(g, s_buf, s_sum);
 }

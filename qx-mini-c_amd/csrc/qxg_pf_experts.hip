@@ -5,8 +5,8 @@
 // into fp16 hi + lo, the matrix cores accumulate in f32.  Here:
 //
 // Rows.  qxp_route lists each expert's (token, rank) pairs, p = 8 * token + rank; a
-// workgroup takes up to 64 of one expert's pairs and a range of its weight rows, so every
-// code is formed once for up to two 32-row tiles.  Activations are packed per token
+// workgroup takes up to 32 or 64 of one expert's pairs and a range of its weight rows, and
+// forms each code once for them.  Activations are packed per token
 // (gate/up, gathered through the list while they are staged) and per pair (down, written
 // by gate/up's epilogue); no copy of them is sorted or padded by expert.
 //
@@ -23,9 +23,9 @@
 // block scale takes the 2^13).  Random 16-byte reads of ready fp16 entries and fp16 sign masks
 // kept the LDS busy for most of the kernel; these take about 6 cycles each.
 //
-// What bounds them: the matrix cores at their sustained rate (about 1.4 PFLOP/s for tens of us,
-// power-limited), with twice the algorithmic work for hi and lo, where experts hold many pairs; the
-// weights' bytes and the about 20 vector instructions per 8 codes where they hold few.
+// What bounds them: the matrix instructions (twice the algorithmic work, for hi and lo) and the about 16
+// vector instructions per 8 codes, which share a SIMD's time nearly without overlap (counted on 128
+// random rows of gate/up: 49k and 59k of 120k cycles).
 #include "qxg_pf.h"
 
 namespace {
@@ -86,32 +86,30 @@ DEV Codes gu_look(const GuBlk<FMT_IQ2S> &w, int s, const uint2 *grid, const uint
 
 // k-steps 8 half .. 8 half + 7 of a block: gate (tile 0) and up (1) of the wave's 32 columns.
 // Tile i's codes are looked up two tiles ahead and formed one ahead.
-template <int F, int MT>
-DEV void gu_half(const GuBlk<F> (&w)[2], int half, const uint4 *buf, const ALane &at, f16x (&G)[2][MT], const uint2 *grid,
+template <int F, int R>
+DEV void gu_half(const GuBlk<F> (&w)[2], int half, const uint4 *buf, const ALane &at, f16x (&G)[2], const uint2 *grid,
                  const uint2 *sgn) {
     Codes c0 = gu_look(w[0], 8 * half, grid, sgn), c1 = gu_look(w[1], 8 * half, grid, sgn);
-    uint4 ah[MT], al[MT];
-    a_read<MT>(ah, al, buf, at, 0);
+    uint4 ah[1], al[1];
+    a_read<R, 1>(ah, al, buf, at, 0);
     h2v m[2] = {odd_mul((w[0].sc >> (16 * half)) & 15u), odd_mul((w[1].sc >> (16 * half)) & 15u)};
     uint4 b = conv(c0, m[0]);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int s = i >> 1, f = i & 1, sn = (i + 1) >> 1, fn = (i + 1) & 1;
-        uint4 bn = b, nh[MT], nl[MT];
+        uint4 bn = b, nh[1], nl[1];
         if (i < 15) {
             if (sn && !(sn & 1)) m[fn] = odd_mul((w[fn].sc >> (16 * half + 4 * (sn >> 1))) & 15u);
             bn = conv(c1, m[fn]);
         }
         if (i < 14) c1 = gu_look(w[f], 8 * half + s + 1, grid, sgn);
-        if (f == 1 && s < 7) a_read<MT>(nh, nl, buf, at, s + 1);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(ah[mt], b, G[f][mt]);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(al[mt], b, G[f][mt]);
+        if (f == 1 && s < 7) a_read<R, 1>(nh, nl, buf, at, s + 1);
+        G[f] = mfma(ah[0], b, G[f]);
+        if (R > 16) G[f] = mfma(al[0], b, G[f]);
         b = bn;
         if (f == 1 && s < 7) {
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) { ah[mt] = nh[mt]; al[mt] = nl[mt]; }
+            ah[0] = nh[0];
+            if (R > 16) al[0] = nl[0];
         }
     }
 }
@@ -126,56 +124,47 @@ DEV float div_ge1(float x, float y) {
 }
 DEV float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }   // 2^e, -126 <= e <= 127
 
-template <int F, int MT>
+template <int F, int R>
 DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *list, uint32_t n, const uint2 *grid,
                  const uint2 *sgn, uint4 *buf, uint32_t *s_row, float *s_xs) {
+    constexpr int NR = R > 16 ? 16 : 8;   // result registers of a tile, hi and lo added
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
     const uint32_t bi = (e * QXG_FFN + 128 * cg + 32 * wave + col) * 8;   // tiles 0 and 1: this row of gate and of up
     GuBlk<F> cur[2], nxt[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f) gu_load(cur[f], a.w[f], bi, h);
-    if (tid < 32 * MT) {
+    if (tid < R) {
         const uint32_t t = list[min((uint32_t)tid, n - 1)] >> 3;
         s_row[tid] = t;
         s_xs[tid] = a.xs[t];
     }
     __syncthreads();   // the rows' tokens, and the tables
-    uint32_t off[4 * MT];
-    stage_offsets<MT>(off, s_row, PF_PITCH(2048), lane);
-    stage_rows<MT>(a.xp, off, 0, buf, wave);
-    const ALane at = a_lane(lane);
-    f16x acc[2][MT];
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[f][mt] = zero16();
+    uint32_t off[R / 8];
+    stage_offsets<R>(off, s_row, PF_PITCH(2048), lane);
+    stage_rows<R>(a.xp, off, 0, buf, wave);
+    const ALane at = a_lane<R>(lane);
+    f16x acc[2] = {zero16(), zero16()};
 #pragma unroll 1
     for (uint32_t b = 0; b < 8; ++b) {
-        f16x G[2][MT];
-#pragma unroll
-        for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) G[f][mt] = zero16();
+        f16x G[2] = {zero16(), zero16()};
         wait_loads<0>();
         __syncthreads();   // the block's first half is staged; every wave is past the last block's second half
-        stage_rows<MT>(a.xp, off, 8 * b + 4, buf + STAGE, wave);
+        stage_rows<R>(a.xp, off, 8 * b + 4, buf + STAGE<R>, wave);
         __builtin_amdgcn_sched_barrier(0);   // the weights' loads stay the youngest: the wait below leaves them in flight
         const uint32_t bn = b < 7 ? b + 1 : 7;
 #pragma unroll
         for (int f = 0; f < 2; ++f) gu_load(nxt[f], a.w[f], bi + bn, h);
         __builtin_amdgcn_sched_barrier(0);
-        gu_half<F, MT>(cur, 0, buf, at, G, grid, sgn);
+        gu_half<F, R>(cur, 0, buf, at, G, grid, sgn);
         wait_loads<2 * GU_LOADS<F>>();
         __syncthreads();
-        if (b < 7) stage_rows<MT>(a.xp, off, 8 * b + 8, buf, wave);
-        gu_half<F, MT>(cur, 1, buf + STAGE, at, G, grid, sgn);
+        if (b < 7) stage_rows<R>(a.xp, off, 8 * b + 8, buf, wave);
+        gu_half<F, R>(cur, 1, buf + STAGE<R>, at, G, grid, sgn);
 #pragma unroll
         for (int f = 0; f < 2; ++f) {
             const float d = fp16_exact(cur[f].d) * (0.125f * CODE_SCALE);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[f][mt][r] = fmaf(d, G[f][mt][r], acc[f][mt][r]);
+            for (int r = 0; r < NR; ++r) acc[f][r] = fmaf(d, R > 16 ? G[f][r] : G[f][r] + G[f][(r + 8) & 15], acc[f][r]);
             cur[f] = nxt[f];
         }
     }
@@ -185,23 +174,21 @@ DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
     float *hs = reinterpret_cast<float *>(buf);
     constexpr int LD = 132;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
-            const float rs = s_xs[row];
-            float gv = acc[0][mt][r] * rs, uv = acc[1][mt][r] * rs;
-            gv = isfinite(gv) ? gv : 0.0f;   // (src/qx_format.c:4284)
-            uv = isfinite(uv) ? uv : 0.0f;
-            const float ex = expf(-gv);      // (infinite below -88: the quotient is 0)
-            hs[row * LD + 32 * wave + col] = (ex < INFINITY ? div_ge1(gv, 1.0f + ex) : 0.0f) * uv;
-        }
+    for (int r = 0; r < NR; ++r) {
+        const uint32_t row = 8 * (r >> 2) + 4 * h + (r & 3);
+        const float rs = s_xs[row];
+        float gv = acc[0][r] * rs, uv = acc[1][r] * rs;
+        gv = isfinite(gv) ? gv : 0.0f;   // (src/qx_format.c:4284)
+        uv = isfinite(uv) ? uv : 0.0f;
+        const float ex = expf(-gv);      // (infinite below -88: the quotient is 0)
+        hs[row * LD + 32 * wave + col] = (ex < INFINITY ? div_ge1(gv, 1.0f + ex) : 0.0f) * uv;
+    }
     __syncthreads();
     // each row's 128 values become the down projection's packed operand, 16 lanes a row with 8
     // values each, under a power-of-two scale of their own; a non-finite value makes the
     // scale a NaN, which zeroes the pair's down row (its own non-finite rule)
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) {
+    for (int i = 0; i < R / 16; ++i) {
         const uint32_t row = 16 * i + (tid >> 4), c = tid & 15;
         // chunk c of the 128 values: k-step and lane half of the down operand's order
         const uint32_t ks = 8 * cg + (a.h_pairs ? 2 * (c >> 2) + ((c >> 1) & 1) : c & 7), hh = a.h_pairs ? c & 1 : c >> 3;
@@ -292,39 +279,52 @@ DEV float dn_scale(const DnHalf<FMT_IQ4> &w, int half, int i) {   // sub-block i
     return fp16_exact(w.m.x & 0xffffu) * (float)(ls - 32);
 }
 
-template <int F, int MT>
+template <int F, int R>
 DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *list, uint32_t n, const uint32_t *grid,
                  const uint2 *sgn, uint4 *buf, uint32_t *s_row, float *s_hs) {
+    constexpr int MT = R > 32 ? 2 : 1, NR = R > 16 ? 16 : 8;   // tiles; result registers of a tile, hi and lo added
+    // half blocks loaded at once: both where the registers allow it (read apart, a block's lines came
+    // twice from beyond L2: 98 MB for 47 of weights; IQ4_XS has whole lines per half)
+    constexpr int NH = MT == 1 && F != FMT_IQ4 ? 2 : 1;
     constexpr bool PER32 = F == FMT_IQ4;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
     uint32_t bi[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f) bi[f] = (e * 2048u + 256 * cg + 64 * wave + 32 * f + col) * 3;
-    DnHalf<F> cur[2], nxt[2];
+    DnHalf<F> cur[2][NH], nxt[2][NH];
 #pragma unroll
-    for (int f = 0; f < 2; ++f) dn_load(cur[f], a.w[2], bi[f], 0, h);
-    if (tid < 32 * MT) s_row[tid] = list[min((uint32_t)tid, n - 1)];
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int i = 0; i < NH; ++i) dn_load(cur[f][i], a.w[2], bi[f], i, h);
+    if (tid < R) s_row[tid] = list[min((uint32_t)tid, n - 1)];
     __syncthreads();   // the rows' pairs, and the tables
-    uint32_t off[4 * MT];
-    stage_offsets<MT>(off, s_row, PF_PITCH(768), lane);
-    stage_rows<MT>(a.hp, off, 0, buf, wave);
-    const ALane at = a_lane(lane);
-    for (int i = tid; i < 6 * 32 * MT; i += 256)   // the rows' scales of each 128 values
-        s_hs[(i / (32 * MT)) * ROWS + i % (32 * MT)] = a.hs[(uint64_t)s_row[i % (32 * MT)] * 8 + i / (32 * MT)];
+    uint32_t off[R / 8];
+    stage_offsets<R>(off, s_row, PF_PITCH(768), lane);
+    stage_rows<R>(a.hp, off, 0, buf, wave);
+    const ALane at = a_lane<R>(lane);
+    for (int i = tid; i < 6 * R; i += 256)   // the rows' scales of each 128 values
+        s_hs[i] = a.hs[(uint64_t)s_row[i % R] * 8 + i / R];
     f16x acc[2][MT];
 #pragma unroll
     for (int f = 0; f < 2; ++f)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[f][mt] = zero16();
 #pragma unroll 1
-    for (int st = 0; st < 6; ++st) {
+    for (int st0 = 0; st0 < 6; st0 += NH)
+#pragma unroll
+    for (int hf = 0; hf < NH; ++hf) {
+        const int st = st0 + hf;
         wait_loads<0>();
         __syncthreads();   // stage st is in; every wave is past stage st - 1
         const int sn = st < 5 ? st + 1 : 5;
-        if (st < 5) stage_rows<MT>(a.hp, off, 4 * sn, buf + (sn & 1) * STAGE, wave);
+        if (st < 5) stage_rows<R>(a.hp, off, 4 * sn, buf + (sn & 1) * STAGE<R>, wave);
+        if (NH == 1 || hf == 0)
 #pragma unroll
-        for (int f = 0; f < 2; ++f) dn_load(nxt[f], a.w[2], bi[f] + (sn >> 1), sn & 1, h);
-        const uint4 *sb = buf + (st & 1) * STAGE;
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int i = 0; i < NH; ++i)
+                    dn_load(nxt[f][i], a.w[2], bi[f] + (NH == 1 ? sn >> 1 : min(st / 2 + 1, 2)), NH == 1 ? sn & 1 : i, h);
+        const uint4 *sb = buf + (st & 1) * STAGE<R>;
         f16x G[2][MT];
 #pragma unroll
         for (int f = 0; f < 2; ++f)
@@ -332,37 +332,41 @@ DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
             for (int mt = 0; mt < MT; ++mt) G[f][mt] = zero16();
         // the column's scale (of the block or of sub-block i) times the rows' scales, onto acc
         auto flush = [&](int f, int i) {
-            const float d = dn_scale(cur[f], st & 1, i);
+            const float d = dn_scale(cur[f][hf], st & 1, i);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f4x hsr = *reinterpret_cast<const f4x *>(s_hs + st * ROWS + 32 * mt + 8 * q + 4 * h);
+                for (int q = 0; q < NR / 4; ++q) {
+                    const f4x hsr = *reinterpret_cast<const f4x *>(s_hs + st * R + 32 * mt + 8 * q + 4 * h);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        acc[f][mt][4 * q + r] = fmaf(d * hsr[r], G[f][mt][4 * q + r], acc[f][mt][4 * q + r]);
-                        if (PER32) G[f][mt][4 * q + r] = 0.0f;
+                        const int k = 4 * q + r;
+                        acc[f][mt][k] = fmaf(d * hsr[r], R > 16 ? G[f][mt][k] : G[f][mt][k] + G[f][mt][(k + 8) & 15], acc[f][mt][k]);
+                        if (PER32) {
+                            G[f][mt][k] = 0.0f;
+                            if (R == 16) G[f][mt][(k + 8) & 15] = 0.0f;
+                        }
                     }
                 }
         };
         auto form = [&](const Codes &c, int f, int s) {
-            return PER32 ? make_uint4(c.m0, c.m1, c.sg.x, c.sg.y) : conv(c, dn_mul(cur[f], s >> 2));
+            return PER32 ? make_uint4(c.m0, c.m1, c.sg.x, c.sg.y) : conv(c, dn_mul(cur[f][hf], s >> 2));
         };
-        Codes c1 = dn_look(cur[1], 0, grid, sgn);
+        Codes c1 = dn_look(cur[1][hf], 0, grid, sgn);
         uint4 ah[MT], al[MT];
-        a_read<MT>(ah, al, sb, at, 0);
-        uint4 b = form(dn_look(cur[0], 0, grid, sgn), 0, 0);
+        a_read<R, MT>(ah, al, sb, at, 0);
+        uint4 b = form(dn_look(cur[0][hf], 0, grid, sgn), 0, 0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int s = i >> 1, f = i & 1;
             uint4 bn = b, nh[MT], nl[MT];
             if (i < 15) bn = form(c1, (i + 1) & 1, (i + 1) >> 1);
-            if (i < 14) c1 = dn_look(cur[f], s + 1, grid, sgn);
-            if (f == 1 && s < 7) a_read<MT>(nh, nl, sb, at, s + 1);
+            if (i < 14) c1 = dn_look(cur[f][hf], s + 1, grid, sgn);
+            if (f == 1 && s < 7) a_read<R, MT>(nh, nl, sb, at, s + 1);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(ah[mt], b, G[f][mt]);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) G[f][mt] = mfma(al[mt], b, G[f][mt]);
+            for (int mt = 0; mt < MT; ++mt) if (R > 16) G[f][mt] = mfma(al[mt], b, G[f][mt]);
             if (PER32 && (s & 1)) flush(f, s >> 1);
             b = bn;
             if (f == 1 && s < 7) {
@@ -373,13 +377,15 @@ DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
 #pragma unroll
         for (int f = 0; f < 2; ++f) {
             if (!PER32) flush(f, 0);
-            cur[f] = nxt[f];
+            if (hf == NH - 1)
+#pragma unroll
+                for (int i = 0; i < NH; ++i) cur[f][i] = nxt[f][i];
         }
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+        for (int r = 0; r < NR; ++r) {
             const uint32_t row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
             if (row >= n) continue;
             float *o = a.y + (uint64_t)s_row[row] * 2048 + 256 * cg + 64 * wave + col;
@@ -394,13 +400,14 @@ DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
 
 namespace {
 // The work items are (expert, pass) pairs in expert order: an expert with c pairs has
-// ceil(c / ROWS) passes of evenly many row tiles (real prompts crowd onto a few experts: every
+// ceil(c / R) passes of evenly many row tiles (real prompts crowd onto a few experts: every
 // pass is its own workgroup, so one expert's passes run side by side).  Every wave finds its
 // workgroup's item from the 128 counts (two a lane, a scan over the wave).
+template <int R>
 DEV bool expert_item(const uint32_t *cnt, uint32_t item, uint32_t &e, uint32_t &m0, uint32_t &n) {
     const int lane = threadIdx.x & 63;
     const uint2 c = reinterpret_cast<const uint2 *>(cnt)[lane];   // (zero past the last expert)
-    const uint32_t p0 = (c.x + ROWS - 1) / ROWS, p1 = (c.y + ROWS - 1) / ROWS;
+    const uint32_t p0 = (c.x + R - 1) / R, p1 = (c.y + R - 1) / R;
     uint32_t incl = p0 + p1;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -425,57 +432,71 @@ DEV bool expert_item(const uint32_t *cnt, uint32_t item, uint32_t &e, uint32_t &
 
 // Workgroup L of the grid (XCD L % 8, round-robin): the column groups of an item run on one
 // XCD, so the item's gathered rows are fetched into one L2.
-#define EXPERT_TILE(GROUPS)                                                                        \
+#define EXPERT_TILE(GROUPS, R)                                                                     \
     const uint32_t j_ = blockIdx.x >> 3, cg = j_ % (GROUPS);                                       \
     uint32_t e, m0, n;                                                                             \
-    if (!expert_item(a.cnt, (j_ / (GROUPS)) * 8 + (blockIdx.x & 7u), e, m0, n)) return;            \
+    if (!expert_item<R>(a.cnt, (j_ / (GROUPS)) * 8 + (blockIdx.x & 7u), e, m0, n)) return;         \
     const uint32_t *list = a.list + (uint64_t)e * QXP_LIST + m0;
 
+// Rows of a pass.  Gate/up takes 32: its about 16 vector instructions per 8 codes do not hide behind the
+// matrix instructions of another tile, and twice the workgroups fill the chip (512 tokens of a
+// prompt 81 us with 64 rows, 80 with 32; 149 tokens 66 and 55; 128 random rows 58 and 53; 64 rows of one
+// expert each 37 and 27).  At most 16 pairs run as one tile of hi and lo rows, half the matrix
+// work (128 random rows, 8 pairs an expert: 69 -> 58 us).
+constexpr int GU_ROWS = 32;
 template <int F>
 __global__ __launch_bounds__(256, 2) void qxp_gate_up(PfExperts a, PfTables P) {
-    EXPERT_TILE(6u)
+    EXPERT_TILE(6u, GU_ROWS)
     constexpr int NG = F == FMT_IQ2 ? 512 : 1024, NS = F == FMT_IQ2 ? 128 : 256;
     __shared__ uint2 s_grid[NG], s_sgn[NS];
-    __shared__ uint4 s_buf[2 * STAGE];   // two stages; the epilogue's rows of 132 floats
-    __shared__ uint32_t s_row[ROWS];
-    __shared__ float s_xs[ROWS];
+    __shared__ uint4 s_buf[2 * STAGE<GU_ROWS>];   // two stages; the epilogue's rows of 132 floats
+    __shared__ uint32_t s_row[GU_ROWS];
+    __shared__ float s_xs[GU_ROWS];
     for (int i = threadIdx.x; i < NG; i += 256) s_grid[i] = (F == FMT_IQ2 ? P.g2 : P.g2s)[i];
     for (int i = threadIdx.x; i < NS; i += 256) s_sgn[i] = (F == FMT_IQ2 ? P.sg7 : P.sg8)[i];
-    if (n <= 32) gu_pass<F, 1>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
-    else gu_pass<F, 2>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
+    if (n <= 16) gu_pass<F, 16>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
+    else gu_pass<F, 32>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
 }
 
-template <int F>
+// Down takes up to R = 32 or 64 (see down_rows)
+template <int F, int R>
 __global__ __launch_bounds__(256, 2) void qxp_down(PfExperts a, PfTables P) {
-    EXPERT_TILE(8u)
+    EXPERT_TILE(8u, R)
     constexpr int NG = F == FMT_IQ3S ? 512 : 256, NS = F == FMT_IQ3 ? 128 : F == FMT_IQ3S ? 256 : 1;
     __shared__ uint32_t s_grid[NG];
     __shared__ uint2 s_sgn[NS];
-    __shared__ uint4 s_buf[2 * STAGE];
-    __shared__ uint32_t s_row[ROWS];
-    __shared__ float s_hs[6 * ROWS];
+    __shared__ uint4 s_buf[2 * STAGE<R>];
+    __shared__ uint32_t s_row[R];
+    __shared__ float s_hs[6 * R];
     for (int i = threadIdx.x; i < NG; i += 256) s_grid[i] = (F == FMT_IQ3 ? P.g3 : F == FMT_IQ3S ? P.g3s : P.kv2)[i];
     if (NS > 1) for (int i = threadIdx.x; i < NS; i += 256) s_sgn[i] = (F == FMT_IQ3 ? P.sg7 : P.sg8)[i];
-    if (n <= 32) dn_pass<F, 1>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
-    else dn_pass<F, 2>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
+    if (n <= 16) dn_pass<F, 16>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
+    else if (n <= 32) dn_pass<F, 32>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
+    else if constexpr (R == 64) dn_pass<F, 64>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
 }
 
 extern "C" {
 // gate/up (IQ2_XS or IQ2_S) and down (IQ3_XXS, IQ3_S or IQ4_XS) of T tokens; the grid holds
-// the most items T tokens can make
-static uint32_t item_bound(const PfExperts &a, uint32_t T) {
-    const uint32_t pairs = T * QXG_TOPK, most = pairs / ROWS + (a.experts < pairs ? a.experts : pairs);
+// the most items T tokens can make with R rows a pass
+static uint32_t item_bound(const PfExperts &a, uint32_t T, uint32_t R) {
+    const uint32_t pairs = T * QXG_TOPK, most = pairs / R + (a.experts < pairs ? a.experts : pairs);
     return (most + 7) / 8 * 8;
 }
 void qxp_launch_gate_up(hipStream_t s, uint32_t type, const PfExperts &a, const PfTables &P, uint32_t T, Timer tm) {
-    const dim3 grid(6 * item_bound(a, T));
+    const dim3 grid(6 * item_bound(a, T, GU_ROWS));
     if (type == 22) qx_launch(qxp_gate_up<FMT_IQ2S>, grid, dim3(256), 0, s, tm, a, P);
     else qx_launch(qxp_gate_up<FMT_IQ2>, grid, dim3(256), 0, s, tm, a, P);
 }
+// Rows of down's passes: with up to 128 tokens, 32 spread a crowded expert over more workgroups (64 rows
+// of one expert each 20 -> 16 us, 37 tokens of a mixed model 20.6 -> 17.8); with more tokens the chip
+// is full and two tiles share the codes (300 tokens 33.6 us, 37.7 with 32 rows).
+static uint32_t down_rows(uint32_t T) { return T <= 128 ? 32 : 64; }
 void qxp_launch_down(hipStream_t s, uint32_t type, const PfExperts &a, const PfTables &P, uint32_t T, Timer tm) {
-    const dim3 grid(8 * item_bound(a, T));
-    if (type == 21) qx_launch(qxp_down<FMT_IQ3S>, grid, dim3(256), 0, s, tm, a, P);
-    else if (type == 23) qx_launch(qxp_down<FMT_IQ4>, grid, dim3(256), 0, s, tm, a, P);
-    else qx_launch(qxp_down<FMT_IQ3>, grid, dim3(256), 0, s, tm, a, P);
+    const uint32_t R = down_rows(T);
+    const dim3 grid(8 * item_bound(a, T, R));
+    auto *k = type == 21 ? (R == 32 ? qxp_down<FMT_IQ3S, 32> : qxp_down<FMT_IQ3S, 64>)
+              : type == 23 ? (R == 32 ? qxp_down<FMT_IQ4, 32> : qxp_down<FMT_IQ4, 64>)
+                           : (R == 32 ? qxp_down<FMT_IQ3, 32> : qxp_down<FMT_IQ3, 64>);
+    qx_launch(k, grid, dim3(256), 0, s, tm, a, P);
 }
 }
