@@ -1,11 +1,13 @@
-"""The output head's top-N picks over vocabularies at the edges of their split (128 slices, 2048
-keys a round of a block): fewer tokens than slices, a ragged last slice, one token more than a
-round a slice.  Exact against a stable sort of the logits of the same call.  Runs through the C
+"""The output head over vocabularies at the edges of its kernels' splits.  The logits (2 rows a wave,
+8192 a round of the launch) row by row against the oracle; the top-N picks (128 slices, 2048
+keys a round of a block: fewer tokens than slices, a ragged last slice, one token more than a
+round a slice) exact against a stable sort of the logits of the same call.  Runs through the C
 ABI (include/qxg.h)."""
 import numpy as np
 import pytest
 
 import qxg
+import qxo
 
 pytestmark = pytest.mark.gpu
 
@@ -24,5 +26,23 @@ def test_topn(vocab):
             _, lg, ids, vals = c.final_head(0 * x, n)   # all equal
             assert not lg.any() and np.array_equal(ids, np.arange(n)) and not vals.any()
     finally:
+        c.close()
+        m.close()
+
+
+@pytest.mark.parametrize("vocab", [1, 7, 8191, 8192, 8193, 16385, 3 * 8192 - 1])
+def test_logits_of_every_round(vocab):
+    m = qxg.MemModel(0, vocab, 8, False, True, seed=3)
+    c, om = qxg.Context(0), qxo.Model(m.path)
+    try:
+        c.load(m.path, verify=False)
+        x = np.random.default_rng(vocab).standard_normal(2048).astype(np.float32)
+        _, lg, _, _ = c.final_head(x, 1)
+        _, want, _, _ = om.final_head(x, vocab, 1)
+        # a row's error: 64 f32 sums of exact products and their tree, some 2^-24 each of values no
+        # larger than 10 times the rows' root mean square: within 1e-5 of the latter
+        assert np.abs(lg - want).max() <= 1e-5 * np.sqrt(np.mean(want.astype(np.float64) ** 2))
+    finally:
+        om.close()
         c.close()
         m.close()
