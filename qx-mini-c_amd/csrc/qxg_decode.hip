@@ -462,10 +462,12 @@ DEV float4 ldf4(const GLB uint8_t *b, uint32_t off) {
 // bytes land at lds + 16 i.  Issued as inline assembly so the compiler neither holds the
 // rows in registers across the stages in between nor orders the workgroup's other LDS
 // accesses behind the copy; the reader waits for it explicitly (wait_loads) at a point
-// where no later-issued load is outstanding.  Non-temporal, as every weight byte.
+// where no later-issued load is outstanding.  The copy needs one wait state after the
+// write of M0 and five after a vector instruction (readfirstlane) that wrote its base; the
+// compiler adds none inside the assembly.  Non-temporal, as every weight byte.
 DEV void dma16(const GLB uint8_t *base, uint32_t off, const void *lds) {
     const uint32_t l = (uint32_t)(uintptr_t)lds;   // low half of the flat address = LDS offset
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
 }
 // s_waitcnt vmcnt(0) as the builtin (0x0F70: vmcnt 0, expcnt and lgkmcnt unconstrained), which
 // the compiler's wait insertion takes into account (after an opaque asm wait it still assumed
@@ -477,11 +479,11 @@ DEV void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); __builtin_amdgcn_fen
 // agent-coherent): 16 bytes a lane, or 4 (lane i's at lds + 4 i).
 DEV void dma16_kv(const GLB uint8_t *base, uint32_t off, const void *lds) {
     const uint32_t l = (uint32_t)(uintptr_t)lds;
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 sc1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1 sc1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
 }
 DEV void dma4_kv(const GLB uint8_t *base, uint32_t off, const void *lds) {
     const uint32_t l = (uint32_t)(uintptr_t)lds;
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1 sc1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %0, %1 sc1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
 }
 
 // layer l's plane `id` (scalar arithmetic on the argument copy)

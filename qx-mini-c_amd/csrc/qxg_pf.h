@@ -31,10 +31,12 @@ DEV f16x zero16() {
     for (int i = 0; i < 16; ++i) z[i] = 0.0f;
     return z;
 }
-// lane i's 16 bytes at base + off land at lds + 16 i (lds the same in every lane)
+// lane i's 16 bytes at base + off land at lds + 16 i (lds the same in every lane).  The copy needs one
+// wait state after the write of M0 and five after a vector instruction (readfirstlane) that wrote
+// its base; the compiler adds none inside the assembly.
 DEV void dma16(const void *base, uint32_t off, const void *lds) {
     const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)lds);
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(l) : "memory", "m0");
 }
 // waits until at most N of the wave's loads (the youngest) are outstanding
 template <int N>
