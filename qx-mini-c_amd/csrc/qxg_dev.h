@@ -52,13 +52,11 @@ DEV uint32_t ldw1(const void *p) { return __builtin_nontemporal_load(reinterpret
 
 DEV int sdot4(uint32_t a, uint32_t b, int c) { return __builtin_amdgcn_sdot4((int)a, (int)b, c, false); }
 // a . b with a zero accumulator, the first of a chain: the three-operand form takes the 0
-// inline, where the accumulating form the compiler picks needs a register copy of 0 first.
+// inline, where the accumulating form needs a register copy of 0 first.  The compiler picks it
+// for a saturating product (only that form has one; four products do not reach the bound), and
+// keeps the wait states that a different opcode needs before it uses the result.
 // sdot4s: the chain's first link when z (a constant at each unrolled call site), else sdot4.
-DEV int sdot4z(uint32_t a, uint32_t b) {
-    int r;
-    asm("v_dot4_i32_i8 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
+DEV int sdot4z(uint32_t a, uint32_t b) { return __builtin_amdgcn_sdot4((int)a, (int)b, 0, true); }
 DEV int sdot4s(uint32_t a, uint32_t b, int c, bool z) { return z ? sdot4z(a, b) : sdot4(a, b, c); }
 DEV uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
 
