@@ -65,7 +65,7 @@ __global__ void qxp_qk(const float *, uint32_t, uint32_t, const float *, const f
 __global__ void qxp_attn(const float *, const int8_t *, const int8_t *, const float *, const float *, uint32_t, uint32_t,
                          uint32_t, uint32_t, float *, float2 *);
 __global__ void qxp_router(const float *, const float *, uint32_t, uint32_t, double *, uint32_t *);
-__global__ void qxp_route(const double *, uint32_t, uint32_t, double *, uint32_t *, uint32_t *);
+__global__ void qxp_route(const double *, uint32_t, uint32_t, double *, uint32_t *, uint4 *);
 __global__ void qxp_combine(const float *, const float *, const double *, float *, float *);
 __global__ void qxp_pack_ctx(const float *, const float2 *, uint32_t, uint32_t, uint8_t *, float *, float *);
 __global__ void qxp_dense_plane(uint32_t, const uint8_t *, const uint8_t *, const uint8_t *, uint32_t, uint32_t, uint32_t, uint8_t *,
@@ -183,7 +183,8 @@ struct qxg_ctx {
         uint8_t *XP = nullptr, *HP = nullptr;
         float2 *md = nullptr;
         double *lg = nullptr, *w = nullptr;
-        uint32_t *cnt = nullptr, *list = nullptr, *tokens = nullptr;
+        uint32_t *cnt = nullptr, *tokens = nullptr;
+        uint4 *sets = nullptr;
         std::vector<void *> all;
     } pf;
     // stage-probe outputs (allocated on first use)
@@ -844,7 +845,7 @@ bool prefill_ready(qxg_ctx *c, char *err, uint64_t n) {
               alloc((void **)&B.XP, T * PF_PITCH(4096)) && alloc((void **)&B.xscale, T * 4) && alloc((void **)&B.HP, PAIRS * PF_PITCH(768)) &&
               alloc((void **)&B.HS, PAIRS * 8 * 4) && alloc((void **)&B.Y, PAIRS * 2048 * 4) &&
               alloc((void **)&B.sums, T * 128 * 4) && alloc((void **)&B.dump, T * 2048 * 4) && alloc((void **)&B.lg, 4 * T * 128 * 8) && alloc((void **)&B.w, PAIRS * 8) &&
-              alloc((void **)&B.cnt, 128 * 4) && alloc((void **)&B.list, 128ull * QXP_LIST * 4) &&
+              alloc((void **)&B.cnt, 128 * 4) && alloc((void **)&B.sets, 128ull * QXP_SET * 16) &&
               alloc((void **)&B.tokens, T * 4);
     // codebooks: grids as magnitude bytes, sign bytes (0x80 where negative), the IQ4_XS byte table as fp16
     std::vector<uint8_t> g2(512 * 8), g2s(1024 * 8), g3(256 * 4), g3s(512 * 4), sg7(128 * 8), sg8(256 * 8);
@@ -914,10 +915,10 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, bool first, 
                        w.ffn_norm, T, B.X1, B.XN, B.XP, B.xscale);
     qx_launch(qxp_router, dim3((T + 15) / 16, (E + 15) / 16, 4), dim3(256), 0, s, timer_for(c, 12), (const float *)B.XN,
               w.router, T, E, B.lg, B.cnt);
-    hipLaunchKernelGGL(qxp_route, dim3((T + 15) / 16), dim3(1024), 0, s, (const double *)B.lg, T, E, B.w, B.cnt, B.list);
+    hipLaunchKernelGGL(qxp_route, dim3((T + 15) / 16), dim3(1024), 0, s, (const double *)B.lg, T, E, B.w, B.cnt, B.sets);
     PfExperts x{};
     x.w[0] = pf_mat(w.gate); x.w[1] = pf_mat(w.up); x.w[2] = pf_mat(w.down);
-    x.experts = E; x.cnt = B.cnt; x.list = B.list; x.xp = B.XP; x.xs = B.xscale; x.hp = B.HP; x.hs = B.HS;
+    x.experts = E; x.cnt = B.cnt; x.sets = B.sets; x.words = (T + 15) / 16; x.xp = B.XP; x.xs = B.xscale; x.hp = B.HP; x.hs = B.HS;
     x.h_pairs = w.down->type == 23; x.y = B.Y;
     qxp_launch_gate_up(s, w.gate->type, x, B.P, T, timer_for(c, 10));
     qxp_launch_down(s, w.down->type, x, B.P, T, timer_for(c, 11));

@@ -215,9 +215,9 @@ struct QxDArgs {
 // lines more than the values, so that rows do not lie at a power-of-two stride (measured neutral:
 // Q/K/V of 512 tokens 40.0 us without and 39.9 with them)
 #define PF_PITCH(K) (4u * (K) + 256u)
-// entries of one expert's pair list: every (token, rank) pair of a chunk (an expert takes a
-// token once, except where non-finite logits make the top-8 repeat it)
-#define QXP_LIST (QXP_MAX * QXG_TOPK)
+// 128-bit words of one expert's set of pairs: a bit per (token, rank) pair p = 8 * token + rank of a
+// chunk, 16 tokens a word
+#define QXP_SET (QXP_MAX / 16)
 
 // codebooks of the prefill GEMMs (built on the host at first use)
 struct PfTables {
@@ -259,7 +259,8 @@ struct PfExperts {
     PfMat w[3];                // gate, up, down: expert e's rows follow e * rows
     uint32_t experts;
     const uint32_t *cnt;       // pairs of each expert
-    const uint32_t *list;      // [expert][QXP_LIST] its pairs
+    const uint4 *sets;         // [expert][QXP_SET] its pairs
+    uint32_t words;            // words in use: of 16 tokens each
     const uint8_t *xp;         // packed normed activations, PF_PITCH(2048) a token
     const float *xs;           // per token: 1 / the row's power-of-two scale, 0 for a non-finite row
     uint8_t *hp;               // packed SwiGLU rows, PF_PITCH(768) a pair

@@ -59,10 +59,11 @@ DEV void stage_rows(const void *rows, const uint32_t (&off)[R / 8], uint32_t lin
 }
 // byte offset in its line of the chunk that lane copies in instruction i
 DEV uint32_t stage_chunk(int i, int lane) { return ((lane ^ (4 * i + (lane >> 4))) & 7) << 4; }
-template <int R>
-DEV void stage_offsets(uint32_t (&off)[R / 8], const uint32_t *s_row, uint32_t row_bytes, int lane) {
+// of the rows of pairs s_pair[], a row for 2^SHIFT pairs
+template <int R, int SHIFT>
+DEV void stage_offsets(uint32_t (&off)[R / 8], const uint32_t *s_pair, uint32_t row_bytes, int lane) {
 #pragma unroll
-    for (int i = 0; i < R / 8; ++i) off[i] = s_row[8 * i + (lane >> 3)] * row_bytes + stage_chunk(i, lane);
+    for (int i = 0; i < R / 8; ++i) off[i] = (s_pair[8 * i + (lane >> 3)] >> SHIFT) * row_bytes + stage_chunk(i, lane);
 }
 // A fragments of k-step s of the stage: lane's row l%32 of each tile, lane half l/32.  Of 16
 // rows there is one fragment, tile rows 0 .. 15 their hi and 16 .. 31 their lo halves: one

@@ -4,10 +4,10 @@
 // code that fp16 holds exactly, an activation row is scaled by a power of two and split
 // into fp16 hi + lo, the matrix cores accumulate in f32.  Here:
 //
-// Rows.  qxp_route lists each expert's (token, rank) pairs, p = 8 * token + rank; a
-// workgroup takes up to 32 or 64 of one expert's pairs and a range of its weight rows, and
-// forms each code once for them.  Activations are packed per token
-// (gate/up, gathered through the list while they are staged) and per pair (down, written
+// Rows.  qxp_route forms each expert's set of (token, rank) pairs, p = 8 * token + rank; a
+// workgroup takes up to 32 or 64 of one expert's pairs, in token order, and a range of its weight
+// rows, and forms each code once for them.  Activations are packed per token
+// (gate/up, gathered through the pairs while they are staged) and per pair (down, written
 // by gate/up's epilogue); no copy of them is sorted or padded by expert.
 //
 // Order of K.  Which 8 values a lane half holds is free as long as A and B agree: a lane
@@ -45,6 +45,35 @@ DEV h2v odd_mul(uint32_t n) {   // (2 n + 1) * 2^11, n < 16: exact
     return h2v{f, f};
 }
 constexpr float CODE_SCALE = 8192.0f;   // 2^13: the codes above are at 2^-13
+
+// the sum of v over lanes 0 .. lane
+DEV uint32_t wave_prefix(uint32_t v) {
+    int s = (int)v;
+    s += __builtin_amdgcn_update_dpp(0, s, 0x111, 0xf, 0xf, false);   // row_shr 1, 2, 4, 8
+    s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xf, 0xf, false);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xf, 0xf, false);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xf, 0xf, false);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xa, 0xf, false);   // row 0's and 2's sum to the row above
+    s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xc, 0xf, false);   // the lower half's to the upper
+    return (uint32_t)s;
+}
+// Pairs m0 .. m0 + n - 1 of expert e in token order (n at most R), the last repeated up to R.  One whole
+// wave; lane l looks at tokens 8 l .. 8 l + 7.
+template <int R>
+DEV void pass_pairs(const PfExperts &a, uint32_t e, uint32_t m0, uint32_t n, uint32_t *s_pair) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint2 m = make_uint2(0u, 0u);
+    if (lane < 2 * a.words) m = reinterpret_cast<const uint2 *>(a.sets + e * QXP_SET)[lane];
+    const uint32_t c = __popc(m.x) + __popc(m.y);
+    uint32_t at = wave_prefix(c) - c - m0;   // (wraps below m0)
+#pragma unroll 1
+    for (uint64_t w = (uint64_t)m.y << 32 | m.x; w; w &= w - 1, ++at)
+        if (at < n) s_pair[at] = 64 * lane + (uint32_t)__builtin_ctzll(w);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (lane >= n && lane < R) s_pair[lane] = s_pair[n - 1];
+}
 
 DEV uint32_t word_at(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 DEV uint32_t byte_at(const uint4 &v, int i) { return (word_at(v, i >> 2) >> (8 * (i & 3))) & 255u; }
@@ -125,23 +154,20 @@ DEV float div_ge1(float x, float y) {
 DEV float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }   // 2^e, -126 <= e <= 127
 
 template <int F, int R>
-DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *list, uint32_t n, const uint2 *grid,
-                 const uint2 *sgn, uint4 *buf, uint32_t *s_row, float *s_xs) {
+DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, uint32_t m0, uint32_t n, const uint2 *grid,
+                 const uint2 *sgn, uint4 *buf, uint32_t *s_pair, float *s_xs) {
     constexpr int NR = R > 16 ? 16 : 8;   // result registers of a tile, hi and lo added
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), h = lane >> 5, col = lane & 31;
     const uint32_t bi = (e * QXG_FFN + 128 * cg + 32 * wave + col) * 8;   // tiles 0 and 1: this row of gate and of up
     GuBlk<F> cur[2], nxt[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f) gu_load(cur[f], a.w[f], bi, h);
-    if (tid < R) {
-        const uint32_t t = list[min((uint32_t)tid, n - 1)] >> 3;
-        s_row[tid] = t;
-        s_xs[tid] = a.xs[t];
-    }
-    __syncthreads();   // the rows' tokens, and the tables
+    if (wave == 0) pass_pairs<R>(a, e, m0, n, s_pair);
+    __syncthreads();   // the pairs, and the tables
     uint32_t off[R / 8];
-    stage_offsets<R>(off, s_row, PF_PITCH(2048), lane);
+    stage_offsets<R, 3>(off, s_pair, PF_PITCH(2048), lane);
     stage_rows<R>(a.xp, off, 0, buf, wave);
+    if (tid < R) s_xs[tid] = a.xs[s_pair[tid] >> 3];   // (read behind the loop's barriers)
     const ALane at = a_lane<R>(lane);
     f16x acc[2] = {zero16(), zero16()};
 #pragma unroll 1
@@ -211,7 +237,7 @@ DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
         int sh = 140 - (int)(__float_as_uint(mx) >> 23);   // mx 2^sh in [2^13, 2^14) (zero and subnormal: 2^100)
         sh = sh > 100 ? 100 : sh < -100 ? -100 : sh;
         if (row < n) {
-            const uint32_t pr = list[row];
+            const uint32_t pr = s_pair[row];
             const float sc = exp2i(sh);
             h8v hi, lo;
 #pragma unroll
@@ -280,8 +306,8 @@ DEV float dn_scale(const DnHalf<FMT_IQ4> &w, int half, int i) {   // sub-block i
 }
 
 template <int F, int R>
-DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *list, uint32_t n, const uint32_t *grid,
-                 const uint2 *sgn, uint4 *buf, uint32_t *s_row, float *s_hs) {
+DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, uint32_t m0, uint32_t n, const uint32_t *grid,
+                 const uint2 *sgn, uint4 *buf, uint32_t *s_pair, float *s_hs) {
     constexpr int MT = R > 32 ? 2 : 1, NR = R > 16 ? 16 : 8;   // tiles; result registers of a tile, hi and lo added
     // half blocks loaded at once: both where the registers allow it (read apart, a block's lines came
     // twice from beyond L2: 98 MB for 47 of weights; IQ4_XS has whole lines per half)
@@ -296,14 +322,14 @@ DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
     for (int f = 0; f < 2; ++f)
 #pragma unroll
         for (int i = 0; i < NH; ++i) dn_load(cur[f][i], a.w[2], bi[f], i, h);
-    if (tid < R) s_row[tid] = list[min((uint32_t)tid, n - 1)];
-    __syncthreads();   // the rows' pairs, and the tables
+    if (wave == 0) pass_pairs<R>(a, e, m0, n, s_pair);
+    __syncthreads();   // the pairs, and the tables
     uint32_t off[R / 8];
-    stage_offsets<R>(off, s_row, PF_PITCH(768), lane);
+    stage_offsets<R, 0>(off, s_pair, PF_PITCH(768), lane);
     stage_rows<R>(a.hp, off, 0, buf, wave);
     const ALane at = a_lane<R>(lane);
     for (int i = tid; i < 6 * R; i += 256)   // the rows' scales of each 128 values
-        s_hs[i] = a.hs[(uint64_t)s_row[i % R] * 8 + i / R];
+        s_hs[i] = a.hs[(uint64_t)s_pair[i % R] * 8 + i / R];
     f16x acc[2][MT];
 #pragma unroll
     for (int f = 0; f < 2; ++f)
@@ -388,7 +414,7 @@ DEV void dn_pass(const PfExperts &a, uint32_t e, uint32_t cg, const uint32_t *li
         for (int r = 0; r < NR; ++r) {
             const uint32_t row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
             if (row >= n) continue;
-            float *o = a.y + (uint64_t)s_row[row] * 2048 + 256 * cg + 64 * wave + col;
+            float *o = a.y + (uint64_t)s_pair[row] * 2048 + 256 * cg + 64 * wave + col;
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
                 const float y = acc[f][mt][r];
@@ -408,12 +434,7 @@ DEV bool expert_item(const uint32_t *cnt, uint32_t item, uint32_t &e, uint32_t &
     const int lane = threadIdx.x & 63;
     const uint2 c = reinterpret_cast<const uint2 *>(cnt)[lane];   // (zero past the last expert)
     const uint32_t p0 = (c.x + R - 1) / R, p1 = (c.y + R - 1) / R;
-    uint32_t incl = p0 + p1;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t v = __shfl_up(incl, o);
-        if (lane >= o) incl += v;
-    }
+    const uint32_t incl = wave_prefix(p0 + p1);
     const uint64_t past = __ballot(incl > item);
     if (!past) return false;
     const int l = __builtin_ctzll(past);
@@ -435,8 +456,7 @@ DEV bool expert_item(const uint32_t *cnt, uint32_t item, uint32_t &e, uint32_t &
 #define EXPERT_TILE(GROUPS, R)                                                                     \
     const uint32_t j_ = blockIdx.x >> 3, cg = j_ % (GROUPS);                                       \
     uint32_t e, m0, n;                                                                             \
-    if (!expert_item<R>(a.cnt, (j_ / (GROUPS)) * 8 + (blockIdx.x & 7u), e, m0, n)) return;         \
-    const uint32_t *list = a.list + (uint64_t)e * QXP_LIST + m0;
+    if (!expert_item<R>(a.cnt, (j_ / (GROUPS)) * 8 + (blockIdx.x & 7u), e, m0, n)) return;
 
 // Rows of a pass.  Gate/up takes 32: its about 16 vector instructions per 8 codes do not hide behind the
 // matrix instructions of another tile, and twice the workgroups fill the chip (512 tokens of a
@@ -450,12 +470,12 @@ __global__ __launch_bounds__(256, 2) void qxp_gate_up(PfExperts a, PfTables P) {
     constexpr int NG = F == FMT_IQ2 ? 512 : 1024, NS = F == FMT_IQ2 ? 128 : 256;
     __shared__ uint2 s_grid[NG], s_sgn[NS];
     __shared__ uint4 s_buf[2 * STAGE<GU_ROWS>];   // two stages; the epilogue's rows of 132 floats
-    __shared__ uint32_t s_row[GU_ROWS];
+    __shared__ uint32_t s_pair[GU_ROWS];
     __shared__ float s_xs[GU_ROWS];
     for (int i = threadIdx.x; i < NG; i += 256) s_grid[i] = (F == FMT_IQ2 ? P.g2 : P.g2s)[i];
     for (int i = threadIdx.x; i < NS; i += 256) s_sgn[i] = (F == FMT_IQ2 ? P.sg7 : P.sg8)[i];
-    if (n <= 16) gu_pass<F, 16>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
-    else gu_pass<F, 32>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_xs);
+    if (n <= 16) gu_pass<F, 16>(a, e, cg, m0, n, s_grid, s_sgn, s_buf, s_pair, s_xs);
+    else gu_pass<F, 32>(a, e, cg, m0, n, s_grid, s_sgn, s_buf, s_pair, s_xs);
 }
 
 // Down takes up to R = 32 or 64 (see down_rows)
@@ -466,13 +486,13 @@ __global__ __launch_bounds__(256, 2) void qxp_down(PfExperts a, PfTables P) {
     __shared__ uint32_t s_grid[NG];
     __shared__ uint2 s_sgn[NS];
     __shared__ uint4 s_buf[2 * STAGE<R>];
-    __shared__ uint32_t s_row[R];
+    __shared__ uint32_t s_pair[R];
     __shared__ float s_hs[6 * R];
     for (int i = threadIdx.x; i < NG; i += 256) s_grid[i] = (F == FMT_IQ3 ? P.g3 : F == FMT_IQ3S ? P.g3s : P.kv2)[i];
     if (NS > 1) for (int i = threadIdx.x; i < NS; i += 256) s_sgn[i] = (F == FMT_IQ3 ? P.sg7 : P.sg8)[i];
-    if (n <= 16) dn_pass<F, 16>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
-    else if (n <= 32) dn_pass<F, 32>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
-    else if constexpr (R == 64) dn_pass<F, 64>(a, e, cg, list, n, s_grid, s_sgn, s_buf, s_row, s_hs);
+    if (n <= 16) dn_pass<F, 16>(a, e, cg, m0, n, s_grid, s_sgn, s_buf, s_pair, s_hs);
+    else if (n <= 32) dn_pass<F, 32>(a, e, cg, m0, n, s_grid, s_sgn, s_buf, s_pair, s_hs);
+    else if constexpr (R == 64) dn_pass<F, 64>(a, e, cg, m0, n, s_grid, s_sgn, s_buf, s_pair, s_hs);
 }
 
 extern "C" {

@@ -649,20 +649,19 @@ extern "C" __global__ __launch_bounds__(256) void qxp_router(const float *xn, co
 }
 
 // Top-8 experts and renormalised weights per token (the decode path's selection,
-// src/qx_format.c:5265-5285), and the experts' pair lists: pair p = 8 t + rank joins list e at
-// the next free place.  The order within a list varies from run to run; a pair's row of the
-// expert GEMMs does not depend on its place.  A workgroup takes 16 tokens, one a wave, counts
-// its pairs by expert in LDS and claims the list places with one atomic per expert (pairs that
-// each took their place themselves waited on the crowded experts' counters: 20 us).
+// src/qx_format.c:5265-5285), and the experts' pairs.  A workgroup takes 16 tokens, one a wave, and
+// writes its word of every expert's set (bit p % 128 of pair p = 8 t + rank) and adds the words'
+// bits to the counts.  The sets come out the same whatever the order of the workgroups; the expert
+// GEMMs take the pairs in token order.  (Lists whose places were claimed by atomics put a pair into
+// another pass from run to run, and a pass of at most 16 rows rounds differently.)
 extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logits, uint32_t T, uint32_t experts,
-                                                             double *wts, uint32_t *cnt, uint32_t *list) {
-    __shared__ uint32_t s_n[128], s_at[128];
+                                                             double *wts, uint32_t *cnt, uint4 *sets) {
+    __shared__ uint4 s_set[128];
     const int tid = threadIdx.x, lane = tid & 63;
-    if (tid < 128) s_n[tid] = 0u;
+    if (tid < 128) s_set[tid] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     const int E = (int)experts;
     const uint32_t t = blockIdx.x * 16 + wave_id();
-    uint32_t e = 0, place = 0;
     if (t < T) {   // whole wave
         double q[4][2];   // the quarters of K
 #pragma unroll
@@ -676,6 +675,7 @@ extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logit
         double w[QXG_TOPK];
         wave_top8(l0, l1, E, id, w);
         double wl = 0.0;
+        uint32_t e = 0;
 #pragma unroll
         for (int q = 0; q < QXG_TOPK; ++q)
             if (lane == q) {
@@ -684,13 +684,17 @@ extern "C" __global__ __launch_bounds__(1024) void qxp_route(const double *logit
             }
         if (lane < QXG_TOPK) {
             wts[t * 8 + lane] = wl;
-            place = atomicAdd(&s_n[e], 1u);
+            const uint32_t bit = 8 * wave_id() + lane;
+            atomicOr(reinterpret_cast<uint32_t *>(&s_set[e]) + (bit >> 5), 1u << (bit & 31));
         }
     }
     __syncthreads();
-    if (tid < 128 && s_n[tid]) s_at[tid] = atomicAdd(&cnt[tid], s_n[tid]);
-    __syncthreads();
-    if (t < T && lane < QXG_TOPK) list[(uint64_t)e * QXP_LIST + s_at[e] + place] = t * 8 + lane;
+    if (tid < 128) {
+        const uint4 m = s_set[tid];
+        sets[tid * QXP_SET + blockIdx.x] = m;
+        const uint32_t n = __popc(m.x) + __popc(m.y) + __popc(m.z) + __popc(m.w);
+        if (n) atomicAdd(&cnt[tid], n);
+    }
 }
 
 // The last layer's output x = x1 + its combined experts (moe_dump: the expert sum alone)
