@@ -329,16 +329,18 @@ extern "C" __global__ __launch_bounds__(640) void qxp_qk(const float *parts, uin
 //           the hi and the lo products summed apart (two chains of matrix instructions);
 //           times ks[pos]; positions past the token masked in the chunks that hold any;
 //   weights e = 2^(score * scale - m), pv = e * vs[pos] split hi + lo under a power-of-two
-//           scale of the column;
-//   context C[dim][col] += V8^T[dim][pos] . pv[pos][col] (A = V codes from a transposed LDS copy
-//           of the chunk), accumulated by the matrix cores.
+//           scale of the column in this chunk (from its largest |pv|, so that a chunk of small
+//           weights behind a large one keeps all its bits);
+//   context C[dim][col] = V8^T[dim][pos] . pv[pos][col] (A = V codes from a transposed LDS copy
+//           of the chunk), added to the running context at the scale's inverse.
 // The result registers of the score product are exactly the k layout the context product's B
 // operand needs (lane l: column l%32, positions 8(r/4) + 4(l/32) + r%4 of register r), so the
 // weights never leave the lane.  The softmax's vector work bounds this kernel, about 17 issue
 // slots a score against 64 matrix cycles per 32 of them, so: m is the running maximum only to
-// within a factor 2^8 and the column's scale only to within 2^5 of its largest weight, and the
-// context is rescaled (64 multiplies) only in the chunks that leave those; the exponent is base
-// 2; the next chunk's K and V rows are loaded while the current one is worked on.  The
+// within a factor 2^8, and the context is rescaled (64 multiplies) only in the chunks that leave
+// that; the exponent is base 2; the next chunk's K and V rows are loaded while the current one is
+// worked on.  (One scale of the column over all chunks spared the 64 additions, which measured
+// the same: 112 us for 512 at 3500 either way, and lost the bits of later, smaller weights.)  The
 // waves' states are merged in LDS, the runs' by qxp_pack_ctx.  (One run, the context rescaled at every
 // chunk: 60 us for 37 tokens at position 2100, now 16; 139 for 512 at 3500, now 105.)
 namespace {
@@ -440,7 +442,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
     }
     __syncthreads();
     const float sf = s_sf[col];
-    float m = -INFINITY, den = 0.0f, psc = 1.0f, top = 0.0f;   // top: the largest weight * vs so far, at the current m
+    float m = -INFINITY, den = 0.0f;
     f16x acc[4];
 #pragma unroll
     for (int d = 0; d < 4; ++d) acc[d] = zero16();
@@ -500,62 +502,51 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
         f4x v4[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) v4[q] = *reinterpret_cast<const f4x *>(&s_vs[wave][8 * q + 4 * h]);
-        float e[16], pv[16], pmx = 0.0f;
-        auto weigh = [&]() {
-            const float mm = m == -INFINITY ? 0.0f : m;
-            pmx = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                e[r] = exp2_fast(fmaf(sc[r], sf, -mm));
-                pv[r] = e[r] * v4[r >> 2][r & 3];
-                pmx = fmaxf(pmx, pv[r]);
-            }
-            if (tail) {   // (a masked position's V scale does not count, whatever it is)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) pv[r] = sc[r] == -INFINITY ? 0.0f : pv[r];
-            }
-            pmx = fmaxf(pmx, __shfl_xor(pmx, 32));
-        };
         const bool grow = cmax > m + 8.0f;
-        if (__ballot(grow) == 0) weigh();
-        if (__ballot(grow || pmx * psc > 32768.0f) != 0) {   // (whole wave)
+        if (__ballot(grow) != 0) {   // (whole wave)
             const float mn = fmaxf(m, cmax);
             const float alpha = mn == -INFINITY || m == -INFINITY ? (m == mn ? 1.0f : 0.0f) : exp2_fast(m - mn);
             m = mn;
-            weigh();
-            top = fmaxf(top * alpha, pmx);
-            const float pn = pow2_scale(top, 10), f = alpha * (pn / psc);   // a power of two times alpha
-            psc = pn;
             den *= alpha;
 #pragma unroll
             for (int d = 0; d < 4; ++d)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[d][r] *= f;
+                for (int r = 0; r < 16; ++r) acc[d][r] *= alpha;
         }
-        top = fmaxf(top, pmx);
+        const float mm = m == -INFINITY ? 0.0f : m;
+        float e[16], pv[16], pmx = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            e[r] = exp2_fast(fmaf(sc[r], sf, -mm));
+            pv[r] = e[r] * v4[r >> 2][r & 3];
+        }
+        if (tail) {   // (a masked position's V scale does not count, whatever it is)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) pv[r] = sc[r] == -INFINITY ? 0.0f : pv[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) pmx = fmaxf(pmx, fabsf(pv[r]));
+        pmx = fmaxf(pmx, __shfl_xor(pmx, 32));
+        const float psc = pow2_scale(pmx, 15), pinv = 1.0f / psc;   // (powers of two: exact)
 #pragma unroll
         for (int r = 0; r < 16; ++r) den += e[r];
         uint4 phi[2], plo[2];
         split8(pv, psc, phi[0], plo[0]);
         split8(pv + 8, psc, phi[1], plo[1]);
-        // context: per 32-dim tile, C[dim][col] += V8^T . pv
+        // context: per 32-dim tile, C[dim][col] = V8^T . pv
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
+            f16x c = zero16();
             const uint32_t *row = vt + (32 * d + col) * 9;
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) {
                 const uint4 vf = i8x8_to_f16(row[4 * s2 + h], row[4 * s2 + 2 + h]);
-                acc[d] = mfma(vf, phi[s2], acc[d]);
-                acc[d] = mfma(vf, plo[s2], acc[d]);
+                c = mfma(vf, phi[s2], c);
+                c = mfma(vf, plo[s2], c);
             }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[d][r] = fmaf(c[r], pinv, acc[d][r]);
         }
-    }
-    {
-        const float inv = 1.0f / psc;   // (a power of two: exact)
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[d][r] *= inv;
     }
     // merge the 4 waves' (max, denominator, context) per column: 2+3 into 0+1, then 1 into 0
     den += __shfl_xor(den, 32);

@@ -1,9 +1,14 @@
-"""Batched prefill where its result could hang on more than the inputs: calls repeated bit for
-bit.  Runs through the C ABI (include/qxg.h)."""
+"""Batched prefill where its result could hang on more than the inputs, or lose bits that a norm
+over whole rows does not show: calls repeated bit for bit, attention heads whose context comes
+from small weights or small V scales alone.
+Models are generated files with a few tensors rewritten, so that the part in question stands
+alone in the output; the oracle reads the same files.  Runs through the C ABI (include/qxg.h)."""
 import numpy as np
 import pytest
 
 import qxg
+import qxo
+from helpers import REL_L2, rel_l2, seeded_kv
 
 pytestmark = pytest.mark.gpu
 
@@ -13,6 +18,35 @@ def ctx():
     c = qxg.Context(0)
     yield c
     c.close()
+
+
+def tensors(path):
+    """{name: (dims, writable bytes)} of a QXF1 file."""
+    data = np.memmap(path, np.uint8, "r+")
+    count, at = int(data[16:20].view(np.uint32)[0]), int(data[24:32].view(np.uint64)[0])
+    found = {}
+    for i in range(count):
+        e = data[at + 208 * i:at + 208 * (i + 1)]
+        dims, (offset, size) = e[112:144].view(np.uint64), e[144:160].view(np.uint64)
+        found[bytes(e[:96]).split(b"\0")[0].decode()] = ([int(v) for v in dims], data[int(offset):int(offset + size)])
+    return found
+
+
+def one_layer(path, **kw):
+    qxg.generate_model(path, layers=1, vocab=256, experts=16, embedding=False, head=False, **kw)
+    return tensors(path)
+
+
+def oracle_q(om, x, pos):
+    """The roped q heads [32, 128] of one residual row (in double)."""
+    w = lambda name: om.tensor("blk.0." + name)[2].view(np.float32).astype(np.float64)
+    xd = x.astype(np.float64)
+    xn = (xd / np.sqrt((xd * xd).mean() + 1e-6) * w("attn_norm.weight")).astype(np.float32)
+    q = qxo.matvec(23, om.tensor("blk.0.attn_q.weight")[2], 4096, 2048, xn).reshape(32, 128).astype(np.float64)
+    q = q / np.sqrt((q * q).mean(1, keepdims=True) + 1e-6) * w("attn_q_norm.weight")
+    angle = pos * 1e6 ** (-np.arange(64) / 64)
+    c, s = np.cos(angle), np.sin(angle)
+    return np.concatenate([q[:, :64] * c - q[:, 64:] * s, q[:, :64] * s + q[:, 64:] * c], 1)
 
 
 @pytest.mark.parametrize("mix,layer", [(0, 0), (1, 1), (1, 2), (1, 3)])
@@ -31,3 +65,62 @@ def test_calls_repeat(ctx, tmp_path, mix, layer, n):
         again = ctx.prefill_layer(layer, 0, x)
         for name, a, b in zip(("ffn_inp", "moe", "out"), first, again):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (name, np.flatnonzero((a != b).any(1)))
+
+
+def kv_head_model(path, kv):
+    """A layer whose attention output is what kv head `kv`'s eight q heads contribute (the O
+    matrix's blocks of other heads scaled by 0) and whose own V rows are 0."""
+    t = one_layer(path, seed=29)
+    o = t["blk.0.attn_output.weight"][1].reshape(2048, 16, 136)
+    o[:, np.arange(16) // 4 != kv, :2] = 0
+    t["blk.0.attn_v.weight"][1].reshape(-1, 136)[:, :2] = 0
+
+
+def attention_rows(ctx, path, om, p0, x, rows):
+    """Each row's distance from the oracle's over the same cache rows."""
+    n = len(x)
+    ctx.load(path, verify=False)
+    ctx.kv_create(1, p0 + n)
+    ctx.kv_write(0, 0, *rows)
+    fi, _, _ = ctx.prefill_layer(0, p0, x)
+    okv = qxo.KV(1, p0 + n)
+    okv.k[0], okv.v[0], okv.ks[0], okv.vs[0] = ctx.kv_read(0, 0, p0 + n)
+    return [rel_l2(fi[t], x[t] + qxo.attention_layer_given_row(om, 0, p0 + t, okv, x[t])[0]) for t in range(n)]
+
+
+@pytest.mark.parametrize("n,lead", [(1, 12), (3, 18), (3, 40)])
+def test_attention_behind_a_sink(ctx, tmp_path, n, lead):
+    """A first position whose score leads by `lead` holds zeros, so that the context is what a later
+    chunk of the same wave adds with weights of e^-lead."""
+    p, p0, kv = tmp_path / "m.qxf", 200, 1
+    kv_head_model(p, kv)
+    om = qxo.Model(p)
+    x = np.random.default_rng(7 + n).standard_normal((n, 2048)).astype(np.float32)
+    k, v, ks, vs = seeded_kv(41, p0)
+    q = np.concatenate([oracle_q(om, x[t], p0 + t)[8 * kv:8 * kv + 8] for t in range(n)])
+    row = np.linalg.lstsq(q, np.ones(len(q)), rcond=None)[0]   # the shortest row with the same score for all of them
+    codes = np.round(row / np.abs(row).max() * 127)
+    k[0, 128 * kv:128 * kv + 128] = codes
+    ks[0] = lead * np.sqrt(128) / (q @ codes).mean()
+    v[:] = 0   # (other heads too: the context row is packed under one scale)
+    v[128:160, 128 * kv:128 * kv + 128] = np.random.default_rng(5).integers(-127, 128, (32, 128))
+    vs *= np.float32(np.exp(lead))
+    errs = attention_rows(ctx, p, om, p0, x, (k, v, ks, vs))
+    om.close()
+    assert max(errs) <= REL_L2, errs
+
+
+@pytest.mark.parametrize("scale", [1e-2, 1e-4, -1e-4])
+def test_attention_after_zero_v_scales(ctx, tmp_path, scale):
+    """Whole chunks of V scales 0 (as unwritten positions hold), then small ones (or negative ones, which
+    a cache may be given)."""
+    p, p0, kv = tmp_path / "m.qxf", 250, 2
+    kv_head_model(p, kv)
+    om = qxo.Model(p)
+    x = 1e-3 * np.random.default_rng(9).standard_normal((2, 2048)).astype(np.float32)
+    k, v, ks, vs = seeded_kv(43, p0)
+    vs[:128] = 0
+    vs[128:] *= scale * 127
+    errs = attention_rows(ctx, p, om, p0, x, (k, v, ks, vs))
+    om.close()
+    assert max(errs) <= REL_L2, errs
