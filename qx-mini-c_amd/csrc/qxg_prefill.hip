@@ -18,6 +18,7 @@
 // the row result is divided by s.  The GEMMs are in qxg_pf_dense.hip (Q/K/V, O) and
 // qxg_pf_experts.hip; here are the stages between them.
 #include "qxg_pf.h"
+#include <cfloat>
 
 // ================================================================= element-wise stages
 // Q4_K embedding rows of tokens[0..T) (src/qx_format.c:3759-3793); block per token.
@@ -441,7 +442,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
         if (seg == 0) s_sf[c] = (float)(1.4426950408889634 / ((double)sc * sqrt(128.0)));
     }
     __syncthreads();
-    const float sf = s_sf[col];
+    const float sf = s_sf[col], sf_most = wave_max_f(sf);
     float m = -INFINITY, den = 0.0f;
     f16x acc[4];
 #pragma unroll
@@ -452,7 +453,9 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
         const uint32_t pb = ci * 32;
         // this chunk's rows: scales and V^T to LDS (a wave's own), K stays in registers
         const uint4 kq[4] = {nx.k[0], nx.k[1], nx.k[2], nx.k[3]};
-        const bool big = __ballot(!(fabsf(nx.ks) < 1.1529215e18f)) != 0;   // 2^60: a score could overflow
+        // a score is a sum below 2^28 times ks and sf: beyond 2^20 the rounding of the maximum, which the
+        // weights' fma does not repeat, would show, beyond 2^128 the score itself is lost
+        const bool big = __ballot(!(fabsf(nx.ks) * fmaxf(sf_most, 0x1p-98f) < 0x1p-8f)) != 0;
         if (lane < 32) {
             s_ks[wave][lane] = nx.ks;
             s_vs[wave][lane] = nx.vs;
@@ -480,16 +483,23 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
             if (s & 1) asm volatile("" ::: "memory");   // later q reads stay below: hoisted together they spill
         }
         // register r: position pb + 8(r/4) + 4h + r%4
-        float sc[16], cmax = -INFINITY;
+        float sc[16], cmax = -INFINITY, f = sf;   // scores, still to be multiplied by f
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const f4x k4 = *reinterpret_cast<const f4x *>(&s_ks[wave][8 * q + 4 * h]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) sc[4 * q + r] = (sh[4 * q + r] + sl[4 * q + r]) * k4[r];
         }
-        if (big) {   // non-finite scores are 0 (src/qx_format.c:5137-5139)
+        if (big) {
+            // rounded once, so that the largest has weight 1.  The reference's scores are doubles: one beyond
+            // f32 stays the largest there is; where K itself is not finite it is 0 (src/qx_format.c:5137-5139)
+            f = 1.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sc[r] = isfinite(sc[r] * sf) ? sc[r] : 0.0f;
+            for (int r = 0; r < 16; ++r) {
+                const float k = s_ks[wave][8 * (r >> 2) + 4 * h + (r & 3)];
+                const double v = (double)(sh[r] + sl[r]) * ((double)k * (double)sf);
+                sc[r] = fabsf(k) <= FLT_MAX / 127.0f ? (float)fmin(fmax(v, -3.0e38), 3.0e38) : 0.0f;
+            }
         }
         const bool tail = pb + 31 > p0 + t0;   // the chunk holds positions past the first token
         if (tail) {
@@ -498,7 +508,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) cmax = fmaxf(cmax, sc[r]);
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 32)) * sf;
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32)) * f;
         f4x v4[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) v4[q] = *reinterpret_cast<const f4x *>(&s_vs[wave][8 * q + 4 * h]);
@@ -517,7 +527,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
         float e[16], pv[16], pmx = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            e[r] = exp2_fast(fmaf(sc[r], sf, -mm));
+            e[r] = exp2_fast(fmaf(sc[r], f, -mm));
             pv[r] = e[r] * v4[r >> 2][r & 3];
         }
         if (tail) {   // (a masked position's V scale does not count, whatever it is)

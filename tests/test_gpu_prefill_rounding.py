@@ -1,6 +1,6 @@
 """Batched prefill where its result could hang on more than the inputs, or lose bits that a norm
 over whole rows does not show: calls repeated bit for bit, attention heads whose context comes
-from small weights or small V scales alone.
+from small weights or small V scales alone, scores near and beyond f32's range.
 Models are generated files with a few tensors rewritten, so that the part in question stands
 alone in the output; the oracle reads the same files.  Runs through the C ABI (include/qxg.h)."""
 import numpy as np
@@ -121,6 +121,29 @@ def test_attention_after_zero_v_scales(ctx, tmp_path, scale):
     k, v, ks, vs = seeded_kv(43, p0)
     vs[:128] = 0
     vs[128:] *= scale * 127
+    errs = attention_rows(ctx, p, om, p0, x, (k, v, ks, vs))
+    om.close()
+    assert max(errs) <= REL_L2, errs
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.9 * 2.0 ** 60])
+def test_attention_large_scores(ctx, tmp_path, scale):
+    """Scores near 2^70, and one of a query and a K scale that are each far inside f32's range while their
+    product is not: finite in the oracle's double, it outweighs every other position.  A non-finite K
+    scale's score is 0."""
+    p, p0, kv = tmp_path / "m.qxf", 70, 0
+    kv_head_model(p, kv)
+    t = tensors(p)
+    t["blk.0.attn_q_norm.weight"][1].view(np.float32)[:] = 2.0 ** 64
+    om = qxo.Model(p)
+    x = np.random.default_rng(11).standard_normal((1, 2048)).astype(np.float32)
+    k, v, ks, vs = seeded_kv(47, p0)
+    q = oracle_q(om, x[0], p0)[8 * kv:8 * kv + 8]
+    row = np.linalg.lstsq(q, np.ones(8), rcond=None)[0]
+    k[40, 128 * kv:128 * kv + 128] = np.round(row / np.abs(row).max() * 127)
+    ks[40] = scale
+    ks[3] = np.nan
+    ks[4] = np.inf
     errs = attention_rows(ctx, p, om, p0, x, (k, v, ks, vs))
     om.close()
     assert max(errs) <= REL_L2, errs
