@@ -143,14 +143,6 @@ DEV void gu_half(const GuBlk<F> (&w)[2], int half, const uint4 *buf, const ALane
     }
 }
 
-// x / y for finite y >= 1 by the hardware reciprocal, one Newton step and a residual
-// correction: within an f32 rounding of the quotient, at a third of the exact division's cost
-DEV float div_ge1(float x, float y) {
-    float r = __builtin_amdgcn_rcpf(y);
-    r = fmaf(fmaf(-y, r, 1.0f), r, r);
-    const float q = x * r;
-    return fmaf(fmaf(-q, y, x), r, q);
-}
 DEV float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }   // 2^e, -126 <= e <= 127
 
 template <int F, int R>
@@ -206,8 +198,7 @@ DEV void gu_pass(const PfExperts &a, uint32_t e, uint32_t cg, uint32_t m0, uint3
         float gv = acc[0][r] * rs, uv = acc[1][r] * rs;
         gv = isfinite(gv) ? gv : 0.0f;   // (src/qx_format.c:4284)
         uv = isfinite(uv) ? uv : 0.0f;
-        const float ex = expf(-gv);      // (infinite below -88: the quotient is 0)
-        hs[row * LD + 32 * wave + col] = (ex < INFINITY ? div_ge1(gv, 1.0f + ex) : 0.0f) * uv;
+        hs[row * LD + 32 * wave + col] = gv / (1.0f + expf(-gv)) * uv;   // (correctly rounded quotient)
     }
     __syncthreads();
     // each row's 128 values become the down projection's packed operand, 16 lanes a row with 8

@@ -1,6 +1,6 @@
 """Batched prefill where its result could hang on more than the inputs, or lose bits that a norm
 over whole rows does not show: calls repeated bit for bit, attention heads whose context comes
-from small weights or small V scales alone, scores near and beyond f32's range.
+from small weights or small V scales alone, scores near and beyond f32's range, SwiGLU far in its tail.
 Models are generated files with a few tensors rewritten, so that the part in question stands
 alone in the output; the oracle reads the same files.  Runs through the C ABI (include/qxg.h)."""
 import numpy as np
@@ -147,3 +147,35 @@ def test_attention_large_scores(ctx, tmp_path, scale):
     errs = attention_rows(ctx, p, om, p0, x, (k, v, ks, vs))
     om.close()
     assert max(errs) <= REL_L2, errs
+
+
+@pytest.mark.parametrize("n", [1, 20])
+def test_swiglu_tail(ctx, tmp_path, n):
+    """Every gate value about -88, where 1 + e^-gate is beyond the range whose reciprocal is a
+    normal f32: silu is near 5e-37 and still counts, the up rows being large."""
+    p = tmp_path / "m.qxf"
+    t = one_layer(p, seed=31)
+    x = np.random.default_rng(13).standard_normal(2048).astype(np.float32)
+    t["blk.0.ffn_gate_inp.weight"][1].view(np.float32)[:] *= np.float32(1e-3)   # keep several experts' weights
+    gate = t["blk.0.ffn_gate_exps.weight"][1].reshape(-1, 8 * 74)
+    gate[:] = gate[0].copy()
+    up = t["blk.0.ffn_up_exps.weight"][1].reshape(-1, 74)
+    up[:, :2] = np.array([0x7400], np.uint16).view(np.uint8)   # fp16 16384
+    norm = t["blk.0.ffn_norm.weight"][1].view(np.float32)
+    norm[:] = 1
+    om = qxo.Model(p)
+    xd = x.astype(np.float64)
+    g = qxo.matvec(17, np.array(gate[0]), 1, 2048, (xd / np.sqrt((xd * xd).mean() + 1e-6)).astype(np.float32))[0]
+    x = (x * -np.sign(g)).astype(np.float32)
+    norm[:] = 88.0 / abs(g)
+    y, want, _, _ = om.moe_layer(0, x)
+    om.close()
+    assert 0 < np.abs(want).max() < 1e-20
+    t["blk.0.attn_output.weight"][1].reshape(-1, 136)[:, :2] = 0   # the expert half's input is x itself
+    ctx.load(p, verify=False)
+    ctx.kv_create(1, 32)
+    fi, moe, _ = ctx.prefill_layer(0, 0, np.tile(x, (n, 1)))
+    assert np.array_equal(fi, np.tile(x, (n, 1)))
+    # e^88 times an error of the gate's f32 sum, 1e-6 of it at most, is 88 times as much of the result
+    for r in range(n):
+        assert rel_l2(moe[r], want) <= 88e-6, (r, rel_l2(moe[r], want))
