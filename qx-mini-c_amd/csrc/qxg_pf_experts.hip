@@ -86,7 +86,8 @@ DEV uint4 ldu128(const void *p) { return *reinterpret_cast<const uint4 *>(p); }
 template <int F> struct GuBlk;                                               // the lane's half of a block
 template <> struct GuBlk<FMT_IQ2> { uint4 q[2]; uint32_t sc, d; };           // 16 grid/sign words, 4 scale bytes
 template <> struct GuBlk<FMT_IQ2S> { uint4 q, sg; uint32_t qh, sc, d; };     // 16 grid bytes, sign bytes, 4 x 8 high bits
-template <int F> constexpr int GU_LOADS = F == FMT_IQ2 ? 4 : 5;              // load instructions of gu_load
+// load instructions of gu_load: a wait counts on them (the listing's test holds the built code to it)
+template <int F> constexpr int GU_LOADS = F == FMT_IQ2 ? 4 : 5;
 DEV void gu_load(GuBlk<FMT_IQ2> &w, const PfMat &m, uint32_t bi, int h) {
     w.q[0] = ldu128(m.qs + bi * 64u + 32 * h);
     w.q[1] = ldu128(m.qs + bi * 64u + 32 * h + 16);

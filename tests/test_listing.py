@@ -137,3 +137,26 @@ def test_assembly_loads_in_flight(listing):
                         queued.add(j)
                         work.append(j)
     assert loads > 50
+
+
+def test_gate_up_counted_wait(listing):
+    """Gate/up waits for its staged rows by leaving the weights' loads, the youngest, in flight: the
+    counted wait in the middle of a block leaves no more than were issued behind the last copy."""
+    waits = 0
+    for name, code in listing.items():
+        if "qxp_gate_up" not in name:
+            continue
+        for i in (i for i, ins in enumerate(code) if ins.op == "s_barrier"):
+            left = since = None   # loads that the barrier's wait leaves in flight; loads since the last copy
+            for before in reversed(code[:i]):
+                if before.op.startswith(("s_branch", "s_cbranch", "global_load_lds")):
+                    break
+                m = re.search(r"vmcnt\((\d+)\)", before.text) if before.op == "s_waitcnt" else None
+                if m and left is None:
+                    left, since = int(m.group(1)), 0
+                elif since is not None:
+                    since += before.op.startswith(("global_load", "global_store", "buffer_", "flat_"))
+            if left:
+                waits += 1
+                assert before.op.startswith("global_load_lds") and since >= left, (name, left, since, code[i])
+    assert waits == 4   # two formats, passes of 16 and of 32 rows
