@@ -319,7 +319,7 @@ void build_tables(std::vector<uint4> &g2, std::vector<uint2> &g3, std::vector<ui
 
 // Writes the step state and the position's RoPE row; with in, also `bytes` of input (at most
 // IO_IN) to dst, through the context's pinned buffer.  The buffer is free for the next call: every
-// call ends by waiting for its stream.
+// call that passes input waits for its stream before it returns, failed or not.
 constexpr uint64_t IO_IN = 512 << 10, IO_OUT = 2 << 20;
 void write_state(qxg_ctx *c, uint32_t pos0, uint32_t step, uint32_t n_prompt, uint32_t force_head, const void *in = nullptr,
                  void *dst = nullptr, uint64_t bytes = 0) {
@@ -637,9 +637,15 @@ bool check_q8(qxg_ctx *c, char *err, uint64_t n) {
     return false;
 }
 
+// Waits for the call's work, also when one of its launches failed: what was queued before still
+// reads the pinned input, which the next call writes.
+bool wait_stream(qxg_ctx *c, char *err, uint64_t n) {
+    const hipError_t launch = hipGetLastError(), stream = hipStreamSynchronize(c->s);
+    return hip_ok(launch, err, n, "launch") && hip_ok(stream, err, n, "stream");
+}
+
 bool finish(qxg_ctx *c, char *err, uint64_t n) {
-    if (!hip_ok(hipGetLastError(), err, n, "launch")) return false;
-    if (!hip_ok(hipStreamSynchronize(c->s), err, n, "stream")) return false;
+    if (!wait_stream(c, err, n)) return false;
     if (c->q8 && !check_q8(c, err, n)) return false;
     return !c->abort || check_abort(c, err, n);
 }
@@ -678,7 +684,7 @@ bool finish_read(qxg_ctx *c, std::initializer_list<HostOut> outs, DevState *stat
     for (const HostOut &o : outs)
         if (o.dst && o.bytes) (void)add(o.src, o.bytes);
     hipLaunchKernelGGL(qxk_gather, dim3(std::max<uint32_t>(1, std::min<uint32_t>(128, most / 2048)), k), dim3(256), 0, c->s, g);
-    if (!hip_ok(hipGetLastError(), err, n, "launch") || !hip_ok(hipStreamSynchronize(c->s), err, n, "stream")) return false;
+    if (!wait_stream(c, err, n)) return false;
     DevState h;
     memcpy(&h, st, st_bytes);
     if (c->q8 && h.q8_fault && !check_q8(c, err, n)) return false;
@@ -1327,7 +1333,10 @@ int qxg_decode_token(qxg_ctx *c, uint32_t token, uint32_t position, int run_head
         d.wsum = c->wsum_dump;
         d.norm = run_head ? c->norm : nullptr;
         d.logits = run_head ? c->logits : nullptr;
-        if (!launch_decode(c, 1, run_head ? 1 : 2, position, false, d, err, err_len)) return 0;
+        if (!launch_decode(c, 1, run_head ? 1 : 2, position, false, d, err, err_len)) {
+            (void)hipStreamSynchronize(c->s);   // (the launch that reads the pinned input)
+            return 0;
+        }
         if (run_head) {
             hipLaunchKernelGGL(qxk_topk, dim3(TOPK_BLOCKS), dim3(256), 0, c->s, c->logits, c->vocab, top_n, c->cand_v,
                                c->cand_i, c->top_v, c->top_i, c->tokens, c->st);
