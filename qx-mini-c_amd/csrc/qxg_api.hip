@@ -172,8 +172,10 @@ struct qxg_ctx {
     // one decode step (embed .. head, top-1, step advance) recorded once and replayed
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
-    // the prefill's dense layout of every layer's Q/K/V and O matrices (qxg_pf_dense.hip)
+    // the prefill's dense layout of every layer's Q/K/V and O matrices (qxg_pf_dense.hip), made by the
+    // first batched prefill after a bind, and where each starts
     uint8_t *dense = nullptr;
+    std::vector<uint64_t> dense_at;
     // batched prefill: codebooks and work buffers for chunks of up to QXP_MAX tokens
     struct Prefill {
         bool ready = false;
@@ -508,31 +510,55 @@ bool build_router_fold(qxg_ctx *c, char *err, uint64_t n) {
     return ok;
 }
 
-// Layer l's Q/K/V (stacked rows) or O matrix in the dense layout: codes, scales, offsets
+// Layer l's Q/K/V (stacked rows) or O matrix in the dense layout: codes, scales and, where a matrix
+// has them (Q5_K), offsets
 constexpr uint64_t DENSE_QKV = 5120ull * 2048, DENSE_O = 2048ull * 4096;
-constexpr uint64_t DENSE_LAYER = (DENSE_QKV + DENSE_O) * 10 / 8;   // a byte a weight and 2 floats per 32 weights
 PfDense dense_args(const qxg_ctx *c, uint32_t l, bool qkv) {
     const LayerW &w = c->L[l];
     PfDense g{};
-    uint8_t *base = c->dense + l * DENSE_LAYER + (qkv ? 0 : DENSE_QKV * 10 / 8);
     const uint64_t n = qkv ? DENSE_QKV : DENSE_O;
-    g.codes = base;
-    g.scale = (const float *)(base + n);
-    g.ofs = g.scale + n / 32;
+    g.codes = c->dense + c->dense_at[2 * l + (qkv ? 0 : 1)];
+    g.scale = (const float *)(g.codes + n);
     g.lines = qkv ? 64 : 128;
     g.cols = qkv ? 5120 : 2048;
     g.seg1 = qkv ? 128 : 0xffffffffu;
     g.seg2 = qkv ? 144 : 0xffffffffu;
     g.ofs_segs = qkv ? (uint32_t)(w.wq->type == 13) | (uint32_t)(w.wk->type == 13) << 1 | (uint32_t)(w.wv->type == 13) << 2
                      : (uint32_t)(w.wo->type == 13);
+    g.ofs = g.ofs_segs ? g.scale + n / 32 : nullptr;
     return g;
 }
 
-// Every layer's Q/K/V and O matrices in the prefill's dense layout (1 GB for 48 layers)
-bool build_dense(qxg_ctx *c, char *err, uint64_t n) {
+void drop_dense(qxg_ctx *c) {
     if (c->dense) (void)hipFree(c->dense);
     c->dense = nullptr;
-    if (!hip_ok(hipMalloc(&c->dense, DENSE_LAYER * c->layers), err, n, "dense layout")) return false;
+    c->dense_at.clear();
+}
+
+// Every layer's Q/K/V and O matrices in the prefill's dense layout, if it is not there yet: 21.2 MB a
+// layer of IQ4_XS (1.02 GB for 48), 23.6 MB where Q/K/V and O both have Q5_K.  Only batched prefills
+// read it, so the first of them after a bind makes it.  room: false where the GPU's memory does not
+// hold it; the prompt then goes by token steps, which need nothing beyond the bound model.
+bool dense_ready(qxg_ctx *c, bool &room, char *err, uint64_t n) {
+    room = true;
+    if (c->dense || !c->layers) return true;
+    uint64_t total = 0;
+    for (uint32_t l = 0; l < c->layers; ++l) {
+        const LayerW &w = c->L[l];
+        const bool q5 = w.wq->type == 13 || w.wk->type == 13 || w.wv->type == 13;
+        c->dense_at.push_back(total);
+        total += DENSE_QKV * (q5 ? 10 : 9) / 8;   // a byte a weight and a float, or two, per 32
+        c->dense_at.push_back(total);
+        total += DENSE_O * (w.wo->type == 13 ? 10 : 9) / 8;
+    }
+    const hipError_t e = hipMalloc(&c->dense, total);
+    if (e != hipSuccess) {
+        drop_dense(c);
+        room = false;
+        if (e != hipErrorOutOfMemory) return hip_ok(e, err, n, "dense layout");
+        (void)hipGetLastError();   // not an error of the call
+        return true;
+    }
     for (uint32_t l = 0; l < c->layers; ++l) {
         const LayerW &w = c->L[l];
         const QTensor *m[4] = {w.wq, w.wk, w.wv, w.wo};
@@ -544,7 +570,8 @@ bool build_dense(qxg_ctx *c, char *err, uint64_t n) {
                                g.lines, ct0[i], (uint8_t *)g.codes, (float *)g.scale, (float *)g.ofs);
         }
     }
-    return hip_ok(hipGetLastError(), err, n, "dense layout") && hip_ok(hipStreamSynchronize(c->s), err, n, "dense layout");
+    if (!hip_ok(hipGetLastError(), err, n, "dense layout")) { drop_dense(c); return false; }
+    return true;
 }
 
 // The routed experts' rows of every layer in the persistent decode's interleaved layout
@@ -808,8 +835,11 @@ uint16_t f16_int(int v) {
 
 // The batched GEMM path takes every bound format in the f32 activation mode; q8_k_compat
 // prefills token by token through the decode kernels, which is how the reference
-// prefills every prompt.
-bool batched_prefill(const qxg_ctx *c) { return !c->q8; }
+// prefills every prompt, and so does a prompt whose dense layout does not fit.
+bool batched_prefill(qxg_ctx *c, bool &batched, char *err, uint64_t n) {
+    batched = !c->q8;
+    return !batched || dense_ready(c, batched, err, n);
+}
 
 // Parts of K of a dense GEMM over T rows: about 320 workgroups (two fit a CU) of at least 8
 // lines each.  Fewer leave CUs idle (a 37-token O projection as one part took 44 us on 16
@@ -1117,7 +1147,7 @@ void qxg_close(qxg_ctx *c) {
                     c->T.rope_cs, c->half_dump, c->wsum_dump};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : c->arenas) (void)hipFree(p);
-    if (c->dense) (void)hipFree(c->dense);
+    drop_dense(c);
     if (c->io) (void)hipHostFree(c->io);
     for (void *p : c->pf.all) (void)hipFree(p);
     for (void *p : c->sg.all) (void)hipFree(p);
@@ -1154,6 +1184,7 @@ int qxg_bind_model(qxg_ctx *c, uint32_t layers, int need_embedding, int need_hea
     (void)hipSetDevice(c->device);
     drop_graph(c);
     c->bound = false;
+    drop_dense(c);
     c->L.assign(layers, LayerW{});
     c->experts = 0;
     bool base = true;
@@ -1235,7 +1266,6 @@ int qxg_bind_model(qxg_ctx *c, uint32_t layers, int need_embedding, int need_hea
         if (!hip_ok(hipMalloc(bufs[i], sizes[i]), err, err_len, "work buffers")) return 0;
     if (!hip_ok(hipMemset(c->tokens, 0, sizes[15]), err, err_len, "work buffers")) return 0;
     if (layers && base && !build_arenas(c, err, err_len)) return 0;
-    if (layers && !build_dense(c, err, err_len)) return 0;
     if (c->mfold) { (void)hipFree(c->mfold); c->mfold = nullptr; }
     if (layers && base && !build_router_fold(c, err, err_len)) return 0;
     if (layers && base && !build_expert_interleave(c, err, err_len)) return 0;
@@ -1931,7 +1961,9 @@ int qxg_prefill(qxg_ctx *c, const uint32_t *tokens, uint32_t n, uint32_t positio
     if (top_n > QXG_MAX_TOPN) top_n = QXG_MAX_TOPN;
     (void)hipSetDevice(c->device);
     c->kt.used = 0;
-    if (!batched_prefill(c)) {
+    bool batched = false;
+    if (!batched_prefill(c, batched, err, err_len)) return 0;
+    if (!batched) {
         if (persistent(c) && c->layers && !residual_out) {
             // the token steps in one persistent launch (the head on the last token only:
             // n_prompt one past the steps keeps it off), then the top-N of its logits
@@ -1991,7 +2023,9 @@ int qxg_prefill_layer(qxg_ctx *c, uint32_t layer, uint32_t n, uint32_t position0
     }
     (void)hipSetDevice(c->device);
     c->kt.used = 0;
-    if (!batched_prefill(c)) {   // token steps of the layer's attention and MoE halves
+    bool batched = false;
+    if (!batched_prefill(c, batched, err, err_len)) return 0;
+    if (!batched) {   // token steps of the layer's attention and MoE halves
         for (uint32_t i = 0; i < n; ++i) {
             const uint64_t o = 2048ull * i;
             if (!hip_ok(hipMemcpyAsync(c->x, x_in + o, 2048 * 4, hipMemcpyHostToDevice, c->s), err, err_len, "upload")) return 0;

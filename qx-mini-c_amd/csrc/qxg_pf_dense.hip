@@ -1,10 +1,10 @@
 // Dense GEMMs of the batched prefill (CDNA4, gfx950): Q/K/V and the O projection.
 //
-// Weights.  qxp_dense_plane lays a matrix out once, when the model is bound: one byte per
-// weight, its integer code + 128 (IQ4_XS kvalue, Q5_K 5-bit code), in the order the matrix
-// instruction reads, [32-row tile][line of 32 K][lane][16 codes], and per row and 32 values
-// the f32 scale (d * (ls - 32) or d * sc) and, for Q5_K, the offset dmin * m: 1.13 bytes a
-// weight, 21 MB a layer.  A code becomes fp16 as bits(1024 + byte) - 1152, two a v_perm and
+// Weights.  qxp_dense_plane lays a matrix out once, before the first batched prefill of a bound
+// model: one byte per weight, its integer code + 128 (IQ4_XS kvalue, Q5_K 5-bit code), in the order
+// the matrix instruction reads, [32-row tile][line of 32 K][lane][16 codes], and per row and 32 values
+// the f32 scale (d * (ls - 32) or d * sc) and, for Q5_K, the offset dmin * m: 1.13 or 1.25 bytes a
+// weight, 21.2 to 23.6 MB a layer.  A code becomes fp16 as bits(1024 + byte) - 1152, two a v_perm and
 // v_pk_add.  From the file's nibbles the same codes took a random LDS read per byte, for every
 // row tile again, which bounded the kernel (56 us for Q/K/V and 49 for O of 512 tokens, now 36 and 27; 25 and
 // 48 of 37, now 10 and 9).  The matrix instructions bound it, about 20 us of the 36.
