@@ -793,20 +793,20 @@ __global__ __launch_bounds__(256, 4) void qxk_head(const uint32_t *dig, const ui
 // top-N (N <= 32) over logits by (value desc, index asc): each block of qxk_topk
 // reduces a slice to N candidates, qxk_topk_merge (one block, the next launch) merges
 // them and writes tokens[step+1] = argmax on generate steps.  A value and its index are one
-// 64-bit key, unique, 0 for none (NaN).  Each wave keeps its keys in registers and takes the
+// 64-bit key, unique, 0 for none (NaN); the lowest bit, below the index, keeps the sign of a zero.  Each wave keeps its keys in registers and takes the
 // largest N times (lane r keeps the r-th), the block's four lists are taken together in wave
 // 0: about 0.2 us a round and one barrier.  (Rounds of the whole block, each scanning the slice
 // again with two barriers: 15 + 15 us for N = 8, now 8 + 8.)
 namespace {
-DEV uint64_t topn_key(float v, uint32_t i) {
+DEV uint64_t topn_key(float v, uint32_t i) {   // i < 2^31
     if (v != v) return 0;
     const uint32_t b = __float_as_uint(v + 0.0f);   // (-0 as +0: equal values go by index)
-    return ((uint64_t)((b >> 31) ? ~b : (b | 0x80000000u)) << 32) | (0xffffffffu - i);
+    return ((uint64_t)((b >> 31) ? ~b : (b | 0x80000000u)) << 32) | ((0x7fffffffu - i) << 1) | (__float_as_uint(v) == 0x80000000u);
 }
 DEV void topn_out(uint64_t k, float &v, uint32_t &i) {
-    const uint32_t b = (uint32_t)(k >> 32);
-    v = k ? __uint_as_float((b >> 31) ? (b & 0x7fffffffu) : ~b) : -INFINITY;
-    i = k ? 0xffffffffu - (uint32_t)k : 0xffffffffu;
+    const uint32_t b = (uint32_t)(k >> 32), neg0 = b == 0x80000000u && (k & 1) ? 0x80000000u : 0u;
+    v = k ? __uint_as_float(((b >> 31) ? (b & 0x7fffffffu) : ~b) | neg0) : -INFINITY;
+    i = k ? 0x7fffffffu - ((uint32_t)k >> 1) : 0xffffffffu;
 }
 // the wave's n largest of its lanes' R keys: lane r (< n <= 32) returns the r-th
 template <int R>
