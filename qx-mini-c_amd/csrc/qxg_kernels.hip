@@ -742,9 +742,10 @@ template <int RPW> struct HeadRows {
 };
 
 // Bounded by the read of the rows (256 MB at 151936).  A wave keeps its digits (25 dwords a lane, twice
-// a row's bytes) and the code bias over all its rounds and has the next round's rows in flight
-// while it works on one; a round's rows lie next to each other over the whole launch.  128 VGPRs: four
-// waves a SIMD.  One round a wave (18992 workgroups) loaded the digits and formed the bias for every
+// a row's bytes) and the code bias over all its rounds and asks for the next round's rows before it
+// works on one; a round's rows lie next to each other over the whole launch.  (The loads are
+// conditional: where the paths join the compiler waits for 7 of the 12 before this round's first
+// product and for all before its second row.)  128 VGPRs: four waves a SIMD.  One round a wave (18992 workgroups) loaded the digits and formed the bias for every
 // two rows: 64.4 us (3.97 TB/s) for 151936 rows, now 52.7 (4.86); the whole call 138.6 -> 127.0 us.
 template <int RPW>
 __global__ __launch_bounds__(256, 4) void qxk_head(const uint32_t *dig, const uint8_t *ql,

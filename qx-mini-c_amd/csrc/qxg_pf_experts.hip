@@ -501,7 +501,12 @@ void qxp_launch_gate_up(hipStream_t s, uint32_t type, const PfExperts &a, const 
 }
 // Rows of down's passes: with up to 128 tokens, 32 spread a crowded expert over more workgroups (64 rows
 // of one expert each 20 -> 16 us, 37 tokens of a mixed model 20.6 -> 17.8); with more tokens the chip
-// is full and two tiles share the codes (300 tokens 33.6 us, 37.7 with 32 rows).
+// is full and two tiles share the codes (300 tokens 33.6 us, 37.7 with 32 rows).  Between them, random
+// rows over 128 experts, launch included, 32 rows against 64 in IQ3_XXS, IQ4_XS and IQ3_S: 96 tokens
+// 36.7/37.3, 47.4/45.3, 42.9/44.2 us; 128 tokens 37.6/37.7, 49.9/46.0, 43.5/47.1; 149 tokens 37.7/37.8,
+// 48.1/45.7, 51.0/47.8; 220 tokens 39.8/41.2, 54.2/52.1, 53.4/51.7.  (What counts is pairs an expert:
+// with 32 experts 64 rows win from 96 tokens on, 128 tokens 23.0/21.8.)  With 64 rows IQ4_XS spills 7
+// registers and IQ3_XXS one.
 static uint32_t down_rows(uint32_t T) { return T <= 128 ? 32 : 64; }
 void qxp_launch_down(hipStream_t s, uint32_t type, const PfExperts &a, const PfTables &P, uint32_t T, Timer tm) {
     const uint32_t R = down_rows(T);

@@ -186,8 +186,8 @@ extern "C" __global__ __launch_bounds__(256) void qxp_pack_ctx(const float *src,
 #pragma unroll
         for (int i = 0; i < 2; ++i) load8(p + 2048 * i, *reinterpret_cast<float(*)[8]>(v + 8 * i));
     } else {
-        // four runs' values and states at a time, so that one load latency covers them (37 tokens
-        // over 12 runs: 11.8 us a run at a time, now 8)
+        // four runs' states, then their values, at a time: the compiler issues the values in groups of
+        // two to four loads, a wait behind each (37 tokens over 12 runs: 11.8 us a run at a time, now 8)
         constexpr int N = 4;
         const float2 *s = md + (uint64_t)t * 32 + (tid >> 4);   // heads tid / 16 and 16 + tid / 16
         float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.0f, 0.0f};
@@ -609,9 +609,9 @@ extern "C" __global__ __launch_bounds__(256, 2) void qxp_attn(const float *qr, c
 // rows still give equal logits).  A workgroup owns a 16 x 16 (token x expert) tile of one
 // quarter of K; its 4 waves split that in 128s, and lane group g = lane / 16 of a wave feeds
 // k-slot g of v_mfma_f64_16x16x4 with float4 g of each 16 k.  The waves' tiles are added in
-// LDS in a fixed order, the quarters (planes of `logits`) by qxp_route.  Latency bounds it: a
-// wave's loads are all in flight before its first product, and a row's four lane groups
-// read one 64-byte piece.  (A workgroup over all of K, loads four iterations at a time: 11.4 us
+// LDS in a fixed order, the quarters (planes of `logits`) by qxp_route.  Latency bounds it: the
+// compiler keeps four of a wave's sixteen loads in flight, the next two issued behind each pair's
+// products; a row's four lane groups read one 64-byte piece.  (A workgroup over all of K, loads four iterations at a time: 11.4 us
 // for 37 tokens and 12.6 for 512; now 4.9 and 10.2.)
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 extern "C" __global__ __launch_bounds__(256) void qxp_router(const float *xn, const float *router, uint32_t T,
