@@ -227,7 +227,9 @@ int qxg_final_head(qxg_ctx *ctx, const float *residual, float *norm_out, float *
  * mode takes those token steps on the device instead: one persistent launch over the
  * prompt where the persistent path serves the model and residual_out is NULL, else the
  * one-kernel-per-phase decode kernels one token at a time; either way the result equals
- * qxg_decode_token over the prompt on the same layer path.
+ * qxg_decode_token over the prompt on the same layer path.  So does an f32 prompt where the
+ * GPU's memory does not hold the batched path's layout of the attention matrices (21 to 24 MB
+ * a layer), which the first batched call after a bind makes.  Equal calls give equal bits.
  * residual_out (may be NULL): n*2048 floats, each token's residual after the
  * last layer.  logits / top_* as in qxg_decode_token.  elapsed_ms: device time of the
  * whole call (HIP events on the context stream). */

@@ -343,7 +343,7 @@ extern "C" __global__ __launch_bounds__(640) void qxp_qk(const float *parts, uin
 // worked on.  (One scale of the column over all chunks spared the 64 additions, which measured
 // the same: 112 us for 512 at 3500 either way, and lost the bits of later, smaller weights.)  The
 // waves' states are merged in LDS, the runs' by qxp_pack_ctx.  (One run, the context rescaled at every
-// chunk: 60 us for 37 tokens at position 2100, now 16; 139 for 512 at 3500, now 105.)
+// chunk: 60 us for 37 tokens at position 2100, now 16; 139 for 512 at 3500, now 106 to 113.)
 namespace {
 constexpr int PA_TT = 4;   // tokens per workgroup
 
