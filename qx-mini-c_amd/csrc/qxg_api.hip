@@ -946,7 +946,7 @@ void prefill_layer(qxg_ctx *c, uint32_t l, uint32_t T, uint32_t p0, bool first, 
     g.part_lines = g.lines / o_parts;
     g.rows_packed = B.XP; g.rows = T; g.row_bytes = PF_PITCH(4096); g.rscale = B.xscale; g.sums = B.sums; g.out = B.PART;
     qxp_launch_dense(s, g, o_parts, timer_for(c, 9));
-    // MoE half: residual + RMSNorm, router logits, top-8 and the experts' pair lists, gate/up + SwiGLU, down, combine
+    // MoE half: residual + RMSNorm, router logits, top-8 and the experts' pairs, gate/up + SwiGLU, down, combine
     hipLaunchKernelGGL(qxp_ffn_norm, dim3(T), dim3(256), 0, s, (const float *)B.X, (const float *)B.PART, o_parts,
                        w.ffn_norm, T, B.X1, B.XN, B.XP, B.xscale);
     qx_launch(qxp_router, dim3((T + 15) / 16, (E + 15) / 16, 4), dim3(256), 0, s, timer_for(c, 12), (const float *)B.XN,
